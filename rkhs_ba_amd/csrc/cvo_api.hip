@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "cvo_internal.h"
+#include "cvo_loop.h"
 
 namespace cvo {
 
@@ -90,6 +91,13 @@ cvo_status ensure(cvo_ctx* ctx, DevBuf& b, size_t bytes) {
   b.cap = cap;
   ctx->ws_bytes += cap;
   return CVO_OK;
+}
+
+static void free_buf(cvo_ctx* ctx, DevBuf& b) {
+  if (b.p) (void)hipFree(b.p);
+  ctx->ws_bytes -= b.cap;
+  b.p = nullptr;
+  b.cap = 0;
 }
 
 template <class T>
@@ -445,6 +453,74 @@ cvo_status ensure_events(cvo_ctx* ctx, size_t n) {
 // done.  Profiling mode launches kernel by kernel with events around each.
 static constexpr int kChunk = 24;
 
+// Iterations of one resident launch.
+static constexpr int kLoopChunk = 1024;
+
+// The iteration loop as resident launches (cvo_loop.hip), where its rows fit
+// the blocks' LDS and the device's compute units are not held by other such
+// launches.  *ran false: nothing changed, or a wait ran out and the state is
+// that of a whole number of iterations; the caller's launch-per-pass loop goes
+// on from there.
+static cvo_status run_resident(cvo_ctx* ctx, const Problems& pr, const KConsts& kc, int max_iter, bool* ran) {
+  *ran = false;
+  const int np = pr.n_probs;
+  if (np != (kc.adaptive ? 3 : 1)) return CVO_OK;
+  int units = 0;
+  if (hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess) return CVO_OK;
+  int rows[3] = {0, 0, 0};
+  for (int q = 0; q < np; ++q) rows[q] = pr.host[q].n_src;
+  LoopShape shape;
+  LoopUnits held;
+  if (!loop_shape(kc, rows, np, units, &shape) || !held.claim(ctx->device, shape.blocks, units)) return CVO_OK;
+  hipStream_t st = ctx->stream;
+  const size_t words = loop_words_bytes(), backup = sizeof(ProblemState) * np;
+  // a workspace limit that holds the rest of the call must not fail for this
+  const size_t args_at = align_up(words + 256 + backup, 256), need = args_at + sizeof(LoopArgs);
+  const bool limited = ctx->ws_limit > 0 && ctx->b_loop.cap < need;
+  if (limited && ctx->ws_bytes + need + need / 4 > ctx->ws_limit) return CVO_OK;
+  CVO_TRY(ensure(ctx, ctx->b_loop, need));
+  char* base = as<char>(ctx->b_loop);
+  launch_zero(base, words + 256, st);
+  LoopArgs a{};
+  a.kc = kc;
+  for (int q = 0; q < np; ++q) a.prob[q] = pr.host[q];
+  // the self problems only sum
+  for (int q = 1; q < np; ++q) a.prob[q].pairs = nullptr;
+  a.rows = shape.rows;
+  a.xa = reinterpret_cast<uint64_t*>(base);
+  a.xb = loop_step_words(a.xa);
+  a.fail = reinterpret_cast<uint32_t*>(base + words);
+  char* saved = base + words + 256;
+  // CVO_LOOP_WAIT_MS: longest wait of one exchange (2 s)
+  const char* wm = std::getenv("CVO_LOOP_WAIT_MS");
+  a.wait_ticks = (uint64_t)((wm && wm[0] ? std::max(0.0, std::atof(wm)) : 2000.0) * 1e5);
+  volatile int32_t* flags = reinterpret_cast<volatile int32_t*>(ctx->pinned);
+  cvo_status status = CVO_OK;
+  for (int it = 0; it < max_iter && status == CVO_OK; it += kLoopChunk) {
+    a.max_iters = std::min(kLoopChunk, max_iter - it);
+    a.tag0 = (uint32_t)it + 1u;
+    hipError_t e = hipMemcpyAsync(saved, pr.states, backup, hipMemcpyDeviceToDevice, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(base + args_at, &a, sizeof(a), hipMemcpyHostToDevice, st);
+    if (e == hipSuccess) e = launch_loop(reinterpret_cast<const LoopArgs*>(base + args_at), kc, shape, st);
+    if (e == hipSuccess)
+      e = hipMemcpyAsync((void*)flags, &pr.states[0].done, sizeof(int32_t), hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipMemcpyAsync((void*)(flags + 1), a.fail, sizeof(int32_t), hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e == hipSuccess && flags[1]) {
+      e = hipMemcpyAsync(pr.states, saved, backup, hipMemcpyDeviceToDevice, st);
+      if (e == hipSuccess) e = hipStreamSynchronize(st);
+      if (e == hipSuccess) break;
+    }
+    if (e != hipSuccess) status = hip_check(ctx, e, "resident loop");
+    else if (flags[0] || it + kLoopChunk >= max_iter) {
+      *ran = true;
+      break;
+    }
+  }
+  if (ctx->ws_limit > 0) free_buf(ctx, ctx->b_loop);
+  return status;
+}
+
 static cvo_status run_loop(cvo_ctx* ctx, const Problems& pr, const KConsts& kc, int max_iter, bool with_step,
                            double* device_seconds) {
   hipStream_t st = ctx->stream;
@@ -504,6 +580,11 @@ static cvo_status run_loop(cvo_ctx* ctx, const Problems& pr, const KConsts& kc, 
     launch_overflow(pr.dev, pr.n_probs, kc, st, pr.host.data());
     CVO_HIP(ctx, hipGetLastError());
   } else {
+    const char* ng = std::getenv("CVO_NO_GRAPH");
+    const bool use_graph = !(ng && ng[0] && ng[0] != '0');
+    bool ran = false;
+    if (use_graph) CVO_TRY(run_resident(ctx, pr, kc, max_iter, &ran));
+    if (!ran) {
     // one chunk of iterations, captured in a graph unless CVO_NO_GRAPH is set
     // (direct launches, e.g. under a kernel tracer)
     auto launch_chunk = [&]() {
@@ -513,8 +594,6 @@ static cvo_status run_loop(cvo_ctx* ctx, const Problems& pr, const KConsts& kc, 
         step_phase(nullptr, nullptr);
       }
     };
-    const char* ng = std::getenv("CVO_NO_GRAPH");
-    const bool use_graph = !(ng && ng[0] && ng[0] != '0');
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     if (use_graph) {
@@ -561,6 +640,7 @@ static cvo_status run_loop(cvo_ctx* ctx, const Problems& pr, const KConsts& kc, 
     }
     if (status != CVO_OK) return status;
     if (se != hipSuccess) return hip_check(ctx, se, "hipStreamSynchronize");
+    }
   }
   CVO_HIP(ctx, hipEventRecord(t1, st));
   CVO_HIP(ctx, hipEventSynchronize(t1));
@@ -764,20 +844,13 @@ extern "C" cvo_status cvo_set_params(cvo_ctx* ctx, const cvo_params* p) {
   return CVO_OK;
 }
 
-static void free_buf(cvo_ctx* ctx, DevBuf& b) {
-  if (b.p) (void)hipFree(b.p);
-  ctx->ws_bytes -= b.cap;
-  b.p = nullptr;
-  b.cap = 0;
-}
-
 // Every arena buffer of a context.
 static std::vector<DevBuf*> all_bufs(cvo_ctx* ctx) {
   std::vector<DevBuf*> v = {&ctx->b_src_pos, &ctx->b_src_feat, &ctx->b_src_sem, &ctx->b_src_geo, &ctx->b_src_key,
                             &ctx->b_src_perm, &ctx->b_grid_store, &ctx->b_pairs, &ctx->b_counts, &ctx->b_ovf,
                             &ctx->b_state, &ctx->b_probs, &ctx->b_gridhdr, &ctx->b_part_a, &ctx->b_part_ovf,
                             &ctx->b_part_s, &ctx->b_part_cnt, &ctx->b_trace, &ctx->b_tmp0, &ctx->b_tmp1,
-                            &ctx->b_tmp2, &ctx->b_tmp3, &ctx->b_cub, &ctx->b_export};
+                            &ctx->b_tmp2, &ctx->b_tmp3, &ctx->b_cub, &ctx->b_export, &ctx->b_loop};
   for (auto& b : ctx->b_ba) v.push_back(&b);
   for (auto& b : ctx->b_frames) v.push_back(&b);
   for (auto& b : ctx->b_mlp) v.push_back(&b);

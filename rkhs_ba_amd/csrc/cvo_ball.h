@@ -101,10 +101,19 @@ __device__ __forceinline__ uint32_t group_bits(uint64_t m) {
   if constexpr (G == 64) {
     return 0u;  // use the 64-bit ballot directly
   } else {
-    constexpr uint32_t kGroupMask = (uint32_t)((1ull << G) - 1ull);
+    constexpr uint32_t kGroupMask = (uint32_t)((1ull << G) - 1ull);  // G = 32: all ones
     return (uint32_t)(m >> (G * ((threadIdx.x & 63) / G))) & kGroupMask;
   }
 }
+
+// The same for any group size up to the wave: 32 bits, 64 for a whole wave.
+template <int G>
+__device__ __forceinline__ auto group_ballot(uint64_t m) {
+  if constexpr (G == 64) return m;
+  else return group_bits<G>(m);
+}
+__device__ __forceinline__ uint32_t group_count(uint32_t m) { return (uint32_t)__popc(m); }
+__device__ __forceinline__ uint32_t group_count(uint64_t m) { return (uint32_t)__popcll(m); }
 
 // Selection of the K smallest keys among a set of targets.  each(fn) calls
 // fn(valid, sorted position) for every target of the set, all G lanes of the

@@ -44,6 +44,29 @@ __device__ __forceinline__ void st_global(float4* p, float4 v) {
   *(__attribute__((address_space(1))) v4f*)p = t;
 }
 
+// The value of lane (id ^ O), without an address register: data-parallel moves
+// inside a row of 16, the LDS crossbar's swizzle across rows of a half wave, the
+// half-wave swap for 32.  All lanes of the wave take part.
+template <int O>
+__device__ __forceinline__ uint32_t xor_lane(uint32_t v) {
+  static_assert(O == 1 || O == 2 || O == 4 || O == 8 || O == 16 || O == 32, "lane distance");
+  if constexpr (O == 1) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true);   // quad 1,0,3,2
+  else if constexpr (O == 2) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true);  // quad 2,3,0,1
+  else if constexpr (O == 8) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xF, 0xF, true);  // row rotate 8
+  else if constexpr (O == 32) {
+    const auto s = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return (threadIdx.x & 32) ? (uint32_t)s[0] : (uint32_t)s[1];
+  } else {
+    return (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, (O << 10) | 0x1F);
+  }
+}
+template <int O>
+__device__ __forceinline__ double xor_lane(double v) {
+  const uint64_t b = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = xor_lane<O>((uint32_t)b), hi = xor_lane<O>((uint32_t)(b >> 32));
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
 __device__ __forceinline__ void affine3(const float* A, const float* b, float y0, float y1, float y2, float& o0,
                                         float& o1, float& o2) {
   o0 = fmaf(A[2], y2, fmaf(A[1], y1, fmaf(A[0], y0, b[0])));

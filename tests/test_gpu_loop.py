@@ -1,0 +1,136 @@
+"""The resident iteration loop against the launch-per-pass loop (CVO_NO_GRAPH=1)
+of the same library, which the other tests pin to the oracle.
+
+Both evaluate the same pairs with the same float operations; only the order of
+the FP64 sums differs (relative 1e-16 a sum), so over a dozen iterations the
+stored pairs are equal and the float poses agree to a few units in the last
+place (2e-6 absolute at entries of order one, metres up to ten)."""
+import os
+import threading
+
+import numpy as np
+import pytest
+
+from conftest import params_from_yaml
+from rkhs_ba_amd import CvoGPU, synth
+
+pytestmark = pytest.mark.gpu
+
+ITERS = 12
+
+
+def pair(n, m, seed=0, classes=0, feats=5, geo=False):
+    src, tgt, T = synth.planes_spheres_pair(seed, max(n, 64), max(m, 64))
+    out = []
+    for c, k in ((src, n), (tgt, m)):
+        rng = np.random.default_rng([seed, k])
+        sem = None
+        if classes:
+            sem = rng.random((c.n, classes)).astype(np.float32)
+            sem /= sem.sum(1, keepdims=True)
+        g = rng.random((c.n, 2)).astype(np.float32) + 0.1 if geo else None
+        f = c.feat[:, :feats] if feats <= 5 else np.concatenate([c.feat, c.feat[:, :feats - 5]], 1)
+        out.append(synth.Cloud(c.xyz, np.ascontiguousarray(f), sem, g).subset(np.arange(k)))
+    return out[0], out[1]
+
+
+def run(cvo, src, tgt, adaptive=False):
+    cvo.set_trace(ITERS)
+    if adaptive:
+        ret, T, _, it = cvo.align_adaptive(src, tgt, np.eye(4))
+    else:
+        ret, T, _, it, _ = cvo.align(src, tgt, np.eye(4))
+    return ret, T, it, cvo.get_trace()
+
+
+def both(p, src, tgt, adaptive=False, pose="fp64", tuning=None, env=None):
+    cvo = CvoGPU(params=p)
+    try:
+        cvo.set_pose_arithmetic(pose)
+        if tuning:
+            cvo.set_tuning(**tuning)
+        print("resident", src.n, tgt.n, flush=True)
+        for k, v in (env or {}).items():
+            os.environ[k] = v
+        try:
+            a = run(cvo, src, tgt, adaptive)
+        finally:
+            for k in env or {}:
+                del os.environ[k]
+        print("per pass", src.n, tgt.n, flush=True)
+        os.environ["CVO_NO_GRAPH"] = "1"
+        try:
+            b = run(cvo, src, tgt, adaptive)
+        finally:
+            del os.environ["CVO_NO_GRAPH"]
+    finally:
+        cvo.close()
+    assert a[0] == b[0] and a[2] == b[2]
+    np.testing.assert_allclose(a[1], b[1], rtol=0, atol=2e-6)
+    assert [(r.nnz, r.max_row, r.num_neighbors) for r in a[3]] == [(r.nnz, r.max_row, r.num_neighbors) for r in b[3]]
+    assert [r.ell for r in a[3]] == pytest.approx([r.ell for r in b[3]], rel=1e-6)
+    return a
+
+
+def params(**kw):
+    p = params_from_yaml("planes_spheres_5k.yaml")
+    p.MAX_ITER = ITERS
+    for k, v in kw.items():
+        setattr(p, k, v)
+    return p
+
+
+# one row; below, at and above a chunk of 8 rows, a block of 16, the 32 blocks
+# that exchange in one level, a lane-count step, and a tile of every block
+@pytest.mark.parametrize("n,m", [(1, 40), (7, 64), (8, 64), (9, 64), (17, 64), (511, 700), (513, 300), (1040, 900),
+                                 (4097, 3001), (8200, 8200), (20011, 20011)])
+def test_sizes(n, m):
+    src, tgt = pair(n, m)
+    both(params(), src, tgt)
+
+
+@pytest.mark.parametrize("kw,cloud,opts", [
+    (dict(nearest_neighbors_max=6), {}, {}),                                   # rows over the cap
+    (dict(is_using_semantics=1, s_ell=0.5, s_sigma=1.0), dict(classes=19), {}),
+    (dict(is_using_semantics=1, s_ell=0.5, s_sigma=1.0, nearest_neighbors_max=9), dict(classes=7, feats=3), {}),
+    (dict(is_using_intensity=0, is_using_geometric_type=1), dict(geo=True), {}),
+    (dict(is_using_kdtree=2), {}, {}),
+    (dict(is_using_kdtree=1), {}, dict(tuning=dict(lanes_per_row=8))),
+    ({}, {}, dict(pose="reference")),
+    ({}, {}, dict(tuning=dict(lanes_per_row=4, cell_scale=0.5, xcd_remap=0))),
+    ({}, dict(feats=8), dict(adaptive=True)),
+    (dict(nearest_neighbors_max=8), {}, dict(adaptive=True)),                  # capped self problems too
+])
+def test_options(kw, cloud, opts):
+    src, tgt = pair(1501, 1303, **cloud)
+    both(params(**kw), src, tgt, **opts)
+
+
+def test_a_wait_that_runs_out_falls_back():
+    # no wait at all: the first word that is not there yet ends the launch, and
+    # the registration is done by the launch-per-pass loop from the saved state
+    src, tgt = pair(1501, 1303)
+    both(params(), src, tgt, env={"CVO_LOOP_WAIT_MS": "0"})
+
+
+def test_threads_share_the_compute_units():
+    # four registrations at once, each wanting every compute unit
+    src, tgt = pair(4500, 4500)
+    want = both(params(), src, tgt)
+    got = [None] * 4
+
+    def work(i):
+        cvo = CvoGPU(params=params())
+        try:
+            got[i] = [cvo.align(src, tgt, np.eye(4))[1] for _ in range(3)]
+        finally:
+            cvo.close()
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for g in got:
+        for T in g:
+            np.testing.assert_allclose(T, want[1], rtol=0, atol=2e-6)
