@@ -72,8 +72,7 @@ __host__ __device__ inline float bf2f(uint16_t b) {
 // (transposes are stride swaps).  64 x 64 block tile, four waves of 32 x 32
 // (2 x 2 tiles of v_mfma_f32_16x16x16_bf16), k-steps of 16 staged in LDS.
 // Epilogue: optional bias (per n), ReLU, mask (zero where a BF16 matrix of the
-// same shape is zero), FP32 store or accumulate, BF16 store, or a max-pool over
-// row groups into packed (value, ~row) keys.
+// same shape is zero), FP32 store or accumulate, BF16 store.
 // ---------------------------------------------------------------------------
 
 typedef short short4_t __attribute__((ext_vector_type(4)));
@@ -94,14 +93,11 @@ struct GemmArgs {
   int relu;
   const uint16_t* mask;  // optional, M x N BF16, zero -> output zero
   int64_t ldm;
-  unsigned long long* pool;  // optional: pool[(m / group) * N + n] = max key
-  int group;                 // rows per pool group (multiple of 64)
 };
 
 __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
   __shared__ uint16_t As[64][16 + 4];
   __shared__ uint16_t Bs[16][64 + 4];
-  __shared__ unsigned long long s_pool[2][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
   const int wm = wave >> 1, wn = wave & 1;
@@ -153,7 +149,6 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
     __syncthreads();
   }
   // epilogue: lane holds rows (lane >> 4) * 4 + v, column lane & 15 of each tile
-  unsigned long long colmax[2] = {0ull, 0ull};
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -165,60 +160,30 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
         if (m >= g.M || n >= g.N) continue;
         float x = acc[i][j][v];
         if (g.bias) x += g.bias[n];
-        if (g.relu) x = x > 0.0f ? x : 0.0f;  // never -0 (pool keys use the bits)
+        if (g.relu) x = x > 0.0f ? x : 0.0f;
         if (g.mask && g.mask[(int64_t)m * g.ldm + n] == 0) x = 0.0f;
         if (g.C) {
           float* cp = g.C + (int64_t)m * g.ldc + n;
           *cp = g.accumulate ? *cp + x : x;
         }
         if (g.Cb) g.Cb[(int64_t)m * g.ldcb + n] = f2bf(x);
-        if (g.pool) {
-          // x >= 0 (ReLU): float bits order like the values; ties -> lower row
-          const unsigned long long key =
-              ((unsigned long long)__float_as_uint(x) << 32) | (unsigned long long)(0xFFFFFFFFu - (uint32_t)(m % g.group));
-          colmax[j] = colmax[j] > key ? colmax[j] : key;
-        }
       }
     }
-  if (g.pool) {
-    // 64 rows of the block belong to one group (group % 64 == 0): reduce the
-    // 4 lane groups, the 2 row tiles (already in colmax) and the 2 waves of
-    // each column half, then one atomic per column
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      unsigned long long k = colmax[j];
-      unsigned long long o = __shfl_xor(k, 16, 64);
-      k = k > o ? k : o;
-      o = __shfl_xor(k, 32, 64);
-      k = k > o ? k : o;
-      colmax[j] = k;
-    }
-    if (lane < 16) {
-      s_pool[wm][wn * 32 + 0 * 16 + lane] = colmax[0];
-      s_pool[wm][wn * 32 + 1 * 16 + lane] = colmax[1];
-    }
-    __syncthreads();
-    if (tid < 64) {
-      const int n = n0 + tid;
-      const unsigned long long a = s_pool[0][tid], b = s_pool[1][tid];
-      const unsigned long long k = a > b ? a : b;
-      if (n < g.N && m0 < g.M) atomicMax(&g.pool[(int64_t)(m0 / g.group) * g.N + n], k);
-    }
-  }
 }
 
 // ---------------------------------------------------------------------------
-// Fused point encoder for inference: the three per-point layers (16 -> 64 ->
-// 128 -> 256, bias and ReLU, BF16 between layers as in the layer-by-layer
-// path) and the max-pool over the cloud in one kernel.  One workgroup per
-// cloud: the weights are staged once, transposed (n rows of k), so both MFMA
-// operands are 16-byte LDS loads; the cloud's points go through in tiles of
-// 128, each of the four waves owning 32 rows of a tile from the input to the
-// pool, so the activations never leave LDS.  Layer 1 (k = 16) runs on
-// v_mfma_f32_16x16x16_bf16, layers 2 and 3 on v_mfma_f32_16x16x32_bf16.  The
-// pool keeps, per column, the largest (value bits, ~row) key of the cloud
-// (ties to the lower row), folded in registers and reduced across lanes and
-// waves in fixed order: one plain store per cloud and channel.
+// Fused point encoder: the three per-point layers (16 -> 64 -> 128 -> 256, bias
+// and ReLU, BF16 between layers) and the max-pool over the cloud in one kernel.
+// One workgroup per cloud, or per slice of a cloud's points when the clouds
+// alone leave compute units idle: the weights are staged once, transposed (n
+// rows of k), so both MFMA operands are 16-byte LDS loads; the points go through
+// in tiles of 128, each of the four waves owning 32 rows of a tile from the
+// input to the pool, so the activations never leave LDS.  Layer 1 (k = 16) runs
+// on v_mfma_f32_16x16x16_bf16, layers 2 and 3 on v_mfma_f32_16x16x32_bf16.  The
+// pool keeps, per column, the largest (value bits, ~row) key of the block's
+// points (ties to the lower row), folded in registers and reduced across lanes
+// and waves in fixed order: one plain store per block and channel, and the
+// largest over a cloud's blocks when the keys are unpacked.
 // ---------------------------------------------------------------------------
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -241,15 +206,38 @@ __device__ __forceinline__ short4_t lds4(const uint16_t* p) {
   return __builtin_bit_cast(short4_t, *reinterpret_cast<const uint2*>(p));
 }
 
+// acc + the product of a 16-row and a 16-column operand over 32 k (a, b: rows
+// of k in LDS).  FINE: as two 16-k products, the order in which the layer-by-
+// layer GEMM sums.
+template <bool FINE>
+__device__ __forceinline__ float4_t mfma32(const uint16_t* a, const uint16_t* b, int kq, float4_t acc) {
+  if constexpr (FINE) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(lds4(a + kq * 4), lds4(b + kq * 4), acc, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(lds4(a + 16 + kq * 4), lds4(b + 16 + kq * 4), acc, 0, 0, 0);
+  } else {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(lds8(a + kq * 8), lds8(b + kq * 8), acc, 0, 0, 0);
+  }
+}
+
+// TRAIN: keeps the activations of both hidden layers (H1, H2) for the backward
+// pass and sums in 16-k steps, so that a batch's activations and pooled points
+// are those of the layer-by-layer GEMMs to the bit.  The three GEMMs took 900
+// us for 256 clouds of 2048 points (they read back what they write, through
+// 2-byte LDS accesses); this 139.
+template <bool TRAIN>
 __global__ __launch_bounds__(256) void encoder_fused_kernel(const uint16_t* __restrict__ X, int npts,
                                                             const uint16_t* __restrict__ W1b,
                                                             const uint16_t* __restrict__ W2b,
                                                             const uint16_t* __restrict__ W3b,
                                                             const float* __restrict__ w,
-                                                            unsigned long long* __restrict__ pool) {
+                                                            unsigned long long* __restrict__ pool, int splits,
+                                                            uint16_t* __restrict__ H1, uint16_t* __restrict__ H2) {
   __shared__ EncLds L;  // 155 KB of the CU's 160 KB
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int cloud = blockIdx.x;
+  const int cloud = (int)blockIdx.x / splits, split = (int)blockIdx.x - cloud * splits;
+  // this block's tiles of the cloud
+  const int tiles = (npts + kFT - 1) / kFT;
+  const int first = tiles * split / splits * kFT, last = min(npts, tiles * (split + 1) / splits * kFT);
   const float* b1 = w + oB1;
   const float* b2 = w + oB2;
   const float* b3 = w + oB3;
@@ -262,7 +250,7 @@ __global__ __launch_bounds__(256) void encoder_fused_kernel(const uint16_t* __re
 #pragma unroll
   for (int t = 0; t < kH3 / 16; ++t) best[t] = 0ull;
   const uint16_t* Xc = X + (size_t)cloud * npts * kMlpInPad;
-  for (int t0 = 0; t0 < npts; t0 += kFT) {
+  for (int t0 = first; t0 < last; t0 += kFT) {
     __syncthreads();  // the weights are staged / the previous tile is done with x
     {
       const int r = tid >> 1, h = (tid & 1) * 8;
@@ -295,19 +283,22 @@ __global__ __launch_bounds__(256) void encoder_fused_kernel(const uint16_t* __re
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the wave's own h1 rows are written
     __builtin_amdgcn_wave_barrier();
+    const size_t row0 = (size_t)cloud * npts + t0 + rw;  // the wave's first point
+    if constexpr (TRAIN) {
+#pragma unroll
+      for (int i = lane; i < 32 * kH1 / 8; i += 64)
+        *reinterpret_cast<uint4*>(H1 + (row0 + i / (kH1 / 8)) * kH1 + (i % (kH1 / 8)) * 8) =
+            *reinterpret_cast<const uint4*>(&L.h1[rw + i / (kH1 / 8)][(i % (kH1 / 8)) * 8]);
+    }
     // layer 2: 64 -> 128
 #pragma unroll 2
     for (int ct = 0; ct < kH2 / 16; ++ct) {
       float4_t acc[2] = {(float4_t){0.0f, 0.0f, 0.0f, 0.0f}, (float4_t){0.0f, 0.0f, 0.0f, 0.0f}};
 #pragma unroll
-      for (int ks = 0; ks < kH1 / 32; ++ks) {
-        const bf16x8_t b = lds8(&L.w2t[ct * 16 + col][ks * 32 + kq * 8]);
+      for (int ks = 0; ks < kH1 / 32; ++ks)
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt) {
-          const bf16x8_t a = lds8(&L.h1[rw + rt * 16 + col][ks * 32 + kq * 8]);
-          acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[rt], 0, 0, 0);
-        }
-      }
+        for (int rt = 0; rt < 2; ++rt)
+          acc[rt] = mfma32<TRAIN>(&L.h1[rw + rt * 16 + col][ks * 32], &L.w2t[ct * 16 + col][ks * 32], kq, acc[rt]);
       const int c = ct * 16 + col;
 #pragma unroll
       for (int rt = 0; rt < 2; ++rt)
@@ -320,6 +311,12 @@ __global__ __launch_bounds__(256) void encoder_fused_kernel(const uint16_t* __re
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);
     __builtin_amdgcn_wave_barrier();
+    if constexpr (TRAIN) {
+#pragma unroll
+      for (int i = lane; i < 32 * kH2 / 8; i += 64)
+        *reinterpret_cast<uint4*>(H2 + (row0 + i / (kH2 / 8)) * kH2 + (i % (kH2 / 8)) * 8) =
+            *reinterpret_cast<const uint4*>(&L.h2[rw + i / (kH2 / 8)][(i % (kH2 / 8)) * 8]);
+    }
     // layer 3: 128 -> 256, four column tiles at a time, folded into the pool
     for (int cc = 0; cc < kH3 / 16; cc += 4) {
       float4_t acc[2][4];
@@ -329,13 +326,11 @@ __global__ __launch_bounds__(256) void encoder_fused_kernel(const uint16_t* __re
         for (int j = 0; j < 4; ++j) acc[rt][j] = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int ks = 0; ks < kH2 / 32; ++ks) {
-        const bf16x8_t a0 = lds8(&L.h2[rw + col][ks * 32 + kq * 8]);
-        const bf16x8_t a1 = lds8(&L.h2[rw + 16 + col][ks * 32 + kq * 8]);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const bf16x8_t b = lds8(&L.w3t[(cc + j) * 16 + col][ks * 32 + kq * 8]);
-          acc[0][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b, acc[0][j], 0, 0, 0);
-          acc[1][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b, acc[1][j], 0, 0, 0);
+          const uint16_t* b = &L.w3t[(cc + j) * 16 + col][ks * 32];
+          acc[0][j] = mfma32<TRAIN>(&L.h2[rw + col][ks * 32], b, kq, acc[0][j]);
+          acc[1][j] = mfma32<TRAIN>(&L.h2[rw + 16 + col][ks * 32], b, kq, acc[1][j]);
         }
       }
 #pragma unroll
@@ -373,7 +368,7 @@ __global__ __launch_bounds__(256) void encoder_fused_kernel(const uint16_t* __re
     const int c = tid;  // 256 channels, one a thread
     unsigned long long k = L.pool[0][c];
     for (int wv = 1; wv < 4; ++wv) k = k > L.pool[wv][c] ? k : L.pool[wv][c];
-    pool[(size_t)cloud * kH3 + c] = k;
+    pool[(size_t)blockIdx.x * kH3 + c] = k;
   }
 }
 
@@ -395,7 +390,6 @@ static GemmArgs gemm_args(const uint16_t* A, int64_t a_sm, int64_t a_sk, const u
   g.M = M;
   g.N = N;
   g.K = K;
-  g.group = 64;
   return g;
 }
 
@@ -542,20 +536,19 @@ __global__ __launch_bounds__(256) void mlp_prep_kernel(const float* __restrict__
   }
 }
 
-__global__ void fill_u64_kernel(unsigned long long* p, int64_t n, unsigned long long v) {
-  int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
-}
-
-// Pooled keys -> z (BF16, [src | tgt] per pair), pooled values (FP32) and the
-// argmax point of every (cloud, channel).
-__global__ void mlp_unpack_pool_kernel(const unsigned long long* __restrict__ pool, int n_pairs,
+// Pooled keys (of each of a cloud's splits) -> z (BF16, [src | tgt] per pair),
+// pooled values (FP32) and the argmax point of every (cloud, channel).
+__global__ void mlp_unpack_pool_kernel(const unsigned long long* __restrict__ pool, int splits, int n_pairs,
                                        uint16_t* __restrict__ z, float* __restrict__ gval,
                                        int32_t* __restrict__ garg) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;  // cloud * 256 + ch
   if (i >= (int64_t)n_pairs * 2 * kH3) return;
   const int cloud = (int)(i / kH3), ch = (int)(i % kH3);
-  const unsigned long long k = pool[i];
+  unsigned long long k = 0ull;
+  for (int q = 0; q < splits; ++q) {
+    const unsigned long long o = pool[((int64_t)cloud * splits + q) * kH3 + ch];
+    k = k > o ? k : o;
+  }
   const float v = __uint_as_float((uint32_t)(k >> 32));
   gval[i] = v;
   garg[i] = (int32_t)(0xFFFFFFFFu - (uint32_t)(k & 0xFFFFFFFFull));
@@ -746,24 +739,127 @@ __global__ __launch_bounds__(128) void mlp_rows_kernel(const float* __restrict__
 }
 
 // dW3[i][ch] = sum over clouds of v(cloud, ch) H2[argmax][i]; db3[ch] = sum v.
-// One thread per (i, ch), clouds summed in index order.
-__global__ void mlp_dw3_kernel(const float* __restrict__ rowv, const int32_t* __restrict__ garg, int n_clouds,
-                               int npts, const uint16_t* __restrict__ H2, float* __restrict__ dW3,
-                               float* __restrict__ db3) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= kH2 * kH3) return;
-  const int i = idx / kH3, ch = idx % kH3;
+// One block per channel, one thread per i, clouds summed in index order: a
+// cloud's row of H2 is one 256-byte read (a thread per (i, ch) with the
+// channels side by side read 2 bytes from as many rows: 211 us at 256 clouds,
+// against 25).
+__global__ __launch_bounds__(kH2) void mlp_dw3_kernel(const float* __restrict__ rowv, const int32_t* __restrict__ garg,
+                                                      int n_clouds, int npts, const uint16_t* __restrict__ H2,
+                                                      float* __restrict__ dW3, float* __restrict__ db3) {
+  const int ch = blockIdx.x, i = threadIdx.x;
   float s = 0.0f, sb = 0.0f;
+#pragma unroll 8
   for (int c = 0; c < n_clouds; ++c) {
     const int64_t row = (int64_t)c * kH3 + ch;
     const float v = rowv[row];
-    if (v == 0.0f) continue;
-    const int64_t pt = (int64_t)c * npts + garg[row];
-    s += v * bf2f(H2[pt * kH2 + i]);
-    sb += v;
+    const float h = bf2f(H2[((int64_t)c * npts + garg[row]) * kH2 + i]);
+    // a zero gradient leaves the sums as they are (h is finite or not)
+    s = v != 0.0f ? s + v * h : s;
+    sb = v != 0.0f ? sb + v : sb;
   }
   dW3[(int64_t)i * kH3 + ch] = s;
   if (i == 0) db3[ch] = sb;
+}
+
+// Weight gradients of the encoder's first two layers over the R rows of the
+// backward pass: dW2 = H1g^T dH2, db2 = colsum dH2, dW1 = Xg^T dH1 (16 input
+// rows), db1 = colsum dH1.  The products are thin and R is long (64 x 128 and
+// 16 x 64 over 65536 rows for 128 pairs): each block takes a range of rows and
+// writes its FP32 partial, mlp_rowgrad_sum_kernel adds the partials in block
+// order.  (One GEMM block per 64 x 64 output tile walked all rows alone: 6.6 and
+// 4.6 ms, and two column sums of 0.1 ms; together here 34 us.)
+// A tile of 64 rows is staged transposed, [column][row], so that both MFMA
+// operands are 16-byte LDS reads along the rows.
+constexpr int kRgTile = 64;
+constexpr int kRgPart = kH1 * kH2 + kMlpInPad * kH1 + kH2 + kH1;
+struct alignas(16) RowGradLds {
+  uint16_t h1[kH1][kRgTile + 8];
+  uint16_t d2[kH2][kRgTile + 8];
+  uint16_t x[kMlpInPad][kRgTile + 8];
+  uint16_t d1[kH1][kRgTile + 8];
+};
+
+// N consecutive columns c0 ... of row r of an array of W columns, to [column][row].
+template <int W, int N>
+__device__ __forceinline__ void stage_transposed(const uint16_t* __restrict__ src, int64_t row, int r, int c0,
+                                                 uint16_t (*dst)[kRgTile + 8]) {
+#pragma unroll
+  for (int j = 0; j < N; j += 4) {
+    const uint2 v = *reinterpret_cast<const uint2*>(src + row * W + c0 + j);
+    dst[c0 + j][r] = (uint16_t)v.x;
+    dst[c0 + j + 1][r] = (uint16_t)(v.x >> 16);
+    dst[c0 + j + 2][r] = (uint16_t)v.y;
+    dst[c0 + j + 3][r] = (uint16_t)(v.y >> 16);
+  }
+}
+
+// R and rows_per are multiples of kRgTile.
+__global__ __launch_bounds__(256) void mlp_rowgrad_kernel(const uint16_t* __restrict__ H1g,
+                                                          const uint16_t* __restrict__ dH2,
+                                                          const uint16_t* __restrict__ Xg,
+                                                          const uint16_t* __restrict__ dH1, int R, int rows_per,
+                                                          float* __restrict__ part) {
+  __shared__ RowGradLds L;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int col = lane & 15, kq = lane >> 4;
+  const int r0 = blockIdx.x * rows_per, r1 = min(R, r0 + rows_per);
+  float4_t acc2[kH2 / 16], acc1 = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int j = 0; j < kH2 / 16; ++j) acc2[j] = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
+  float csum = 0.0f;  // thread t < 128: column t of dH2; t < 192: column t - 128 of dH1
+  for (int t0 = r0; t0 < r1; t0 += kRgTile) {
+    __syncthreads();
+    {
+      const int r = tid >> 2, q = tid & 3;
+      const int64_t row = (int64_t)t0 + r;
+      stage_transposed<kH1, 16>(H1g, row, r, q * 16, L.h1);
+      stage_transposed<kH2, 32>(dH2, row, r, q * 32, L.d2);
+      stage_transposed<kMlpInPad, 4>(Xg, row, r, q * 4, L.x);
+      stage_transposed<kH1, 16>(dH1, row, r, q * 16, L.d1);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int ks = 0; ks < kRgTile; ks += 32) {
+      const bf16x8_t a2 = lds8(&L.h1[wave * 16 + col][ks + kq * 8]);
+#pragma unroll
+      for (int j = 0; j < kH2 / 16; ++j)
+        acc2[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, lds8(&L.d2[j * 16 + col][ks + kq * 8]), acc2[j], 0, 0, 0);
+      acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lds8(&L.x[col][ks + kq * 8]),
+                                                     lds8(&L.d1[wave * 16 + col][ks + kq * 8]), acc1, 0, 0, 0);
+    }
+    if (tid < kH2 + kH1) {
+      const uint16_t* c = tid < kH2 ? L.d2[tid] : L.d1[tid - kH2];
+#pragma unroll
+      for (int k = 0; k < kRgTile; k += 2) {
+        const uint32_t v = *reinterpret_cast<const uint32_t*>(c + k);
+        csum += bf2f((uint16_t)v);
+        csum += bf2f((uint16_t)(v >> 16));
+      }
+    }
+  }
+  // lane: rows (lane >> 4) * 4 + v, column lane & 15 of each 16 x 16 tile
+  float* out = part + (size_t)blockIdx.x * kRgPart;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+#pragma unroll
+    for (int j = 0; j < kH2 / 16; ++j) out[(wave * 16 + kq * 4 + v) * kH2 + j * 16 + col] = acc2[j][v];
+    out[kH1 * kH2 + (kq * 4 + v) * kH1 + wave * 16 + col] = acc1[v];
+  }
+  if (tid < kH2 + kH1) out[kH1 * kH2 + kMlpInPad * kH1 + tid] = csum;
+}
+
+__global__ __launch_bounds__(256) void mlp_rowgrad_sum_kernel(const float* __restrict__ part, int n_parts,
+                                                              float* __restrict__ grad) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= kRgPart) return;
+  float s = 0.0f;
+#pragma unroll 8
+  for (int p = 0; p < n_parts; ++p) s += part[(size_t)p * kRgPart + i];
+  constexpr int o1 = kH1 * kH2, o2 = o1 + kMlpInPad * kH1, o3 = o2 + kH2;
+  if (i < o1) grad[oW2 + i] = s;
+  else if (i < o1 + kMlpIn * kH1) grad[oW1 + i - o1] = s;
+  else if (i >= o3) grad[oB1 + i - o3] = s;
+  else if (i >= o2) grad[oB2 + i - o2] = s;
 }
 
 // Column sums of an M x N matrix (FP32 or BF16), one block per column, fixed
@@ -839,7 +935,7 @@ namespace {
 
 enum {
   WS_PTS = 0, WS_X, WS_CEN, WS_H1, WS_H2, WS_POOL, WS_Z, WS_GVAL, WS_GARG, WS_Z1, WS_O, WS_TGT, WS_DO, WS_DOB,
-  WS_DZ1, WS_DZ, WS_ROWV, WS_XG, WS_H1G, WS_DH2, WS_DH1, WS_LOSS, WS_QT, WS_CONF, WS_STAGE, WS_COUNT
+  WS_DZ1, WS_DZ, WS_ROWV, WS_XG, WS_H1G, WS_DH2, WS_DH1, WS_LOSS, WS_QT, WS_CONF, WS_STAGE, WS_PART, WS_COUNT
 };
 static_assert(WS_COUNT <= 32, "the model's workspace array holds 32 buffers");
 
@@ -848,22 +944,28 @@ T* wsp(cvo_model* m, int i) {
   return reinterpret_cast<T*>(m->ws[i].p);
 }
 
+// Blocks a cloud's points are split over: enough for every compute unit when
+// the clouds alone are too few, at most one per tile.
+int encoder_splits(int clouds, int npts) {
+  return std::max(1, std::min((npts + kFT - 1) / kFT, 256 / clouds));
+}
+
 // Forward over n_pairs pairs of npts points; inputs already in WS_PTS
-// ([pair][cloud][point][8] FP32).  Leaves z1 (BF16) and o (FP32).  fused:
-// the point encoder in one kernel (inference); otherwise layer by layer with
-// the activations h1, h2 kept for the backward pass (training).
-cvo_status forward(cvo_model* m, int n_pairs, int npts, bool fused = false) {
+// ([pair][cloud][point][8] FP32).  Leaves z1 (BF16) and o (FP32).  train: keeps
+// the activations h1, h2 for the backward pass.
+cvo_status forward(cvo_model* m, int n_pairs, int npts, bool train) {
   cvo_ctx* ctx = m->ctx;
   hipStream_t s = ctx->stream;
   const int clouds = 2 * n_pairs;
   const int64_t P = (int64_t)clouds * npts;
   CVO_TRY(ensure(ctx, m->ws[WS_X], sizeof(uint16_t) * P * kMlpInPad));
   CVO_TRY(ensure(ctx, m->ws[WS_CEN], sizeof(float) * 12 * clouds));
-  if (!fused) {
+  if (train) {
     CVO_TRY(ensure(ctx, m->ws[WS_H1], sizeof(uint16_t) * P * kH1));
     CVO_TRY(ensure(ctx, m->ws[WS_H2], sizeof(uint16_t) * P * kH2));
   }
-  CVO_TRY(ensure(ctx, m->ws[WS_POOL], sizeof(unsigned long long) * clouds * kH3));
+  const int splits = encoder_splits(clouds, npts);
+  CVO_TRY(ensure(ctx, m->ws[WS_POOL], sizeof(unsigned long long) * clouds * splits * kH3));
   CVO_TRY(ensure(ctx, m->ws[WS_Z], sizeof(uint16_t) * n_pairs * kZ));
   CVO_TRY(ensure(ctx, m->ws[WS_GVAL], sizeof(float) * clouds * kH3));
   CVO_TRY(ensure(ctx, m->ws[WS_GARG], sizeof(int32_t) * clouds * kH3));
@@ -874,36 +976,12 @@ cvo_status forward(cvo_model* m, int n_pairs, int npts, bool fused = false) {
   const float* w = m->w;
   const int64_t npool = (int64_t)clouds * kH3;
   GemmArgs g;
-  if (fused) {
-    hipLaunchKernelGGL(encoder_fused_kernel, dim3(clouds), dim3(256), 0, s, wsp<uint16_t>(m, WS_X), npts, m->W1b,
-                       m->W2b, m->W3b, w, wsp<unsigned long long>(m, WS_POOL));
-  } else {
-  // layer 1: 16 (padded) -> 64
-  g = gemm_args(wsp<uint16_t>(m, WS_X), kMlpInPad, 1, m->W1b, kH1, 1, (int)P, kH1, kMlpInPad);
-  g.bias = w + oB1;
-  g.relu = 1;
-  g.Cb = wsp<uint16_t>(m, WS_H1);
-  g.ldcb = kH1;
-  gemm(g, s);
-  // layer 2: 64 -> 128
-  g = gemm_args(wsp<uint16_t>(m, WS_H1), kH1, 1, m->W2b, kH2, 1, (int)P, kH2, kH1);
-  g.bias = w + oB2;
-  g.relu = 1;
-  g.Cb = wsp<uint16_t>(m, WS_H2);
-  g.ldcb = kH2;
-  gemm(g, s);
-  // layer 3: 128 -> 256 with the max-pool epilogue
-  hipLaunchKernelGGL(fill_u64_kernel, dim3((unsigned)((npool + 255) / 256)), dim3(256), 0, s,
-                     wsp<unsigned long long>(m, WS_POOL), npool, 0ull);
-  g = gemm_args(wsp<uint16_t>(m, WS_H2), kH2, 1, m->W3b, kH3, 1, (int)P, kH3, kH2);
-  g.bias = w + oB3;
-  g.relu = 1;
-  g.pool = wsp<unsigned long long>(m, WS_POOL);
-  g.group = npts;
-  gemm(g, s);
-  }
+  hipLaunchKernelGGL(train ? encoder_fused_kernel<true> : encoder_fused_kernel<false>, dim3(clouds * splits), dim3(256),
+                     0, s, wsp<uint16_t>(m, WS_X), npts, m->W1b, m->W2b, m->W3b, w,
+                     wsp<unsigned long long>(m, WS_POOL), splits, train ? wsp<uint16_t>(m, WS_H1) : nullptr,
+                     train ? wsp<uint16_t>(m, WS_H2) : nullptr);
   hipLaunchKernelGGL(mlp_unpack_pool_kernel, dim3((unsigned)((npool + 255) / 256)), dim3(256), 0, s,
-                     wsp<unsigned long long>(m, WS_POOL), n_pairs, wsp<uint16_t>(m, WS_Z), wsp<float>(m, WS_GVAL),
+                     wsp<unsigned long long>(m, WS_POOL), splits, n_pairs, wsp<uint16_t>(m, WS_Z), wsp<float>(m, WS_GVAL),
                      wsp<int32_t>(m, WS_GARG));
   // head
   g = gemm_args(wsp<uint16_t>(m, WS_Z), kZ, 1, m->W4b, kZ1, 1, n_pairs, kZ1, kZ);
@@ -1053,7 +1131,7 @@ extern "C" cvo_status cvo_model_gradient(cvo_ctx* ctx, cvo_model* m, int32_t n_p
   CVO_TRY(check_batch(ctx, n_pairs, npts));
   hipStream_t s = ctx->stream;
   CVO_TRY(upload_points(m, n_pairs, npts, a, b, false));
-  CVO_TRY(forward(m, n_pairs, npts));
+  CVO_TRY(forward(m, n_pairs, npts, true));
   const int clouds = 2 * n_pairs;
   const int R = clouds * kH3;
   CVO_TRY(ensure(ctx, m->ws[WS_TGT], sizeof(float) * 7 * n_pairs));
@@ -1067,6 +1145,9 @@ extern "C" cvo_status cvo_model_gradient(cvo_ctx* ctx, cvo_model* m, int32_t n_p
   CVO_TRY(ensure(ctx, m->ws[WS_DH2], sizeof(uint16_t) * (size_t)R * kH2));
   CVO_TRY(ensure(ctx, m->ws[WS_DH1], sizeof(uint16_t) * (size_t)R * kH1));
   CVO_TRY(ensure(ctx, m->ws[WS_LOSS], sizeof(float) * n_pairs));
+  // at most 128 partials, of at least two tiles (R = 512 rows a pair)
+  const int rows_per = std::max(2, (R / kRgTile + 127) / 128) * kRgTile, parts = (R + rows_per - 1) / rows_per;
+  CVO_TRY(ensure(ctx, m->ws[WS_PART], sizeof(float) * (size_t)parts * kRgPart));
   CVO_HIP(ctx, hipMemcpyAsync(m->ws[WS_TGT].p, targets, sizeof(float) * 7 * n_pairs, hipMemcpyHostToDevice, s));
   hipLaunchKernelGGL(mlp_loss_kernel, dim3((n_pairs + 63) / 64), dim3(64), 0, s, wsp<float>(m, WS_O),
                      wsp<float>(m, WS_TGT), wsp<float>(m, WS_CEN), n_pairs, wsp<float>(m, WS_DO),
@@ -1102,28 +1183,20 @@ extern "C" cvo_status cvo_model_gradient(cvo_ctx* ctx, cvo_model* m, int32_t n_p
                      wsp<int32_t>(m, WS_GARG), npts, wsp<uint16_t>(m, WS_X), wsp<uint16_t>(m, WS_H1),
                      wsp<uint16_t>(m, WS_H2), m->W3b, wsp<uint16_t>(m, WS_XG), wsp<uint16_t>(m, WS_H1G),
                      wsp<uint16_t>(m, WS_DH2), wsp<float>(m, WS_ROWV));
-  hipLaunchKernelGGL(mlp_dw3_kernel, dim3((kH2 * kH3 + 255) / 256), dim3(256), 0, s, wsp<float>(m, WS_ROWV),
+  hipLaunchKernelGGL(mlp_dw3_kernel, dim3(kH3), dim3(kH2), 0, s, wsp<float>(m, WS_ROWV),
                      wsp<int32_t>(m, WS_GARG), clouds, npts, wsp<uint16_t>(m, WS_H2), gr + oW3, gr + oB3);
-  // dW2 = H1g^T dH2, db2 = colsum(dH2), dH1 = (dH2 W2^T) * [H1g > 0]
-  g = gemm_args(wsp<uint16_t>(m, WS_H1G), 1, kH1, wsp<uint16_t>(m, WS_DH2), kH2, 1, kH1, kH2, R);
-  g.C = gr + oW2;
-  g.ldc = kH2;
-  gemm(g, s);
-  hipLaunchKernelGGL(mlp_colsum_kernel, dim3(kH2), dim3(256), 0, s, nullptr, wsp<uint16_t>(m, WS_DH2), R, kH2,
-                     gr + oB2);
+  // dH1 = (dH2 W2^T) * [H1g > 0], then the weight gradients of both layers
   g = gemm_args(wsp<uint16_t>(m, WS_DH2), kH2, 1, m->W2b, 1, kH2, R, kH1, kH2);
   g.mask = wsp<uint16_t>(m, WS_H1G);
   g.ldm = kH1;
   g.Cb = wsp<uint16_t>(m, WS_DH1);
   g.ldcb = kH1;
   gemm(g, s);
-  // dW1 = Xg^T dH1 (first 8 input rows), db1 = colsum(dH1)
-  g = gemm_args(wsp<uint16_t>(m, WS_XG), 1, kMlpInPad, wsp<uint16_t>(m, WS_DH1), kH1, 1, kMlpIn, kH1, R);
-  g.C = gr + oW1;
-  g.ldc = kH1;
-  gemm(g, s);
-  hipLaunchKernelGGL(mlp_colsum_kernel, dim3(kH1), dim3(256), 0, s, nullptr, wsp<uint16_t>(m, WS_DH1), R, kH1,
-                     gr + oB1);
+  hipLaunchKernelGGL(mlp_rowgrad_kernel, dim3(parts), dim3(256), 0, s, wsp<uint16_t>(m, WS_H1G),
+                     wsp<uint16_t>(m, WS_DH2), wsp<uint16_t>(m, WS_XG), wsp<uint16_t>(m, WS_DH1), R, rows_per,
+                     wsp<float>(m, WS_PART));
+  hipLaunchKernelGGL(mlp_rowgrad_sum_kernel, dim3((kRgPart + 255) / 256), dim3(256), 0, s, wsp<float>(m, WS_PART), parts,
+                     gr);
   CVO_HIP(ctx, hipGetLastError());
   if (grad_out) {
     CVO_HIP(ctx, hipMemcpyAsync(grad_out, gr, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost, s));
@@ -1166,7 +1239,7 @@ static cvo_status propose_impl(cvo_ctx* ctx, const cvo_model* mc, int32_t n_pair
     CVO_TRY(ensure_events(ctx, 2));
     CVO_HIP(ctx, hipEventRecord(ctx->ev_pool[0], s));
   }
-  CVO_TRY(forward(m, n_pairs, npts, true));
+  CVO_TRY(forward(m, n_pairs, npts, false));
   if (ctx->profiling) {
     CVO_HIP(ctx, hipEventRecord(ctx->ev_pool[1], s));
     CVO_HIP(ctx, hipEventSynchronize(ctx->ev_pool[1]));

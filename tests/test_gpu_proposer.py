@@ -114,3 +114,28 @@ def test_training_reduces_loss(cvo_gpu):
         last = p.train_step(a, b, t, 1e-3)
     p.close()
     assert last < 0.7 * first, (first, last)
+
+
+@pytest.mark.parametrize("n,npts", [(1, 64), (2, 192), (3, 640), (130, 128)])
+def test_split_clouds_match_oracle(prop, n, npts):
+    """Forward and gradient where a cloud's points are one wave's rows, part of a
+    tile, several tiles over several blocks, and one block a cloud (260 clouds);
+    rows of the weight gradients in two tiles a block and more."""
+    a, b, t = batch(5, min(n, 3), npts)
+    reps = -(-n // a.shape[0])
+    a, b, t = (np.tile(x, (reps,) + (1,) * (x.ndim - 1))[:n] for x in (a, b, t))
+    w = prop.get_weights().astype(np.float64)
+    say(f"proposer split {n} pairs x {npts}")
+    _, _, raw = prop.propose(a, b)
+    k = min(n, 3)
+    o, _ = M.forward(w, a[:k].astype(np.float64), b[:k].astype(np.float64), quantize=True)
+    assert rel(raw[:k], o) < 1e-2
+    # a pair's proposals do not depend on how its clouds are split
+    _, _, alone = prop.propose(a[:1], b[:1])
+    assert np.array_equal(alone[0], raw[0])
+    loss, g = prop.gradient(a, b, t)
+    if n > 3:
+        return
+    Lo, go = M.gradient(w, a.astype(np.float64), b.astype(np.float64), t.astype(np.float64), quantize=True)
+    assert abs(loss - Lo) <= 1e-2 * abs(Lo)
+    assert rel(g, go) < 1e-2
