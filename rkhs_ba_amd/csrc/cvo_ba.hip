@@ -9,7 +9,8 @@
 //   assoc / overflow  per-edge association between the frames' world points,
 //                     with per-edge stored pairs and largest row
 //   ba_edges          edge on/off; stop when no edge has enough pairs
-//   (ba_pair -> ba_edge_reduce -> ba_solve) x (iterations_per_solve + 1)
+//   ba_moments        per-edge moments of the stored pairs
+//   (ba_eval -> ba_assemble -> ba_solve) x (iterations_per_solve + 1)
 //                     Levenberg-Marquardt over the fixed pairs
 //   ba_finish         per-edge lengthscale, pose change, convergence
 //
@@ -19,7 +20,18 @@
 // parameterisation T <- T Exp([rho; phi]) (local_parameterization_se3.hpp:
 // 21-99).  With w = P1 - P2 (world), u = [w; P1 x w] the local Jacobians are
 // j1 = M1 u and j2 = -M2 u, M = [[R^T, 0], [-R^T [t]x, R^T]], so each edge only
-// accumulates S = sum u u^T, h = sum r u and c = sum r^2 over its pairs.
+// needs S = sum u u^T, h = sum r u and c = sum r^2 over its pairs.
+//
+// These are polynomials in the poses: with A = T2^-1 T1 (3x4), A0 the same at the
+// poses of the association, d0 = A0 p~ - p2 (a pair's offset in frame 2 then) and
+// e = (A - A0) p~, R2^T w = d = d0 + e.  So the pairs are read once an outer
+// iteration, into sums over them of {1, d0, d0 d0^T}, a {1, d0, d0 d0^T, |d0|^2 d0}
+// and a^2 {1, d0, d0 d0^T, |d0|^2 d0, |d0|^4} times the monomials of p1 up to the
+// degree that each meets, and every candidate of the solve evaluates the
+// polynomials.  d0 is small (the association's radius) and p1 is taken about its
+// cloud's centre, so that the expansion loses no digits: the poses of a 12-frame
+// window after 12 outer iterations equal those of sums over the pairs at every
+// candidate to 2e-16 (relative).
 //
 // The Ceres solve is replaced by this Levenberg-Marquardt schedule:
 //   D = clamp(diag(H), 1e-6, 1e32); solve (H + D/mu) d = -g;
@@ -50,10 +62,10 @@ constexpr int kBaMaxFrames = 64;
 constexpr int kBaMaxFree = 20;                 // free frames: 120 dof, Cholesky in 115 KB of LDS
 constexpr int kBaMaxDof = 6 * kBaMaxFree;
 constexpr int kBaMaxEdges = 4096;
-constexpr int kBaTerms = 28;                   // S (21, upper triangle), h (6), c (1)
 constexpr int kBaContrib = 121;                // B11, B12, B22 (36 each), g1, g2 (6 each), c
-constexpr int kBaRowsPerBlock = 256;           // pair pass: one row per thread
-constexpr int kPairLoads = 4;                  // pair pass: loads in flight per lane
+constexpr int kMomRows = 512;                  // source rows of a moment block
+constexpr int kMomTiles = 5;                   // 16 x 16 tiles of the moment matrix that are used
+constexpr int kMomPart = kMomTiles * 256;
 constexpr int kSolveThreads = 256;             // four waves: the Cholesky's trailing update spread over rows
 static_assert(kSolveThreads == 256 && 6 * kBaMaxFree <= kSolveThreads, "the solve's reductions assume four waves");
 constexpr int kChol = 8;                       // Cholesky block: columns a panel
@@ -64,7 +76,7 @@ struct BaEdge {
   int64_t nnz, nnz_last;
   int32_t f1, f2;
   int32_t K, last_max, iters_per_ell, on;
-  int32_t n_rows, n_pair_blocks;
+  int32_t n_rows, n_blocks;
   int32_t pad0, pad1;
 };
 
@@ -81,6 +93,7 @@ struct BaDev {
   int32_t free_idx[kBaMaxFrames];
   int32_t frame_of_free[kBaMaxFree];
   float frame_norm[kBaMaxFrames];
+  double centre[kBaMaxFrames * 3];  // of each cloud, in its frame
   double X[kBaMaxFrames * 12];     // current poses, row-major 3x4 (world <- sensor)
   double Xe[kBaMaxFrames * 12];    // poses of the pending pair pass
   double Xold[kBaMaxFrames * 12];  // poses at the start of the outer iteration
@@ -221,161 +234,485 @@ __global__ __launch_bounds__(256) void ba_edges_kernel(BaDev* __restrict__ ba, B
   }
 }
 
-// FP64 pair pass at the poses Xe, block partials of S (21), h (6), c (1).
-// Each wave takes 64 source rows of one edge (lane i owns row i and its world
-// point), prefix-sums their pair counts and spreads the flattened pairs over
-// its lanes, so every lane's loads are independent and the lanes stay busy
-// whatever the row lengths.
-__global__ __launch_bounds__(kBaRowsPerBlock) void ba_pair_kernel(const BaDev* __restrict__ ba,
-                                                                  const BaEdge* __restrict__ edges,
-                                                                  const AssocProblem* __restrict__ probs,
-                                                                  double* __restrict__ part, int max_blocks) {
-  if (ba->done || !ba->eval_pending) return;
-  const int e = blockIdx.y;
-  const BaEdge& ed = edges[e];
-  if (!ed.on || (int)blockIdx.x >= ed.n_pair_blocks) return;
-  const AssocProblem& P = probs[e];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wr0 = blockIdx.x * kBaRowsPerBlock + wave * 64;
-  // pairs are stored at the row stride of this iteration's cap (the
-  // reference re-strides its pair matrix the same way)
-  const size_t row_stride = (size_t)P.st->K;
-  double T1[12], T2[12];
-#pragma unroll
-  for (int i = 0; i < 12; ++i) {
-    T1[i] = ba->Xe[12 * ed.f1 + i];
-    T2[i] = ba->Xe[12 * ed.f2 + i];
+// ---------------------------------------------------------------------------
+// Moments of an edge's pairs
+// ---------------------------------------------------------------------------
+
+// Monomials x^i y^j z^k of degree <= 4, by degree: 1; x, y, z; xx, xy, xz, yy,
+// yz, zz; 10 of degree 3; 15 of degree 4.  The first 4 carry a linear form, the
+// first 10 a quadratic one.
+constexpr int kMono = 35, kQuad = 10, kLin = 4;
+struct MonoTables {
+  int8_t mul[kQuad][kQuad];  // index of the product of two of the first ten
+  constexpr MonoTables() : mul() {
+    int e[kMono][3] = {};
+    int n = 0;
+    for (int d = 0; d <= 4; ++d)
+      for (int i = d; i >= 0; --i)
+        for (int j = d - i; j >= 0; --j) {
+          e[n][0] = i;
+          e[n][1] = j;
+          e[n][2] = d - i - j;
+          ++n;
+        }
+    for (int a = 0; a < kQuad; ++a)
+      for (int b = 0; b < kQuad; ++b)
+        for (int m = 0; m < kMono; ++m)
+          if (e[m][0] == e[a][0] + e[b][0] && e[m][1] == e[a][1] + e[b][1] && e[m][2] == e[a][2] + e[b][2])
+            mul[a][b] = (int8_t)m;
   }
-  // the lane's own row: world point and pair count
-  const int r_own = wr0 + lane;
-  uint32_t cnt = 0;
-  double X0 = 0.0, X1 = 0.0, X2 = 0.0;
-  if (r_own < P.n_src) {
-    cnt = ld_global(P.counts + r_own);
-    const float4 x4 = ld_global(P.src_pos + r_own);
-    const double p0 = x4.x, p1 = x4.y, p2 = x4.z;
-    X0 = fma(T1[2], p2, fma(T1[1], p1, fma(T1[0], p0, T1[3])));
-    X1 = fma(T1[6], p2, fma(T1[5], p1, fma(T1[4], p0, T1[7])));
-    X2 = fma(T1[10], p2, fma(T1[9], p1, fma(T1[8], p0, T1[11])));
-  }
-  uint32_t incl = cnt;
+};
+__constant__ MonoTables kMonoTab;
+
+// Row moments and where their sums lie.  The moment matrix has 37 rows (a sum
+// over a source row's pairs each) by 35 monomials of the row's point; rows are
+// laid out so that 16 x 16 tiles hold what is used: tile row 0 the moments of
+// degree 0 and 1 in d0, which meet monomials up to degree 4 (tiles 0, 1, 2), tile
+// rows 1 and 2 those of degree 2 to 4, which meet degree <= 2 (tiles 3, 4).
+constexpr int kM_n = 0, kM_a0 = 1, kM_b0 = 2, kM_D1 = 3, kM_a1 = 6, kM_b1 = 9;
+constexpr int kM_D2 = 16, kM_a2 = 22, kM_b2 = 28, kM_a3 = 34, kM_b3 = 37, kM_b4 = 40, kMomRowsUsed = 41;
+
+// Sum of moment m times monomial q in the summed tiles.
+__device__ __forceinline__ double mom(const double* s_m, int m, int q) {
+  const int tile = m < 16 ? q >> 4 : 2 + (m >> 4);
+  return s_m[tile * 256 + (m & 15) * 16 + (q & 15)];
+}
+
+// The relative map T2^-1 T1 (row-major 3x4) of two poses.
+__device__ __forceinline__ void relative_map(const double* T1, const double* T2, double A[12]) {
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t t = __shfl_up(incl, o, 64);
-    if (lane >= o) incl += t;
-  }
-  const uint32_t total = __shfl(incl, 63, 64);
-  const uint32_t excl = incl - cnt;
-  double acc[kBaTerms];
+  for (int r = 0; r < 3; ++r) {
 #pragma unroll
-  for (int k = 0; k < kBaTerms; ++k) acc[k] = 0.0;
-  // kPairLoads pairs a lane a trip: the loads go out unconditionally (past
-  // the end a lane reloads the last pair, which it then skips) so that all
-  // are in flight before the first is used, then the pairs are summed in
-  // flattened order, lane by lane as one pair a trip would
-  for (uint32_t base = 0; base < total; base += 64 * kPairLoads) {
-    int kr[kPairLoads];
-    float4 yv[kPairLoads];
-#pragma unroll
-    for (int u = 0; u < kPairLoads; ++u) {
-      const uint32_t idx = min(base + (uint32_t)(u * 64 + lane), total - 1);
-      // row of flattened pair idx: the last lane whose exclusive offset <= idx
-      int k = 0;
-#pragma unroll
-      for (int s = 32; s > 0; s >>= 1) {
-        const uint32_t ex = __shfl(excl, k + s, 64);
-        if (ex <= idx) k += s;
-      }
-      const uint32_t slot = idx - __shfl(excl, k, 64);
-      kr[u] = k;
-      yv[u] = ld_global(P.pairs4 + (size_t)(wr0 + k) * row_stride + slot);
-    }
-#pragma unroll
-    for (int t = 0; t < kPairLoads; ++t) {
-      const int k = kr[t];
-      const double Y0 = __shfl(X0, k, 64), Y1 = __shfl(X1, k, 64), Y2 = __shfl(X2, k, 64);
-      if (base + (uint32_t)(t * 64 + lane) < total) {
-        // FP64 with explicit fused multiply-adds (the library is built with
-        // contraction off for the FP32 gates)
-        const float4 y4 = yv[t];
-        const double a = (double)y4.w;
-        const double q0 = y4.x, q1 = y4.y, q2 = y4.z;
-        const double w0 = Y0 - fma(T2[2], q2, fma(T2[1], q1, fma(T2[0], q0, T2[3])));
-        const double w1 = Y1 - fma(T2[6], q2, fma(T2[5], q1, fma(T2[4], q0, T2[7])));
-        const double w2 = Y2 - fma(T2[10], q2, fma(T2[9], q1, fma(T2[8], q0, T2[11])));
-        const double res = a * fma(w2, w2, fma(w1, w1, w0 * w0));
-        const double u[6] = {w0, w1, w2, fma(Y1, w2, -Y2 * w1), fma(Y2, w0, -Y0 * w2), fma(Y0, w1, -Y1 * w0)};
-        int q = 0;
-#pragma unroll
-        for (int i = 0; i < 6; ++i)
-#pragma unroll
-          for (int j = i; j < 6; ++j) {
-            acc[q] = fma(u[i], u[j], acc[q]);
-            ++q;
-          }
-#pragma unroll
-        for (int i = 0; i < 6; ++i) acc[21 + i] = fma(res, u[i], acc[21 + i]);
-        acc[27] = fma(res, res, acc[27]);
-      }
-    }
-  }
-  // fixed-order block partial: wave shuffles, then the four waves in LDS
-  __shared__ double s_w[kBaTerms][kBaRowsPerBlock / 64];
-#pragma unroll
-  for (int k = 0; k < kBaTerms; ++k) {
-    double v = acc[k];
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    if (lane == 0) s_w[k][wave] = v;
-  }
-  __syncthreads();
-  if (tid < kBaTerms) {
-    double v = 0.0;
-    for (int w = 0; w < kBaRowsPerBlock / 64; ++w) v += s_w[tid][w];
-    part[((size_t)e * max_blocks + blockIdx.x) * kBaTerms + tid] = v;
+    for (int c = 0; c < 3; ++c)
+      A[r * 4 + c] = fma(T2[8 + r], T1[8 + c], fma(T2[4 + r], T1[4 + c], T2[r] * T1[c]));
+    A[r * 4 + 3] = fma(T2[8 + r], T1[11] - T2[11], fma(T2[4 + r], T1[7] - T2[7], T2[r] * (T1[3] - T2[3])));
   }
 }
 
-// Per-edge totals of the pair pass and the edge's blocks of the normal
-// equations at the poses Xe: B11 = M1 S M1^T, B12 = -M1 S M2^T,
-// B22 = M2 S M2^T, g1 = M1 h, g2 = -M2 h.
-__global__ __launch_bounds__(256) void ba_edge_reduce_kernel(const BaDev* __restrict__ ba,
+// The pairs' moments, once an outer iteration (at the association's poses, X).
+// A lane owns a source row and reads its pairs in order, four loads in flight;
+// FP64 sums of 37 moments in registers.  Then the wave's 64 rows times their
+// monomials: sums over rows of products, so FP64 matrix instructions
+// (v_mfma_f64_16x16x4, 16 rows of the cloud staged in LDS at a time).  Block
+// partials of the five tiles.  Bound by FP64 issue and the rows' uneven lengths;
+// a pass over the pairs of each candidate took 187 us and 11 for its sums, nine
+// times an outer iteration (window of 12 frames of 5k to 40k points), this 298 us
+// once and 8 us for each candidate's polynomials (window: 61.7 -> 45.3 ms for 12 outer
+// iterations).
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void ba_moments_kernel(const BaDev* __restrict__ ba, const BaEdge* __restrict__ edges,
+                                                         const AssocProblem* __restrict__ probs,
+                                                         double* __restrict__ part, int max_blocks) {
+  if (ba->done || !ba->eval_pending) return;
+  const int e = blockIdx.y;
+  const BaEdge& ed = edges[e];
+  if (!ed.on || (int)blockIdx.x >= ed.n_blocks) return;
+  const AssocProblem& P = probs[e];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  typedef double double4_t __attribute__((ext_vector_type(4)));
+  constexpr int kSM = 49, kSQ = 49;  // doubles a staged row of moments / monomials (odd: no bank pattern)
+  __shared__ double s_stage[4][16 * (kSM + kSQ)];
+  double* s_m = s_stage[wave];
+  double* s_q = s_m + 16 * kSM;
+  // pairs are stored at the row stride of this iteration's cap (the
+  // reference re-strides its pair matrix the same way)
+  const size_t row_stride = (size_t)P.st->K;
+  double A[12];
+  relative_map(ba->X + 12 * ed.f1, ba->X + 12 * ed.f2, A);
+  const double c0 = ba->centre[3 * ed.f1], c1 = ba->centre[3 * ed.f1 + 1], c2 = ba->centre[3 * ed.f1 + 2];
+  double4_t acc[kMomTiles];
+#pragma unroll
+  for (int t = 0; t < kMomTiles; ++t) acc[t] = (double4_t){0.0, 0.0, 0.0, 0.0};
+  for (int base = blockIdx.x * kMomRows; base < (int)(blockIdx.x + 1) * kMomRows && base < P.n_src; base += 256) {
+    const int r = base + wave * 64 + lane;
+    uint32_t cnt = 0;
+    double y0 = 0.0, y1 = 0.0, y2 = 0.0, x = 0.0, y = 0.0, z = 0.0;
+    if (r < P.n_src) {
+      cnt = ld_global(P.counts + r);
+      const float4 p4 = ld_global(P.src_pos + r);
+      const double p0 = p4.x, p1 = p4.y, p2 = p4.z;
+      y0 = fma(A[2], p2, fma(A[1], p1, fma(A[0], p0, A[3])));
+      y1 = fma(A[6], p2, fma(A[5], p1, fma(A[4], p0, A[7])));
+      y2 = fma(A[10], p2, fma(A[9], p1, fma(A[8], p0, A[11])));
+      x = p0 - c0;
+      y = p1 - c1;
+      z = p2 - c2;
+    }
+    if (__ballot(cnt != 0) == 0ull) continue;  // the wave's rows hold no pair
+    double D1[3] = {}, D2[6] = {}, a0 = 0.0, a1[3] = {}, a2[6] = {}, a3[3] = {};
+    double b0 = 0.0, b1[3] = {}, b2[6] = {}, b3[3] = {}, b4 = 0.0;
+    auto add = [&](const float4& q) {
+      const double d[3] = {y0 - (double)q.x, y1 - (double)q.y, y2 - (double)q.z};
+      const double a = (double)q.w, b = a * a;
+      const double n2 = fma(d[2], d[2], fma(d[1], d[1], d[0] * d[0]));
+      const double an = a * n2, bn = b * n2;
+      a0 += a;
+      b0 += b;
+      b4 = fma(bn, n2, b4);
+      int k = 0;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        D1[i] += d[i];
+        a1[i] = fma(a, d[i], a1[i]);
+        b1[i] = fma(b, d[i], b1[i]);
+        a3[i] = fma(an, d[i], a3[i]);
+        b3[i] = fma(bn, d[i], b3[i]);
+#pragma unroll
+        for (int j = i; j < 3; ++j) {
+          const double dd = d[i] * d[j];
+          D2[k] += dd;
+          a2[k] = fma(a, dd, a2[k]);
+          b2[k] = fma(b, dd, b2[k]);
+          ++k;
+        }
+      }
+    };
+    {
+      const float4* row = P.pairs4 + (size_t)r * row_stride;
+      uint32_t s = 0;
+      for (; s + 4 <= cnt; s += 4) {
+        const float4 q0 = ld_global(row + s), q1 = ld_global(row + s + 1), q2 = ld_global(row + s + 2),
+                     q3 = ld_global(row + s + 3);
+        add(q0);
+        add(q1);
+        add(q2);
+        add(q3);
+      }
+      for (; s < cnt; ++s) add(ld_global(row + s));
+    }
+#pragma unroll 1
+    for (int quarter = 0; quarter < 4; ++quarter) {
+      if ((lane >> 4) == quarter) {
+        double* m = s_m + (lane & 15) * kSM;
+        double* q = s_q + (lane & 15) * kSQ;
+        m[kM_n] = (double)cnt;
+        m[kM_a0] = a0;
+        m[kM_b0] = b0;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          m[kM_D1 + i] = D1[i];
+          m[kM_a1 + i] = a1[i];
+          m[kM_b1 + i] = b1[i];
+          m[kM_a3 + i] = a3[i];
+          m[kM_b3 + i] = b3[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 6; ++i) {
+          m[kM_D2 + i] = D2[i];
+          m[kM_a2 + i] = a2[i];
+          m[kM_b2 + i] = b2[i];
+        }
+#pragma unroll
+        for (int i = 12; i < 16; ++i) m[i] = 0.0;
+        m[kM_b4] = b4;
+#pragma unroll
+        for (int i = kMomRowsUsed; i < 48; ++i) m[i] = 0.0;
+        // monomials: those of degree d from those of degree d - 1
+        double v[kMono];
+        v[0] = 1.0;
+        v[1] = x;
+        v[2] = y;
+        v[3] = z;
+        v[4] = x * x;
+        v[5] = x * y;
+        v[6] = x * z;
+        v[7] = y * y;
+        v[8] = y * z;
+        v[9] = z * z;
+#pragma unroll
+        for (int i = 0; i < 6; ++i) v[10 + i] = x * v[4 + i];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) v[16 + i] = y * v[7 + i];
+        v[19] = z * v[9];
+#pragma unroll
+        for (int i = 0; i < 10; ++i) v[20 + i] = x * v[10 + i];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[30 + i] = y * v[16 + i];
+        v[34] = z * v[19];
+#pragma unroll
+        for (int i = 0; i < kMono; ++i) q[i] = v[i];
+#pragma unroll
+        for (int i = kMono; i < 48; ++i) q[i] = 0.0;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+      for (int k0 = 0; k0 < 16; k0 += 4) {
+        const double* m = s_m + (k0 + (lane >> 4)) * kSM + (lane & 15);
+        const double* q = s_q + (k0 + (lane >> 4)) * kSQ + (lane & 15);
+        const double m0 = m[0], q0 = q[0];
+        acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(m0, q0, acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(m0, q[16], acc[1], 0, 0, 0);
+        acc[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(m0, q[32], acc[2], 0, 0, 0);
+        acc[3] = __builtin_amdgcn_mfma_f64_16x16x4f64(m[16], q0, acc[3], 0, 0, 0);
+        acc[4] = __builtin_amdgcn_mfma_f64_16x16x4f64(m[32], q0, acc[4], 0, 0, 0);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+  }
+  // the four waves' tiles in order; lane: rows (lane >> 4) + 4 v, column lane & 15
+  double* out = part + ((size_t)e * max_blocks + blockIdx.x) * kMomPart;
+  static_assert(16 * (kSM + kSQ) >= kMomPart, "a wave's tiles fit its staging");
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < kMomTiles; ++t)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) s_stage[wave][t * 256 + ((lane >> 4) + 4 * v) * 16 + (lane & 15)] = acc[t][v];
+  __syncthreads();
+  for (int i = tid; i < kMomPart; i += 256)
+    out[i] = ((s_stage[0][i] + s_stage[1][i]) + s_stage[2][i]) + s_stage[3][i];
+}
+
+// An edge's moments: the blocks' partials in order.
+__global__ __launch_bounds__(256) void ba_moments_sum_kernel(const BaDev* __restrict__ ba,
                                                              const BaEdge* __restrict__ edges,
                                                              const double* __restrict__ part, int max_blocks,
-                                                             double* __restrict__ contrib) {
+                                                             double* __restrict__ moments) {
+  if (ba->done || !ba->eval_pending) return;
+  const int e = blockIdx.x;
+  const BaEdge& ed = edges[e];
+  if (!ed.on) return;
+  const int i = blockIdx.y * 256 + threadIdx.x;
+  const double* p = part + (size_t)e * max_blocks * kMomPart + i;
+  double v = 0.0;
+#pragma unroll 8
+  for (int b = 0; b < ed.n_blocks; ++b) v += p[(size_t)b * kMomPart];
+  moments[(size_t)e * kMomPart + i] = v;
+}
+
+// S, h and c of an edge at the poses Xe from its moments, and the edge's blocks
+// of the normal equations: B11 = M1 S M1^T, B12 = -M1 S M2^T, B22 = M2 S M2^T,
+// g1 = M1 h, g2 = -M2 h.  In frame 2 with u' = [d; s x d], s = A p~ + R2^T t2,
+// u = diag(R2, R2) u':
+//   V_ik[f] = sum f d_i d_k for f = 1, s_b, s_b s_c    (S')
+//   F_i[f] = sum f a |d|^2 d_i for f = 1, s_b          (h')
+// as polynomials over the monomials.  Four lanes per V and F entry (each a
+// quarter of the outer sum's terms, added in order), one wave for c.
+__global__ __launch_bounds__(384) void ba_eval_kernel(const BaDev* __restrict__ ba, const BaEdge* __restrict__ edges,
+                                                      const double* __restrict__ moments,
+                                                      double* __restrict__ contrib) {
   if (ba->done || !ba->eval_pending) return;
   const int e = blockIdx.x;
   const BaEdge& ed = edges[e];
   if (!ed.on) return;
   const int tid = threadIdx.x;
-  __shared__ double s_p[kBaTerms][8];
-  __shared__ double s_t[kBaTerms];
-  __shared__ double s_S[36], s_M1[36], s_M2[36], s_T1[36], s_T2[36];
-  if (tid < kBaTerms * 8) {
-    const int k = tid >> 3, l = tid & 7;
-    double v = 0.0;
-    for (int b = l; b < ed.n_pair_blocks; b += 8) v += part[((size_t)e * max_blocks + b) * kBaTerms + k];
-    s_p[k][l] = v;
+  __shared__ double s_m[kMomPart];
+  __shared__ double s_e[3][kLin];        // e_i over (1, x, y, z)
+  __shared__ double s_f[10][kQuad];      // 1; s_b; s_b s_c (00 01 02 11 12 22)
+  __shared__ double s_ee[6][kQuad];      // e_i e_k
+  __shared__ double s_g[kQuad];          // |e|^2
+  __shared__ double s_fe[12][kQuad];     // f e_i, f = 1, s_b
+  __shared__ double s_V[60], s_F[12], s_c;
+  __shared__ int8_t s_mul[kQuad][kQuad];
+  __shared__ double s_M1[36], s_M2[36], s_N1[36], s_N2[36], s_S[36], s_h[6], s_T1[36], s_T2[36];
+  for (int i = tid; i < kMomPart; i += blockDim.x) s_m[i] = moments[(size_t)e * kMomPart + i];
+  if (tid < kQuad * kQuad) s_mul[tid / kQuad][tid % kQuad] = kMonoTab.mul[tid / kQuad][tid % kQuad];
+  const double* T2 = ba->Xe + 12 * ed.f2;
+  if (tid == 128) pose_M(ba->Xe + 12 * ed.f1, s_M1);
+  if (tid == 192) pose_M(T2, s_M2);
+  if (tid < 3) {
+    double A[12], A0[12];
+    relative_map(ba->Xe + 12 * ed.f1, T2, A);
+    relative_map(ba->Xold + 12 * ed.f1, ba->Xold + 12 * ed.f2, A0);
+    const double* c = ba->centre + 3 * ed.f1;
+    const int r = tid;
+    double Ar[4], A0r[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {  // row r, without indexing registers
+      Ar[k] = r == 0 ? A[k] : (r == 1 ? A[4 + k] : A[8 + k]);
+      A0r[k] = r == 0 ? A0[k] : (r == 1 ? A0[4 + k] : A0[8 + k]);
+    }
+    const double at = fma(Ar[2], c[2], fma(Ar[1], c[1], fma(Ar[0], c[0], Ar[3])));
+    const double a0t = fma(A0r[2], c[2], fma(A0r[1], c[1], fma(A0r[0], c[0], A0r[3])));
+    // (R2^T t2)_r
+    const double tau = fma(T2[8 + r], T2[11], fma(T2[4 + r], T2[7], T2[r] * T2[3]));
+    s_e[r][0] = at - a0t;
+    s_f[1 + r][0] = at + tau;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      s_e[r][1 + k] = Ar[k] - A0r[k];
+      s_f[1 + r][1 + k] = Ar[k];
+    }
+#pragma unroll
+    for (int k = kLin; k < kQuad; ++k) s_f[1 + r][k] = 0.0;
   }
-  if (tid == 0) pose_M(ba->Xe + 12 * ed.f1, s_M1);
-  if (tid == 1) pose_M(ba->Xe + 12 * ed.f2, s_M2);
+  if (tid >= 64 && tid < 64 + kQuad) s_f[0][tid - 64] = tid == 64 ? 1.0 : 0.0;
   __syncthreads();
-  if (tid < kBaTerms) {
-    double v = 0.0;
-    for (int l = 0; l < 8; ++l) v += s_p[tid][l];
-    s_t[tid] = v;
+  // products of two linear forms: thread (form pair, monomial)
+  if (tid < 24 * kQuad) {
+    const int w = tid / kQuad, q = tid - w * kQuad;
+    const double* u;
+    const double* v;
+    double* out;
+    if (w < 12) {
+      const int k = w < 6 ? w : w - 6;
+      const int i = k < 3 ? 0 : (k < 5 ? 1 : 2), j = k < 3 ? k : (k < 5 ? k - 2 : 2);
+      u = w < 6 ? s_e[i] : s_f[1 + i];
+      v = w < 6 ? s_e[j] : s_f[1 + j];
+      out = w < 6 ? s_ee[k] : s_f[4 + k];
+    } else {
+      u = s_f[(w - 12) / 3];
+      v = s_e[(w - 12) % 3];
+      out = s_fe[w - 12];
+    }
+    double x = 0.0;
+#pragma unroll
+    for (int i = 0; i < kLin; ++i)
+#pragma unroll
+      for (int j = 0; j < kLin; ++j)
+        if (s_mul[i][j] == q) x = fma(u[i], v[j], x);
+    out[q] = x;
   }
   __syncthreads();
+  if (tid < kQuad) s_g[tid] = (s_ee[0][tid] + s_ee[3][tid]) + s_ee[5][tid];
+  __syncthreads();
+  if (tid < 240) {
+    const int o = tid >> 2, part = tid & 3, f = o / 6, k = o - f * 6;
+    const int i = k < 3 ? 0 : (k < 5 ? 1 : 2), j = k < 3 ? k : (k < 5 ? k - 2 : 2);
+    const int nf = f == 0 ? 1 : (f < 4 ? kLin : kQuad);
+    double x = 0.0;
+    for (int a = part; a < nf; a += 4) {
+      double y = mom(s_m, kM_D2 + k, a);
+#pragma unroll
+      for (int l = 0; l < kLin; ++l) {
+        const int q = s_mul[a][l];
+        y = fma(s_e[j][l], mom(s_m, kM_D1 + i, q), y);
+        y = fma(s_e[i][l], mom(s_m, kM_D1 + j, q), y);
+      }
+#pragma unroll
+      for (int l = 0; l < kQuad; ++l) y = fma(s_ee[k][l], mom(s_m, kM_n, s_mul[a][l]), y);
+      x = fma(s_f[f][a], y, x);
+    }
+    const double x1 = __shfl_xor(x, 1, 64);
+    x = (tid & 1) ? x1 + x : x + x1;
+    const double x2 = __shfl_xor(x, 2, 64);
+    x = (tid & 2) ? x2 + x : x + x2;
+    if (part == 0) s_V[o] = x;
+  } else if (tid >= 256 && tid < 304) {
+    const int o = (tid - 256) >> 2, part = tid & 3, f = o / 3, i = o - f * 3;
+    const int nf = f == 0 ? 1 : kLin;
+    double x = 0.0;
+    if (part < nf) {
+      // f's monomial `part`: a3, a2 e, and the quadratics of e times a1
+      double y = mom(s_m, kM_a3 + i, part);
+#pragma unroll
+      for (int l = 0; l < kLin; ++l) {
+        const int q = s_mul[part][l];
+        const double tr = (mom(s_m, kM_a2, q) + mom(s_m, kM_a2 + 3, q)) + mom(s_m, kM_a2 + 5, q);
+        y = fma(tr, s_e[i][l], y);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const int lo = min(i, k), hi = max(i, k), ik = lo == 0 ? hi : lo + hi + 1;
+          y = fma(2.0 * mom(s_m, kM_a2 + ik, q), s_e[k][l], y);
+        }
+      }
+#pragma unroll
+      for (int l = 0; l < kQuad; ++l) {
+        const int q = s_mul[part][l];
+        y = fma(s_g[l], mom(s_m, kM_a1 + i, q), y);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const int lo = min(i, k), hi = max(i, k), ik = lo == 0 ? hi : lo + hi + 1;
+          y = fma(2.0 * s_ee[ik][l], mom(s_m, kM_a1 + k, q), y);
+        }
+      }
+      x = s_f[f][part] * y;
+    }
+    // |e|^2 a0 (f e_i)
+    for (int a = part; a < kQuad; a += 4) {
+      double y = 0.0;
+#pragma unroll
+      for (int l = 0; l < kQuad; ++l) y = fma(s_g[l], mom(s_m, kM_a0, s_mul[a][l]), y);
+      x = fma(s_fe[o][a], y, x);
+    }
+    const double x1 = __shfl_xor(x, 1, 64);
+    x = (tid & 1) ? x1 + x : x + x1;
+    const double x2 = __shfl_xor(x, 2, 64);
+    x = (tid & 2) ? x2 + x : x + x2;
+    if (part == 0) s_F[o] = x;
+  } else if (tid >= 320) {
+    // c = sum a^2 |d|^4
+    const int l = tid - 320;
+    double x = 0.0;
+    for (int t = l; t < 1 + 12 + kQuad + 60 + 30 * kLin + 100; t += 64) {
+      int k = t;
+      if (k < 1) {
+        x += mom(s_m, kM_b4, 0);
+        continue;
+      }
+      k -= 1;
+      if (k < 12) {  // 4 e . b3
+        x = fma(4.0 * s_e[k >> 2][k & 3], mom(s_m, kM_b3 + (k >> 2), k & 3), x);
+        continue;
+      }
+      k -= 12;
+      if (k < kQuad) {  // 2 |e|^2 tr b2
+        const double tr = (mom(s_m, kM_b2, k) + mom(s_m, kM_b2 + 3, k)) + mom(s_m, kM_b2 + 5, k);
+        x = fma(2.0 * s_g[k], tr, x);
+        continue;
+      }
+      k -= kQuad;
+      if (k < 60) {  // 4 e^T b2 e
+        const int ik = k / kQuad, q = k - ik * kQuad;
+        const double w = ik == 0 || ik == 3 || ik == 5 ? 4.0 : 8.0;
+        x = fma(w * s_ee[ik][q], mom(s_m, kM_b2 + ik, q), x);
+        continue;
+      }
+      k -= 60;
+      if (k < 30 * kLin) {  // 4 |e|^2 e . b1
+        const int i = k / 40, a = (k - i * 40) >> 2, q = k & 3;
+        x = fma(4.0 * s_g[a] * s_e[i][q], mom(s_m, kM_b1 + i, s_mul[a][q]), x);
+        continue;
+      }
+      k -= 30 * kLin;
+      const int a = k / kQuad, q = k - a * kQuad;  // |e|^4 b0
+      x = fma(s_g[a] * s_g[q], mom(s_m, kM_b0, s_mul[a][q]), x);
+    }
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+    if (l == 0) s_c = x;
+  }
+  __syncthreads();
+  // S' and h' of u' = [d; s x d]; (s x d)_a = s_a1 d_a2 - s_a2 d_a1
   if (tid < 36) {
-    // full symmetric S from the packed upper triangle
-    const int i = tid / 6, j = tid % 6;
-    const int a = min(i, j), b = max(i, j);
-    const int k = a * 6 - a * (a - 1) / 2 + (b - a);
-    s_S[tid] = s_t[k];
+    const int i = tid / 6, j = tid - i * 6;
+    auto pk = [](int a, int b) { const int lo = min(a, b), hi = max(a, b); return lo == 0 ? hi : lo + hi + 1; };
+    auto V = [&](int f, int a, int b) { return s_V[f * 6 + pk(a, b)]; };
+    double x;
+    if (i < 3 && j < 3) {
+      x = V(0, i, j);
+    } else if (i >= 3 && j >= 3) {
+      const int a = i - 3, b = j - 3;
+      const int a1 = (a + 1) % 3, a2 = (a + 2) % 3, b1 = (b + 1) % 3, b2 = (b + 2) % 3;
+      x = (V(4 + pk(a1, b1), a2, b2) - V(4 + pk(a1, b2), a2, b1)) - (V(4 + pk(a2, b1), a1, b2) - V(4 + pk(a2, b2), a1, b1));
+    } else {
+      const int a = max(i, j) - 3, b = min(i, j), a1 = (a + 1) % 3, a2 = (a + 2) % 3;
+      x = V(1 + a1, a2, b) - V(1 + a2, a1, b);
+    }
+    s_S[tid] = x;
+  } else if (tid >= 64 && tid < 70) {
+    const int i = tid - 64;
+    if (i < 3) {
+      s_h[i] = s_F[i];
+    } else {
+      const int a = i - 3, a1 = (a + 1) % 3, a2 = (a + 2) % 3;
+      s_h[i] = s_F[(1 + a1) * 3 + a2] - s_F[(1 + a2) * 3 + a1];
+    }
+  } else if (tid >= 128 && tid < 200) {
+    // N = M diag(R2, R2)
+    const int which = (tid - 128) / 36, idx = (tid - 128) % 36, i = idx / 6, j = idx % 6;
+    const double* M = which ? s_M2 : s_M1;
+    const int b = j < 3 ? 0 : 3, c = j - b;
+    double v = 0.0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) v = fma(M[i * 6 + b + k], T2[k * 4 + c], v);
+    (which ? s_N2 : s_N1)[idx] = v;
   }
   __syncthreads();
   if (tid < 72) {
     const int which = tid / 36, idx = tid % 36, i = idx / 6, j = idx % 6;
-    const double* M = which ? s_M2 : s_M1;
+    const double* M = which ? s_N2 : s_N1;
     double v = 0.0;
     for (int k = 0; k < 6; ++k) v += M[i * 6 + k] * s_S[k * 6 + j];
     (which ? s_T2 : s_T1)[idx] = v;
@@ -385,18 +722,18 @@ __global__ __launch_bounds__(256) void ba_edge_reduce_kernel(const BaDev* __rest
   if (tid < 108) {
     const int blk = tid / 36, idx = tid % 36, i = idx / 6, j = idx % 6;
     const double* Tm = (blk == 2) ? s_T2 : s_T1;
-    const double* M = (blk == 0) ? s_M1 : s_M2;
+    const double* M = (blk == 0) ? s_N1 : s_N2;
     double v = 0.0;
     for (int k = 0; k < 6; ++k) v += Tm[i * 6 + k] * M[j * 6 + k];
     out[tid] = (blk == 1) ? -v : v;
   } else if (tid < 120) {
     const int which = (tid - 108) / 6, i = (tid - 108) % 6;
-    const double* M = which ? s_M2 : s_M1;
+    const double* M = which ? s_N2 : s_N1;
     double v = 0.0;
-    for (int k = 0; k < 6; ++k) v += M[i * 6 + k] * s_t[21 + k];
+    for (int k = 0; k < 6; ++k) v += M[i * 6 + k] * s_h[k];
     out[tid] = which ? -v : v;
   } else if (tid == 120) {
-    out[120] = s_t[27];
+    out[120] = s_c;
   }
 }
 
@@ -807,7 +1144,7 @@ static T* as(DevBuf& b) {
 
 enum {
   BA_PAIRS = 0, BA_COUNTS, BA_OVF, BA_STATE, BA_PROBS, BA_PART_A, BA_PART_OVF, BA_PART_CNT,
-  BA_DEV, BA_EDGES, BA_H, BA_HN, BA_PAIR_PART, BA_CONTRIB, BA_FLAG, BA_PAIR_IDS
+  BA_DEV, BA_EDGES, BA_H, BA_HN, BA_PAIR_PART, BA_CONTRIB, BA_MOMENTS, BA_PAIR_IDS
 };
 
 // Six buffers per frame: sorted source (pos, feat, sem, geo), grid store and
@@ -856,8 +1193,9 @@ struct BaLaunch {
   BaDev* ba;
   BaEdge* edges;
   AssocProblem* probs;
-  int n_edges, total_blocks, max_pair_blocks, lm_rounds, n_asm_blocks;
+  int n_edges, total_blocks, max_mom_blocks, lm_rounds, n_asm_blocks;
   double* part;
+  double* moments;
   double* contrib;
   double* H;  // two n x n halves: current linearisation and evaluation
   KConsts kc;
@@ -872,19 +1210,27 @@ static void ba_assoc_phase(const BaLaunch& L, hipStream_t s) {
   hipLaunchKernelGGL(ba_edges_kernel, dim3(1), dim3(256), 0, s, L.ba, L.edges, L.probs);
 }
 
+// e0 / e1 (optional): events at the moment kernel's own start and end.
+static void ba_moments_phase(const BaLaunch& L, hipStream_t s, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
+  const dim3 g(L.max_mom_blocks, L.n_edges), b(256);
+  if (e0) hipExtLaunchKernelGGL(ba_moments_kernel, g, b, 0, s, e0, e1, 0, L.ba, L.edges, L.probs, L.part, L.max_mom_blocks);
+  else hipLaunchKernelGGL(ba_moments_kernel, g, b, 0, s, L.ba, L.edges, L.probs, L.part, L.max_mom_blocks);
+  hipLaunchKernelGGL(ba_moments_sum_kernel, dim3(L.n_edges, kMomTiles), dim3(256), 0, s, L.ba, L.edges, L.part,
+                     L.max_mom_blocks, L.moments);
+}
+
 static void ba_lm_round(const BaLaunch& L, hipStream_t s) {
-  hipLaunchKernelGGL(ba_pair_kernel, dim3(L.max_pair_blocks, L.n_edges), dim3(kBaRowsPerBlock), 0, s, L.ba,
-                     L.edges, L.probs, L.part, L.max_pair_blocks);
-  hipLaunchKernelGGL(ba_edge_reduce_kernel, dim3(L.n_edges), dim3(256), 0, s, L.ba, L.edges, L.part,
-                     L.max_pair_blocks, L.contrib);
+  hipLaunchKernelGGL(ba_eval_kernel, dim3(L.n_edges), dim3(384), 0, s, L.ba, L.edges, L.moments, L.contrib);
   hipLaunchKernelGGL(ba_assemble_kernel, dim3(L.n_asm_blocks), dim3(64), 0, s, L.ba, L.edges, L.contrib, L.H);
   hipLaunchKernelGGL(ba_solve_kernel, dim3(1), dim3(kSolveThreads), 0, s, L.ba, L.H);
 }
 
 static void ba_iteration(const BaLaunch& L, hipStream_t s) {
   ba_assoc_phase(L, s);
-  if (L.n_edges > 0)
+  if (L.n_edges > 0) {
+    ba_moments_phase(L, s);
     for (int k = 0; k < L.lm_rounds; ++k) ba_lm_round(L, s);
+  }
   hipLaunchKernelGGL(ba_finish_kernel, dim3(1), dim3(64), 0, s, L.ba, L.edges);
 }
 
@@ -937,13 +1283,13 @@ extern "C" cvo_status cvo_align_multiframe(cvo_ctx* ctx, int32_t n_frames, const
   // per-edge association problems
   const int cap = p.multiframe_num_neighbors;
   size_t tot_rows = 0;
-  int total_blocks = 0, max_pair_blocks = 1;
+  int total_blocks = 0, max_mom_blocks = 1;
   std::vector<size_t> row_off(n_edges + 1, 0);
   for (int e = 0; e < n_edges; ++e) {
     const int n = frames[edges[2 * e]]->n;
     row_off[e + 1] = row_off[e] + (size_t)n;
     total_blocks += (n + rb - 1) / rb;
-    max_pair_blocks = std::max(max_pair_blocks, (n + kBaRowsPerBlock - 1) / kBaRowsPerBlock);
+    max_mom_blocks = std::max(max_mom_blocks, (n + kMomRows - 1) / kMomRows);
   }
   tot_rows = row_off[n_edges];
   const size_t E1 = (size_t)std::max(n_edges, 1);
@@ -959,8 +1305,9 @@ extern "C" cvo_status cvo_align_multiframe(cvo_ctx* ctx, int32_t n_frames, const
   CVO_TRY(ensure(ctx, B[BA_DEV], sizeof(BaDev)));
   CVO_TRY(ensure(ctx, B[BA_EDGES], sizeof(BaEdge) * E1));
   CVO_TRY(ensure(ctx, B[BA_H], sizeof(double) * 2 * kBaMaxDof * kBaMaxDof));
-  CVO_TRY(ensure(ctx, B[BA_PAIR_PART], sizeof(double) * kBaTerms * (size_t)max_pair_blocks * E1));
+  CVO_TRY(ensure(ctx, B[BA_PAIR_PART], sizeof(double) * kMomPart * (size_t)max_mom_blocks * E1));
   CVO_TRY(ensure(ctx, B[BA_CONTRIB], sizeof(double) * kBaContrib * E1));
+  CVO_TRY(ensure(ctx, B[BA_MOMENTS], sizeof(double) * kMomPart * E1));
   // the export needs each stored pair's target (its sorted position)
   if (per_edge) CVO_TRY(ensure(ctx, B[BA_PAIR_IDS], sizeof(uint32_t) * std::max<size_t>(tot_rows, 1) * cap));
   CVO_HIP(ctx, hipMemsetAsync(B[BA_OVF].p, 0, sizeof(uint32_t) * std::max<size_t>(tot_rows, 1), st));
@@ -1010,7 +1357,7 @@ extern "C" cvo_status cvo_align_multiframe(cvo_ctx* ctx, int32_t n_frames, const
     ed.f2 = f2;
     ed.K = cap;
     ed.n_rows = n;
-    ed.n_pair_blocks = (n + kBaRowsPerBlock - 1) / kBaRowsPerBlock;
+    ed.n_blocks = (n + kMomRows - 1) / kMomRows;
   }
   if (n_edges > 0) {
     CVO_HIP(ctx, hipMemcpyAsync(B[BA_PROBS].p, hp.data(), sizeof(AssocProblem) * n_edges, hipMemcpyHostToDevice, st));
@@ -1038,6 +1385,7 @@ extern "C" cvo_status cvo_align_multiframe(cvo_ctx* ctx, int32_t n_frames, const
     hb->free_idx[f] = (!hold_const || !hold_const[f]) ? o++ : -1;
     if (hb->free_idx[f] >= 0) hb->frame_of_free[hb->free_idx[f]] = f;
     hb->frame_norm[f] = frames[f]->max_norm;
+    for (int d = 0; d < 3; ++d) hb->centre[3 * f + d] = 0.5 * ((double)frames[f]->bmin[d] + (double)frames[f]->bmax[d]);
     for (int i = 0; i < 12; ++i) hb->X[12 * f + i] = poses[12 * f + i];
   }
   hb->done = p.multiframe_max_iters <= 0 ? 1 : 0;
@@ -1053,10 +1401,11 @@ extern "C" cvo_status cvo_align_multiframe(cvo_ctx* ctx, int32_t n_frames, const
   L.probs = as<AssocProblem>(B[BA_PROBS]);
   L.n_edges = n_edges;
   L.total_blocks = total_blocks;
-  L.max_pair_blocks = max_pair_blocks;
+  L.max_mom_blocks = max_mom_blocks;
   L.lm_rounds = std::max(0, p.multiframe_iterations_per_solve) + 1;
   L.n_asm_blocks = std::max(1, nfree * nfree + nfree);
   L.part = as<double>(B[BA_PAIR_PART]);
+  L.moments = as<double>(B[BA_MOMENTS]);
   L.contrib = as<double>(B[BA_CONTRIB]);
   L.H = as<double>(B[BA_H]);
   L.kc = kc;
@@ -1119,30 +1468,35 @@ extern "C" cvo_status cvo_align_multiframe(cvo_ctx* ctx, int32_t n_frames, const
         if (eh[e].on) pair_bytes += 16.0 * S + 20.0 * eh[e].n_rows;
       }
       float ms_pair = 0.0f, ms_solve = 0.0f;
-      int pair_launches = 0;
-      for (int k = 0; k < (n_edges > 0 ? L.lm_rounds : 0); ++k) {
-        int32_t pend[2] = {0, 0};
-        (void)hipMemcpyAsync(pend, &L.ba->eval_pending, sizeof(int32_t) * 2, hipMemcpyDeviceToHost, st);
+      int pair_launches = 0, solve_launches = 0;
+      auto pending = [&]() {
+        int32_t pend = 0;
+        (void)hipMemcpyAsync(&pend, &L.ba->eval_pending, sizeof(int32_t), hipMemcpyDeviceToHost, st);
         (void)hipStreamSynchronize(st);
-        const bool work = pend[0] != 0;
-        // the pair kernel timed alone
-        hipExtLaunchKernelGGL(ba_pair_kernel, dim3(L.max_pair_blocks, n_edges), dim3(kBaRowsPerBlock), 0, st, ev[4],
-                              ev[5], 0, L.ba, L.edges, L.probs, L.part, L.max_pair_blocks);
-        hipLaunchKernelGGL(ba_edge_reduce_kernel, dim3(n_edges), dim3(256), 0, st, L.ba, L.edges, L.part,
-                           L.max_pair_blocks, L.contrib);
-        hipLaunchKernelGGL(ba_assemble_kernel, dim3(L.n_asm_blocks), dim3(64), 0, st, L.ba, L.edges, L.contrib,
-                           L.H);
-        hipLaunchKernelGGL(ba_solve_kernel, dim3(1), dim3(kSolveThreads), 0, st, L.ba, L.H);
+        return pend != 0;
+      };
+      if (n_edges > 0) {
+        // the moment kernel timed alone
+        const bool work = pending();
+        ba_moments_phase(L, st, ev[4], ev[5]);
+        (void)hipStreamSynchronize(st);
+        if (work) {
+          (void)hipEventElapsedTime(&ms_pair, ev[4], ev[5]);
+          pair_launches = 1;
+          ctx->stats.bytes[CVO_KSTAT_BA_PAIR] += pair_bytes;
+        }
+      }
+      for (int k = 0; k < (n_edges > 0 ? L.lm_rounds : 0); ++k) {
+        const bool work = pending();
+        (void)hipEventRecord(ev[4], st);
+        ba_lm_round(L, st);
         (void)hipEventRecord(ev[3], st);
         (void)hipEventSynchronize(ev[3]);
-        float a = 0, b = 0;
-        (void)hipEventElapsedTime(&a, ev[4], ev[5]);
-        (void)hipEventElapsedTime(&b, ev[5], ev[3]);
+        float b = 0;
+        (void)hipEventElapsedTime(&b, ev[4], ev[3]);
         if (work) {
-          ms_pair += a;
           ms_solve += b;
-          pair_launches++;
-          ctx->stats.bytes[CVO_KSTAT_BA_PAIR] += pair_bytes;
+          solve_launches++;
         }
       }
       hipLaunchKernelGGL(ba_finish_kernel, dim3(1), dim3(64), 0, st, L.ba, L.edges);
@@ -1153,7 +1507,7 @@ extern "C" cvo_status cvo_align_multiframe(cvo_ctx* ctx, int32_t n_frames, const
       ctx->stats.ms[CVO_KSTAT_BA_PAIR] += ms_pair;
       ctx->stats.launches[CVO_KSTAT_BA_PAIR] += pair_launches;
       ctx->stats.ms[CVO_KSTAT_BA_SOLVE] += ms_solve;
-      ctx->stats.launches[CVO_KSTAT_BA_SOLVE] += pair_launches;
+      ctx->stats.launches[CVO_KSTAT_BA_SOLVE] += solve_launches;
       le = hipGetLastError();
     } else {
       ba_iteration(L, st);

@@ -158,3 +158,23 @@ def test_align_frames_updates_pose_vec_in_place(ba_gpu, oracle):
     P, it, _ = oracle.align_multiframe(p, clouds, inits, [1, 0, 0], [(0, 1), (1, 2), (0, 2)])
     for f, T in zip(frames, P):
         np.testing.assert_allclose(f.pose_vec.reshape(3, 4), T[:3, :4], rtol=0, atol=1e-8)
+
+
+@pytest.mark.parametrize("sizes,shift", [((1, 64, 700), 0.0), ((63, 65, 513), 0.0), ((511, 512, 1025), 0.0),
+                                         ((1500, 1300, 1700), 100.0)])
+def test_moments_match_oracle(ba_gpu, oracle, sizes, shift):
+    """The solve's polynomials in the poses where a frame is one row, a wave's
+    rows and one more, a moment block's rows and one more, and far from the
+    world's origin.  The oracle sums over the pairs at every candidate; both are
+    FP64, so 1e-9 as above, and 1e-8 at 100 m (the pair offsets, 0.1 m, lose
+    three digits more in its world coordinates)."""
+    p = params_from_yaml("ba_window.yaml")
+    p.multiframe_max_iters = 2
+    p.multiframe_min_nonzeros = 1
+    clouds, gts, inits = window(seed=11, n_frames=3, n_min=2000)
+    clouds = [c.subset(np.arange(n)) for c, n in zip(clouds, sizes)]
+    inits = inits.copy()
+    inits[:, :3, 3] += shift
+    g, P, it = run_both(ba_gpu, oracle, p, clouds, inits, [1, 0, 0], [(0, 1), (1, 2), (2, 0)])
+    assert g["iters"] == it
+    np.testing.assert_allclose(g["poses"][:, :3, :4], P[:, :3, :4], rtol=0, atol=1e-8 if shift else 1e-9)
