@@ -333,6 +333,8 @@ std::vector<float> level_sizes(const KConsts& kc, float ell_hi, float ell_lo, fl
   float r_hi = radius_for(kc, ell_hi, max_norm, tq);
   float r_lo = radius_for(kc, ell_lo, max_norm, tq) * cell_scale;
   if (!(r_hi > 0)) r_hi = 1.0f;
+  // one lengthscale: the one level its passes use
+  if (ell_hi == ell_lo) return {r_hi * cell_scale * 1.02f};
   float h = r_hi * 1.02f;
   for (int l = 0; l < kMaxLevels; ++l) {
     hs.push_back(h);
@@ -362,7 +364,23 @@ void apply_tuning(const cvo_tuning& t, KConsts& kc, bool batched) {
   kc.xcd_remap = t.xcd_remap;
 }
 
-void apply_tuning(const cvo_ctx* ctx, KConsts& kc, bool batched) { apply_tuning(ctx->tuning, kc, batched); }
+// Until a context is tuned, batched launches take 8 lanes a row and cells of half
+// the ball's radius: they fill the device whatever the lanes, so what counts is
+// the work, and clipped to the ball smaller cells and smaller groups enumerate
+// and mask less of it.  96 starts over 20k points, 300 iterations: 16 lanes
+// 729 / 601 / 590 ms at cell scale 1 / 0.7 / 0.5, 8 lanes 583 / 504 / 480, 4 lanes
+// (one-variant build) 625 / 517 / 489; the 12-frame window 42.3 / 39.2 / 38.7 and
+// 41.2 / 39.8 / 38.0.  A single registration takes cell scale 0.7: 60k street
+// 86.4 / 82.3 / 82.6 ms, K nearest at 20k 24.0 / 22.7 / 23.6, no difference below
+// 5k points; a single pass keeps 1 (its one grid is built for it alone).
+void apply_tuning(const cvo_ctx* ctx, KConsts& kc, bool batched) {
+  cvo_tuning t = ctx->tuning;
+  if (t.source == CVO_TUNE_DEFAULT) {
+    if (batched) t.lanes_per_row = t.lanes_small_ell = 8;
+    t.cell_scale = t.cell_scale_small_ell = batched ? 0.5f : (kc.mode == MODE_ALIGN ? 0.7f : 1.0f);
+  }
+  apply_tuning(t, kc, batched);
+}
 
 // Buffers and descriptors of n_probs problems sharing one source and target;
 // each problem owns the association blocks of its rows at max_group lanes per

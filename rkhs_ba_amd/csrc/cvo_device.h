@@ -44,6 +44,39 @@ __device__ __forceinline__ void st_global(float4* p, float4 v) {
   *(__attribute__((address_space(1))) v4f*)p = t;
 }
 
+// A value that is the same in all lanes, in a scalar register.
+__device__ __forceinline__ float uni(float v) {
+  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+template <class T>
+__device__ __forceinline__ const T* uni(const T* p) {
+  const uint64_t b = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
+  return reinterpret_cast<const T*>(((uint64_t)hi << 32) | lo);
+}
+
+// A grid level that is the same in all lanes.
+__device__ __forceinline__ GridLevel uniform_level(const GridLevel& s) {
+  GridLevel g;
+  g.h = uni(s.h);
+  g.inv_h = uni(s.inv_h);
+  g.ox = uni(s.ox);
+  g.oy = uni(s.oy);
+  g.oz = uni(s.oz);
+  g.nx = uni(s.nx);
+  g.ny = uni(s.ny);
+  g.nz = uni(s.nz);
+  g.cell_start = uni(s.cell_start);
+  g.pos = uni(s.pos);
+  g.feat = uni(s.feat);
+  g.sem = uni(s.sem);
+  g.geo = uni(s.geo);
+  g.inv_perm = uni(s.inv_perm);
+  return g;
+}
+
 // The value of lane (id ^ O), without an address register: data-parallel moves
 // inside a row of 16, the LDS crossbar's swizzle across rows of a half wave, the
 // half-wave swap for 32.  All lanes of the wave take part.

@@ -140,7 +140,24 @@ __device__ __forceinline__ void assoc_block(const AssocProblem& P, const KConsts
   const ExactK ek = exact_consts(kc);
   // a copy: the pair stores below cannot alias it, so its fields stay in
   // registers instead of being reloaded after every store
-  const GridLevel GL = P.grid->lv[st->level];
+  GridLevel GL = P.grid->lv[st->level];
+  if constexpr (!KNN && ROWS != kMaxRowsPerBlock) {
+    // batched launches have no vector registers to spare for what is the same
+    // in all lanes
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+      mp.A[i] = uni(mp.A[i]);
+      mp.Rq[i] = uni(mp.Rq[i]);
+      mp.As[i] = uni(mp.As[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      mp.b[i] = uni(mp.b[i]);
+      mp.Tq[i] = uni(mp.Tq[i]);
+      mp.bs[i] = uni(mp.bs[i]);
+    }
+    GL = uniform_level(GL);
+  }
   const int row0 = lb * RB;
   const int nrows = min(RB, P.n_src - row0);
   if (FC != 0) {
@@ -264,12 +281,13 @@ __device__ __forceinline__ void assoc_pass(const AssocProblem& P, const KConsts&
 
 // ONE: a single problem, its descriptor by value in the kernel arguments (read
 // with scalar loads, no dependent load before the first state read).
-// Occupancy: a single problem runs at five waves per SIMD (96 VGPRs, a
-// 16-byte spill; the 60k street registration 128.3 -> 125.0 ms, six waves
-// spill 96 bytes and take 157 ms); several problems at four (128 VGPRs: at
-// five the batched variant spills 64 bytes and the 96-start run slows 8%).
+// Occupancy: five waves per SIMD (96 VGPRs; six spill 96 bytes: the 60k street
+// registration 125 against 157 ms).  Batched launches need the maps and the grid
+// level in scalar registers for it (with them in vector registers five waves
+// spill 64 bytes and are slower than four): 96 starts over 20k points, 300
+// iterations, 8 lanes a row, 644 -> 583 ms.
 template <int FC, int KC, bool ONE>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(ONE ? 5 : 4))) void assoc_kernel(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void assoc_kernel(
     const AssocProblem* __restrict__ probs, int n_probs, KConsts kc, AssocProblem one) {
   if constexpr (ONE) {
     assoc_pass<FC, KC, false, true>(one, kc);

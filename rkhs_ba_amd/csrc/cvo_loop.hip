@@ -78,20 +78,7 @@ __host__ __device__ inline int loop_row_groups(int blocks, int xcd_remap) {
   return xcd_remap && blocks % 8 == 0 ? 8 : 1;
 }
 
-__device__ __forceinline__ float uni(float v) {
-  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
-}
-__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-template <class T>
-__device__ __forceinline__ const T* uni(const T* p) {
-  const uint64_t b = reinterpret_cast<uint64_t>(p);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
-  return reinterpret_cast<const T*>(((uint64_t)hi << 32) | lo);
-}
-
-// The state's maps and a grid level from LDS into scalar registers (the same
-// for the whole block).
+// The state's maps from LDS into scalar registers (the same for the whole block).
 // SRC: the rows may be moved by a source map (the self problem of the target).
 template <bool SRC>
 __device__ __forceinline__ void uniform_maps(const ProblemState& s, Maps& m) {
@@ -109,25 +96,6 @@ __device__ __forceinline__ void uniform_maps(const ProblemState& s, Maps& m) {
   }
   m.src_xf = SRC && uni(s.has_src_xf) != 0;
 }
-__device__ __forceinline__ GridLevel uniform_level(const GridLevel& s) {
-  GridLevel g;
-  g.h = uni(s.h);
-  g.inv_h = uni(s.inv_h);
-  g.ox = uni(s.ox);
-  g.oy = uni(s.oy);
-  g.oz = uni(s.oz);
-  g.nx = uni(s.nx);
-  g.ny = uni(s.ny);
-  g.nz = uni(s.nz);
-  g.cell_start = uni(s.cell_start);
-  g.pos = uni(s.pos);
-  g.feat = uni(s.feat);
-  g.sem = uni(s.sem);
-  g.geo = uni(s.geo);
-  g.inv_perm = uni(s.inv_perm);
-  return g;
-}
-
 __device__ __forceinline__ void put_word(uint64_t* p, uint32_t payload, uint32_t tag) {
   __hip_atomic_store(p, ((uint64_t)tag << 32) | payload, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
