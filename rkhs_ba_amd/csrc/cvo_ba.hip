@@ -68,7 +68,7 @@ constexpr int kMomTiles = 5;                   // 16 x 16 tiles of the moment ma
 constexpr int kMomPart = kMomTiles * 256;
 constexpr int kSolveThreads = 256;             // four waves: the Cholesky's trailing update spread over rows
 static_assert(kSolveThreads == 256 && 6 * kBaMaxFree <= kSolveThreads, "the solve's reductions assume four waves");
-constexpr int kChol = 8;                       // Cholesky block: columns a panel
+constexpr int kChol = 8;                       // Cholesky block: columns a panel (even, as the dof are)
 constexpr int kTri = 8;                        // triangular solves: steps a load batch
 
 struct BaEdge {
@@ -748,24 +748,15 @@ __device__ inline double wave_max(double v) {
   return v;
 }
 
-// Flat element e of the trailing lower triangle of an n x n factorisation,
-// ordered by column descending: column k = n - 1 - m holds entries
-// m (m + 1) / 2 ... m (m + 1) / 2 + m, rows k ... n - 1.  So the elements of
-// the columns right of j are exactly e < (n - j - 1)(n - j) / 2.
-__device__ inline void trailing_index(int e, int n, int& i, int& k) {
+// Flat element e < n (n + 1) / 2 of an n x n lower triangle, ordered by column
+// descending: column k = n - 1 - m holds entries m (m + 1) / 2 ...
+// m (m + 1) / 2 + m, rows k ... n - 1.
+__device__ inline void triangle_index(int e, int n, int& i, int& k) {
   int m = (int)((sqrtf(8.0f * (float)e + 1.0f) - 1.0f) * 0.5f);
   while ((m + 1) * (m + 2) / 2 <= e) ++m;
   while (m * (m + 1) / 2 > e) --m;
   k = n - 1 - m;
   i = k + (e - m * (m + 1) / 2);
-}
-
-// Orders one wave's LDS accesses across the point (other lanes' writes before
-// it are seen by reads after it); the compiler moves no LDS access over it.
-__device__ __forceinline__ void panel_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Lane l's value of v (l uniform), moved through scalar registers.
@@ -963,33 +954,51 @@ __global__ __launch_bounds__(kSolveThreads) void ba_solve_kernel(BaDev* __restri
     }
     __syncthreads();
     // blocked right-looking Cholesky, kChol columns a block: wave 0 factors
-    // the block's panel (rows below the block, its columns) alone -- a wave's
-    // LDS operations complete in order, so wave-scope fences order it --
-    // then all four waves subtract the block's columns from the trailing
-    // triangle, per element in the same order as column by column (the
-    // result is the unblocked one bit for bit); the diagonal's reciprocal
-    // goes to s_inv
+    // the block's panel (rows from the block on, its columns) in registers,
+    // rows j0 + lane and j0 + lane + 64 a lane, entries of the block's own rows
+    // by readlane; then all four waves subtract the block's columns from the
+    // trailing triangle in 2x2 tiles, per element in the same order as column
+    // by column (the result is the unblocked one bit for bit).  What is left
+    // above the diagonal is not read.  The diagonal's reciprocal goes to s_inv
     bool fail = false;
     for (int j0 = 0; j0 < n; j0 += kChol) {
       const int jb = min(kChol, n - j0);
       if (wave == 0) {
+        const int r0 = j0 + lane, r1 = r0 + 64;
+        double* R0 = s_A + min(r0, n - 1) * ld;
+        double* R1 = s_A + min(r1, n - 1) * ld;
+        double p0[kChol], p1[kChol];
+#pragma unroll
+        for (int c = 0; c < kChol; ++c) {
+          const int j = min(j0 + c, n - 1);
+          p0[c] = R0[j];
+          p1[c] = R1[j];
+        }
         int f = 0;
-        for (int c = 0; c < jb; ++c) {
-          const int j = j0 + c;
-          const double ajj = s_A[j * ld + j];
+#pragma unroll
+        for (int c = 0; c < kChol; ++c) {
+          if (c >= jb || f) break;  // uniform
+          const double ajj = readlane_f64(p0[c], c);
           if (!(ajj > 0.0)) {
             f = 1;
             break;
           }
           const double inv = 1.0 / sqrt(ajj);
-          for (int i = j + 1 + lane; i < n; i += 64) s_A[i * ld + j] *= inv;
-          if (lane == 0) s_inv[j] = inv;
-          panel_lds_sync();  // the scaled column, read across lanes below
-          for (int i = j + 1 + lane; i < n; i += 64) {
-            const double lij = s_A[i * ld + j];
-            for (int k = j + 1; k < j0 + jb && k <= i; ++k) s_A[i * ld + k] -= lij * s_A[k * ld + j];
+          if (lane == 0) s_inv[j0 + c] = inv;
+          if (lane > c) p0[c] *= inv;
+          p1[c] *= inv;
+#pragma unroll
+          for (int k = c + 1; k < kChol; ++k) {
+            const double lkj = readlane_f64(p0[c], k);
+            p0[k] -= p0[c] * lkj;
+            p1[k] -= p1[c] * lkj;
           }
-          panel_lds_sync();  // the next column's diagonal and entries
+        }
+#pragma unroll
+        for (int c = 0; c < kChol; ++c) {
+          if (c >= jb) break;
+          if (r0 < n) R0[j0 + c] = p0[c];
+          if (r1 < n) R1[j0 + c] = p1[c];
         }
         if (lane == 0) s_fail = f;
       }
@@ -998,25 +1007,33 @@ __global__ __launch_bounds__(kSolveThreads) void ba_solve_kernel(BaDev* __restri
         fail = true;
         break;
       }
-      // the trailing triangle {(i, k): j0 + jb <= k <= i < n} as M flat
-      // elements (the columns right of column j0 + jb - 1), four per thread
-      // a trip with all reads issued before the writes
-      const int rem = n - j0 - jb;
-      const int M = rem * (rem + 1) / 2;
-      for (int e0 = tid; e0 < M; e0 += 4 * kSolveThreads) {
-        int ii[4], kk[4];
-        double x[4];
+      // 2x2 tiles, those on and below the diagonal in flat order; n and the
+      // block are even, and where columns are left the block is a whole one.
+      // Single elements, four a thread with an index each, and the panel through
+      // LDS: 77 us a launch at 66 dof, so 50
+      const int base = j0 + jb, T = (n - base) / 2;
+      for (int e = tid; e < T * (T + 1) / 2; e += kSolveThreads) {
+        int i, k;
+        triangle_index(e, T, i, k);
+        i = base + 2 * i;
+        k = base + 2 * k;
+        double* Ai = s_A + i * ld;
+        double* Bi = Ai + ld;
+        const double* Ak = s_A + k * ld + j0;
+        const double* Bk = Ak + ld;
+        double x00 = Ai[k], x01 = Ai[k + 1], x10 = Bi[k], x11 = Bi[k + 1];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int e = min(e0 + u * kSolveThreads, M - 1);
-          trailing_index(e, n, ii[u], kk[u]);
-          double a = s_A[ii[u] * ld + kk[u]];
-          for (int c = 0; c < jb; ++c) a -= s_A[ii[u] * ld + j0 + c] * s_A[kk[u] * ld + j0 + c];
-          x[u] = a;
+        for (int c = 0; c < kChol; ++c) {
+          const double a0 = Ai[j0 + c], a1 = Bi[j0 + c], b0 = Ak[c], b1 = Bk[c];
+          x00 -= a0 * b0;
+          x01 -= a0 * b1;
+          x10 -= a1 * b0;
+          x11 -= a1 * b1;
         }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          if (e0 + u * kSolveThreads < M) s_A[ii[u] * ld + kk[u]] = x[u];
+        Ai[k] = x00;
+        Ai[k + 1] = x01;
+        Bi[k] = x10;
+        Bi[k + 1] = x11;
       }
       __syncthreads();
     }

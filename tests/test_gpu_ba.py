@@ -178,3 +178,19 @@ def test_moments_match_oracle(ba_gpu, oracle, sizes, shift):
     g, P, it = run_both(ba_gpu, oracle, p, clouds, inits, [1, 0, 0], [(0, 1), (1, 2), (2, 0)])
     assert g["iters"] == it
     np.testing.assert_allclose(g["poses"][:, :3, :4], P[:, :3, :4], rtol=0, atol=1e-8 if shift else 1e-9)
+
+
+@pytest.mark.parametrize("free", [1, 2, 10, 11, 20])
+def test_solve_sizes_match_oracle(ba_gpu, oracle, free):
+    """The normal equations of 6 dof (less than a factorisation block) to 120
+    (the most; two rows a lane, 74 edges: more than a wave lists at once).  Two
+    outer iterations as above: 1e-9."""
+    p = params_from_yaml("ba_window.yaml")
+    p.multiframe_max_iters = 2
+    p.multiframe_min_nonzeros = 1
+    n = free + 1
+    clouds, gts, inits = window(seed=5, n_frames=n, n_min=600, n_max=700)
+    edges = [(i, j) for i in range(n) for j in range(i + 1, min(n, i + 5))]
+    g, P, it = run_both(ba_gpu, oracle, p, clouds, inits, [1] + [0] * free, edges)
+    assert g["iters"] == it
+    np.testing.assert_allclose(g["poses"][:, :3, :4], P[:, :3, :4], rtol=0, atol=1e-9)
