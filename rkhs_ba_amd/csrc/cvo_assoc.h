@@ -238,7 +238,6 @@ __device__ __forceinline__ RowConsts row_consts(const KConsts& kc, bool own_ell,
 struct RowResult {
   double acc[7];  // omega(3), v(3), ip
   uint32_t stored;
-  uint32_t seen;  // candidates enumerated
   bool overflow;
 };
 
@@ -254,7 +253,6 @@ __device__ __forceinline__ void assoc_row(const AssocProblem& P, const KConsts& 
 #pragma unroll
   for (int c = 0; c < 7; ++c) out.acc[c] = 0.0;
   out.stored = 0;
-  out.seen = 0;
   out.overflow = false;
   const uint32_t Ku = (uint32_t)K;
   if (!kc.use_geo) {
@@ -345,7 +343,6 @@ __device__ __forceinline__ void assoc_row(const AssocProblem& P, const KConsts& 
     }
     const uint32_t total = __shfl(incl, G - 1, G);
     const uint32_t excl = incl - rl;
-    out.seen += total;
     for (uint32_t base = 0; base < total; base += G) {
       const uint32_t idx = base + (uint32_t)g;
       // the run holding candidate idx: the last run whose prefix is <= idx
@@ -432,7 +429,6 @@ __device__ __forceinline__ void knn_row(const AssocProblem& P, const KConsts& kc
 #pragma unroll
   for (int c = 0; c < 7; ++c) out.acc[c] = 0.0;
   out.stored = 0;
-  out.seen = 0;
   out.overflow = false;
   const uint32_t Ku = (uint32_t)max(K, 0);
   if (Ku == 0) return;

@@ -13,7 +13,7 @@
 //                                   block runs the device controller
 //                                   (:464-544, :1289-1433)
 //
-// Rows are processed by groups of G = 8 or 16 lanes (256 / G rows per
+// Rows are processed by groups of G = 4, 8 or 16 lanes (256 / G rows per
 // 256-thread block), G chosen per iteration from the lengthscale.  Reductions
 // are block partials summed in fixed order, so results are bitwise
 // reproducible run to run.

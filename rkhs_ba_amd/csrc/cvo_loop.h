@@ -10,7 +10,7 @@
 namespace cvo {
 
 constexpr int kMaxLoopDevices = 64;
-constexpr size_t kLoopMaxLds = 128 * 1024;  // dynamic LDS of a block, beside its static 12 KB
+constexpr size_t kLoopMaxLds = 128 * 1024;  // dynamic LDS of a block, beside up to 8 KB of static LDS
 
 // Arguments of a launch, in device memory.
 struct LoopArgs {

@@ -59,14 +59,13 @@ constexpr int kChunk = 8;
 
 // Words a block publishes after the association: the registration's six flow
 // sums and, with self problems, every problem's ip sum, two words a double; then
-// the stored pairs of each problem, the registration's longest row and its
-// candidates.
+// the stored pairs of each problem and the registration's longest row.
 template <int NP>
 struct AssocWords {
   static constexpr int kDoubles = NP == 1 ? 6 : 6 + NP;
-  static constexpr int kCounts = NP + 2;
-  static constexpr int kCount0 = 2 * kDoubles, kMaxRow = kCount0 + NP, kSeen = kMaxRow + 1;
-  static constexpr int kUsed = kSeen + 1;
+  static constexpr int kCounts = NP + 1;
+  static constexpr int kCount0 = 2 * kDoubles, kMaxRow = kCount0 + NP;
+  static constexpr int kUsed = kMaxRow + 1;
   static constexpr int kStride = NP == 1 ? 16 : 32;
   static_assert(kUsed <= kStride, "the words exceed their line");
 };
@@ -238,7 +237,7 @@ struct LoopShared {
   int n_levels[NP];
   double red[kLoopWaves][9];
   double capped[kLoopWaves][7];  // a wave's sums over its capped rows
-  uint32_t counts[NP + 2];       // stored pairs per problem, longest row, candidates
+  uint32_t counts[NP + 1];       // stored pairs per problem, longest row
   float dir[6];                  // the flow's direction, for the step terms
   double xi[6], norm;            // the normalised flow and the flow's norm
   uint64_t nnz;                  // totals of the association
@@ -254,7 +253,7 @@ using SharedPtr = __attribute__((address_space(3))) LoopShared<NP>*;
 // The waves' partial sums of an association to LDS.
 template <int NP>
 __device__ __forceinline__ void block_partials(LoopShared<NP>& S, const double (&sums)[AssocWords<NP>::kDoubles],
-                                               const uint32_t (&nz)[NP], uint32_t mx, uint32_t seen) {
+                                               const uint32_t (&nz)[NP], uint32_t mx) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if constexpr (NP == 1) {
     const double x = wave_sums(sums);
@@ -277,7 +276,6 @@ __device__ __forceinline__ void block_partials(LoopShared<NP>& S, const double (
   for (int q = 0; q < NP; ++q)
     if (nz[q]) atomicAdd(&S.counts[q], nz[q]);
   if (mx) atomicMax(&S.counts[NP], mx);
-  if (seen) atomicAdd(&S.counts[NP + 1], seen);
 }
 
 // A block's rows in LDS.
@@ -292,13 +290,12 @@ struct RowLds {
 };
 
 // Association of the block's rows [lo, hi) (local indices) of one problem, G
-// lanes a row.  Adds to acc, the stored pairs to nz, the longest row to mx, the
-// candidates to seen; a row over its cap is marked instead.
+// lanes a row.  Adds to acc, the stored pairs to nz, the longest row to mx;
+// a row over its cap is marked instead.
 template <int FC, int KC, bool KNN, int G>
 __device__ __forceinline__ void loop_rows(const AssocProblem& P, const KConsts& kc, const GridLevel& GL,
                                           const Maps& mp, int mode, float ell, int K, int lo, int hi, const RowLds& R,
-                                          int* any_capped, double acc[7], uint32_t& nz, uint32_t& mx,
-                                          uint32_t& seen) {
+                                          int* any_capped, double acc[7], uint32_t& nz, uint32_t& mx) {
   const int tid = threadIdx.x, g = tid & (G - 1), grp = tid / G;
   const int F = Dim<FC>::get(kc.F), KS = Dim<KC>::get(kc.Ks);
   const ExactK ek = exact_consts(kc);
@@ -320,7 +317,6 @@ __device__ __forceinline__ void loop_rows(const AssocProblem& P, const KConsts& 
     }
     if (g == 0) {
       R.cnt[i] = res.overflow ? kCapped : res.stored;
-      seen += res.seen;
       if (res.overflow) *any_capped = 1;
       else {
         nz += res.stored;
@@ -708,7 +704,7 @@ __global__ __launch_bounds__(kLoopThreads) void loop_kernel(const LoopArgs* args
     double sums[W::kDoubles];
 #pragma unroll
     for (int c = 0; c < W::kDoubles; ++c) sums[c] = 0.0;
-    uint32_t nz[NP], mx = 0, seen = 0;
+    uint32_t nz[NP], mx = 0;
 #pragma unroll
     for (int q = 0; q < NP; ++q) {
       nz[q] = 0;
@@ -723,11 +719,10 @@ __global__ __launch_bounds__(kLoopThreads) void loop_kernel(const LoopArgs* args
       const int K = uni(st.K);
       const int mode = q == 0 ? MODE_ALIGN : MODE_IP;
       double acc[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-      uint32_t mxq = 0, seenq = 0;
+      uint32_t mxq = 0;
       const int n = seg[q + 1] - seg[q];
 #define CVO_LOOP_ROWS(G)                                                                                         \
-  loop_rows<FC, KC, KNN, G>(P, kc, GL, mp, mode, ell0, K, seg[q], seg[q + 1], R, &S.any_capped, acc, nz[q], mxq, \
-                            seenq)
+  loop_rows<FC, KC, KNN, G>(P, kc, GL, mp, mode, ell0, K, seg[q], seg[q + 1], R, &S.any_capped, acc, nz[q], mxq)
       // as many lanes a row as one round of the block's threads holds
       if constexpr (KNN) {
         if (uni(state_group(&st)) == 8) CVO_LOOP_ROWS(8);
@@ -741,13 +736,12 @@ __global__ __launch_bounds__(kLoopThreads) void loop_kernel(const LoopArgs* args
 #undef CVO_LOOP_ROWS
       if (q == 0) {
         mx = mxq;
-        seen = seenq;
 #pragma unroll
         for (int c = 0; c < 6; ++c) sums[c] = acc[c];
       }
       if constexpr (NP > 1) sums[6 + q] = acc[6];
     }
-    block_partials<NP>(S, sums, nz, mx, seen);
+    block_partials<NP>(S, sums, nz, mx);
     __syncthreads();
     if constexpr (!KNN) {
       if (S.any_capped) {  // uniform
