@@ -39,6 +39,11 @@ void launch_math_check(int n_cubic, const double* coef, double* re, double* im, 
 void launch_gather(const uint32_t* order, int n, const float* xyz, const float* feat, int F, const float* sem, int K,
                    const float* geo, float4* pos, float* feat_s, float* sem_s, float* geo_s, uint32_t* inv_perm,
                    hipStream_t s);
+void launch_small_source(const float* xyz, int n, const float* bmin, const float* bmax, const float* feat, int F,
+                         const float* sem, int K, const float* geo, float4* pos, float* feat_s, float* sem_s,
+                         float* geo_s, hipStream_t s);
+void launch_small_levels(const float* xyz, int n, const GridDev& G, uint32_t max_cells, const float* feat, int F,
+                         const float* sem, int K, const float* geo, hipStream_t s);
 void launch_morton(const float* xyz, int n, const float* bmin, const float* bmax, uint32_t* key, hipStream_t s);
 void launch_export(const AssocProblem* P_dev, int n_src, int64_t* counts_orig, const int64_t* row_ptr, int32_t* col,
                    float* val, int phase, int sort_threshold, hipStream_t s);
@@ -192,23 +197,17 @@ float radius_for(const KConsts& kc, float ell, float max_norm, float tq) {
   return kc.rq_coef * ell * (1.0f + max_norm / 500.0f) * 1.0001f + 1e-4f * (1.0f + max_norm + tq) + 1e-6f;
 }
 
+// Clouds up to this size are sorted a block in LDS (64 KB of words), all levels of
+// a grid at once: the most that needs no larger LDS allowance, and the one block's
+// sort grows as n log^2 n (about 40 us here) where a level of the general path
+// takes about as long in launches whatever its size.
+constexpr int kSmallCloud = 8192;
+
 // Spatially sorted source rows (Morton order over the source bounding box).
 cvo_status prepare_source_into(cvo_ctx* ctx, const cvo_dcloud* s, DevBuf& b_pos, DevBuf& b_feat, DevBuf& b_sem,
                                DevBuf& b_geo) {
   hipStream_t st = ctx->stream;
   const int n = s->n;
-  CVO_TRY(ensure(ctx, ctx->b_src_key, sizeof(uint32_t) * n * 2));
-  CVO_TRY(ensure(ctx, ctx->b_src_perm, sizeof(uint32_t) * n * 2));
-  uint32_t* keys = as<uint32_t>(ctx->b_src_key);
-  uint32_t* keys2 = keys + n;
-  uint32_t* idx = as<uint32_t>(ctx->b_src_perm);
-  uint32_t* idx2 = idx + n;
-  launch_morton(s->xyz, n, s->bmin, s->bmax, keys, st);
-  launch_iota(idx, n, st);
-  size_t tmp = 0;
-  CVO_HIP(ctx, hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, keys, keys2, idx, idx2, n, 0, 30, st));
-  CVO_TRY(ensure(ctx, ctx->b_cub, tmp));
-  CVO_HIP(ctx, hipcub::DeviceRadixSort::SortPairs(ctx->b_cub.p, tmp, keys, keys2, idx, idx2, n, 0, 30, st));
   CVO_TRY(ensure(ctx, b_pos, sizeof(float4) * n));
   float* fs = nullptr;
   float* ss = nullptr;
@@ -225,6 +224,24 @@ cvo_status prepare_source_into(cvo_ctx* ctx, const cvo_dcloud* s, DevBuf& b_pos,
     CVO_TRY(ensure(ctx, b_geo, sizeof(float) * (size_t)n * 2));
     gs = as<float>(b_geo);
   }
+  if (n <= kSmallCloud) {
+    launch_small_source(s->xyz, n, s->bmin, s->bmax, s->feat, s->F, s->sem, s->K, s->geo, as<float4>(b_pos), fs, ss,
+                        gs, st);
+    CVO_HIP(ctx, hipGetLastError());
+    return CVO_OK;
+  }
+  CVO_TRY(ensure(ctx, ctx->b_src_key, sizeof(uint32_t) * n * 2));
+  CVO_TRY(ensure(ctx, ctx->b_src_perm, sizeof(uint32_t) * n * 2));
+  uint32_t* keys = as<uint32_t>(ctx->b_src_key);
+  uint32_t* keys2 = keys + n;
+  uint32_t* idx = as<uint32_t>(ctx->b_src_perm);
+  uint32_t* idx2 = idx + n;
+  launch_morton(s->xyz, n, s->bmin, s->bmax, keys, st);
+  launch_iota(idx, n, st);
+  size_t tmp = 0;
+  CVO_HIP(ctx, hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, keys, keys2, idx, idx2, n, 0, 30, st));
+  CVO_TRY(ensure(ctx, ctx->b_cub, tmp));
+  CVO_HIP(ctx, hipcub::DeviceRadixSort::SortPairs(ctx->b_cub.p, tmp, keys, keys2, idx, idx2, n, 0, 30, st));
   launch_gather(idx2, n, s->xyz, s->feat, s->F, s->sem, s->K, s->geo, as<float4>(b_pos), fs, ss, gs, nullptr,
                 st);
   CVO_HIP(ctx, hipGetLastError());
@@ -278,39 +295,46 @@ cvo_status build_grid_into(cvo_ctx* ctx, const cvo_dcloud* t, const std::vector<
   }
   CVO_TRY(ensure(ctx, b_store, total));
   char* base = as<char>(b_store);
-  // temporaries: keys, keys2, idx, idx2, counts
-  CVO_TRY(ensure(ctx, ctx->b_tmp0, sizeof(uint32_t) * (size_t)n * 4));
-  CVO_TRY(ensure(ctx, ctx->b_tmp1, sizeof(uint32_t) * ((size_t)max_cells + 1)));
-  uint32_t* keys = as<uint32_t>(ctx->b_tmp0);
-  uint32_t* keys2 = keys + n;
-  uint32_t* idx = keys2 + n;
-  uint32_t* idx2 = idx + n;
-  uint32_t* counts = as<uint32_t>(ctx->b_tmp1);
   for (int l = 0; l < L; ++l) {
     GridLevel& lv = G.lv[l];
-    uint32_t nc = (uint32_t)lv.nx * (uint32_t)lv.ny * (uint32_t)lv.nz;
-    uint32_t* cell_start = reinterpret_cast<uint32_t*>(base + off_cells[l]);
-    launch_zero(counts, sizeof(uint32_t) * (nc + 1), st);
-    launch_grid_count(t->xyz, n, lv, keys, counts, st);
-    size_t tmp = 0;
-    CVO_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, counts, cell_start, (int)nc + 1, st));
-    size_t tmp2 = 0;
-    int bits = 1;
-    while ((1u << bits) < nc && bits < 32) ++bits;
-    CVO_HIP(ctx, hipcub::DeviceRadixSort::SortPairs(nullptr, tmp2, keys, keys2, idx, idx2, n, 0, bits, st));
-    CVO_TRY(ensure(ctx, ctx->b_cub, std::max(tmp, tmp2)));
-    CVO_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(ctx->b_cub.p, tmp, counts, cell_start, (int)nc + 1, st));
-    launch_iota(idx, n, st);
-    CVO_HIP(ctx, hipcub::DeviceRadixSort::SortPairs(ctx->b_cub.p, tmp2, keys, keys2, idx, idx2, n, 0, bits, st));
-    lv.cell_start = cell_start;
+    lv.cell_start = reinterpret_cast<const uint32_t*>(base + off_cells[l]);
     lv.pos = reinterpret_cast<const float4*>(base + off_pos[l]);
     lv.feat = t->feat ? reinterpret_cast<const float*>(base + off_feat[l]) : nullptr;
     lv.sem = t->sem ? reinterpret_cast<const float*>(base + off_sem[l]) : nullptr;
     lv.geo = t->geo ? reinterpret_cast<const float*>(base + off_geo[l]) : nullptr;
     lv.inv_perm = reinterpret_cast<const uint32_t*>(base + off_inv[l]);
-    launch_gather(idx2, n, t->xyz, t->feat, t->F, t->sem, t->K, t->geo, const_cast<float4*>(lv.pos),
-                  const_cast<float*>(lv.feat), const_cast<float*>(lv.sem), const_cast<float*>(lv.geo),
-                  const_cast<uint32_t*>(lv.inv_perm), st);
+  }
+  if (n <= kSmallCloud) {
+    launch_small_levels(t->xyz, n, G, max_cells, t->feat, t->F, t->sem, t->K, t->geo, st);
+  } else {
+    // temporaries: keys, keys2, idx, idx2, counts
+    CVO_TRY(ensure(ctx, ctx->b_tmp0, sizeof(uint32_t) * (size_t)n * 4));
+    CVO_TRY(ensure(ctx, ctx->b_tmp1, sizeof(uint32_t) * ((size_t)max_cells + 1)));
+    uint32_t* keys = as<uint32_t>(ctx->b_tmp0);
+    uint32_t* keys2 = keys + n;
+    uint32_t* idx = keys2 + n;
+    uint32_t* idx2 = idx + n;
+    uint32_t* counts = as<uint32_t>(ctx->b_tmp1);
+    for (int l = 0; l < L; ++l) {
+      GridLevel& lv = G.lv[l];
+      uint32_t nc = (uint32_t)lv.nx * (uint32_t)lv.ny * (uint32_t)lv.nz;
+      uint32_t* cell_start = const_cast<uint32_t*>(lv.cell_start);
+      launch_zero(counts, sizeof(uint32_t) * (nc + 1), st);
+      launch_grid_count(t->xyz, n, lv, keys, counts, st);
+      size_t tmp = 0;
+      CVO_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, counts, cell_start, (int)nc + 1, st));
+      size_t tmp2 = 0;
+      int bits = 1;
+      while ((1u << bits) < nc && bits < 32) ++bits;
+      CVO_HIP(ctx, hipcub::DeviceRadixSort::SortPairs(nullptr, tmp2, keys, keys2, idx, idx2, n, 0, bits, st));
+      CVO_TRY(ensure(ctx, ctx->b_cub, std::max(tmp, tmp2)));
+      CVO_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(ctx->b_cub.p, tmp, counts, cell_start, (int)nc + 1, st));
+      launch_iota(idx, n, st);
+      CVO_HIP(ctx, hipcub::DeviceRadixSort::SortPairs(ctx->b_cub.p, tmp2, keys, keys2, idx, idx2, n, 0, bits, st));
+      launch_gather(idx2, n, t->xyz, t->feat, t->F, t->sem, t->K, t->geo, const_cast<float4*>(lv.pos),
+                    const_cast<float*>(lv.feat), const_cast<float*>(lv.sem), const_cast<float*>(lv.geo),
+                    const_cast<uint32_t*>(lv.inv_perm), st);
+    }
   }
   CVO_HIP(ctx, hipGetLastError());
   CVO_TRY(ensure(ctx, b_hdr, sizeof(GridDev)));
