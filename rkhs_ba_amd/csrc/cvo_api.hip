@@ -197,11 +197,17 @@ float radius_for(const KConsts& kc, float ell, float max_norm, float tq) {
   return kc.rq_coef * ell * (1.0f + max_norm / 500.0f) * 1.0001f + 1e-4f * (1.0f + max_norm + tq) + 1e-6f;
 }
 
-// Clouds up to this size are sorted a block in LDS (64 KB of words), all levels of
-// a grid at once: the most that needs no larger LDS allowance, and the one block's
-// sort grows as n log^2 n (about 40 us here) where a level of the general path
-// takes about as long in launches whatever its size.
-constexpr int kSmallCloud = 8192;
+// A cloud may be sorted by one block in LDS, all levels of a grid at once, or level
+// by level over the device.  The block's sort grows in steps of the padded size
+// whatever the levels, the device's takes about 27 us of launches a level
+// whatever the size.  An inner product (the source's order and one level),
+// device passes / block sort: 108 / 111 us at 1000 points, 128 / 125 at 2000, 132 /
+// 158 at 3000, 152 / 229 at 5000, 158 / 246 at 8192; the set-up of a registration
+// with ten levels 404 / 176, 422 / 213, 503 / 285 and 518 / 308 at the last four.  So
+// one level (or a source order) takes the block up to 2048 points, and three
+// levels repay the dearest sort, 44 us above a device pass; 8192 words are the
+// 64 KB that need no larger LDS allowance.
+static bool sorts_in_a_block(int n, int levels) { return n <= (levels >= 3 ? 8192 : 2048); }
 
 // Spatially sorted source rows (Morton order over the source bounding box).
 cvo_status prepare_source_into(cvo_ctx* ctx, const cvo_dcloud* s, DevBuf& b_pos, DevBuf& b_feat, DevBuf& b_sem,
@@ -224,7 +230,7 @@ cvo_status prepare_source_into(cvo_ctx* ctx, const cvo_dcloud* s, DevBuf& b_pos,
     CVO_TRY(ensure(ctx, b_geo, sizeof(float) * (size_t)n * 2));
     gs = as<float>(b_geo);
   }
-  if (n <= kSmallCloud) {
+  if (sorts_in_a_block(n, 1)) {
     launch_small_source(s->xyz, n, s->bmin, s->bmax, s->feat, s->F, s->sem, s->K, s->geo, as<float4>(b_pos), fs, ss,
                         gs, st);
     CVO_HIP(ctx, hipGetLastError());
@@ -304,7 +310,7 @@ cvo_status build_grid_into(cvo_ctx* ctx, const cvo_dcloud* t, const std::vector<
     lv.geo = t->geo ? reinterpret_cast<const float*>(base + off_geo[l]) : nullptr;
     lv.inv_perm = reinterpret_cast<const uint32_t*>(base + off_inv[l]);
   }
-  if (n <= kSmallCloud) {
+  if (sorts_in_a_block(n, L)) {
     launch_small_levels(t->xyz, n, G, max_cells, t->feat, t->F, t->sem, t->K, t->geo, st);
   } else {
     // temporaries: keys, keys2, idx, idx2, counts

@@ -1,7 +1,7 @@
-"""Small clouds are sorted by one block in LDS, larger ones by the general
-passes: the same cloud padded past the limit with points out of every kernel's
-reach takes the general path and must give the same association, pairs and
-values bit for bit."""
+"""Small clouds are sorted by one block in LDS (up to 2048 points at one grid
+level, up to 8192 at three or more), larger ones by the general passes: the same
+cloud padded past the limit with points out of every kernel's reach takes the
+general path and must give the same association, pairs and values bit for bit."""
 import numpy as np
 import pytest
 
@@ -41,3 +41,29 @@ def test_small_path_equals_general(cvo_gpu, n, crowded):
     np.testing.assert_array_equal(a.col, b.col)
     np.testing.assert_array_equal(a.val, b.val)
     assert n < 255 or len(a.col) > 0
+
+
+@pytest.mark.parametrize("n", [2047, 2048, 2049, 4097, 8192, 8193])
+@pytest.mark.parametrize("ell", [0.5, 0.22, 0.05])
+def test_levels_of_a_registration_equal_general(cvo_gpu, n, ell):
+    """A registration's grid has a level for every lengthscale between ell_min and
+    ell_init: its first association, at the coarsest, a middle and the finest."""
+    p = params_from_yaml("planes_spheres_5k.yaml")
+    p.ell_init, p.ell_min = ell, (0.5 if ell < 0.5 else 0.05)
+    p.MAX_ITER, p.is_exporting_association = 1, 1
+    cvo_gpu.write_params(p)
+    src, tgt, T = synth.planes_spheres_pair(4, n, n)
+
+    def padded(c, far):
+        pad = LIMIT + 2 - c.n
+        xyz = np.concatenate([c.xyz, np.repeat(c.xyz[:1] + np.float32(far), pad, 0)])
+        return synth.Cloud(xyz, np.concatenate([c.feat, np.repeat(c.feat[:1], pad, 0)]))
+
+    print(f"levels n={n} ell={ell}", flush=True)
+    a = cvo_gpu.align(src, tgt, T, association=True)[4]
+    b = cvo_gpu.align(padded(src, 100.0), padded(tgt, -100.0), T, association=True)[4]
+    np.testing.assert_array_equal(a.row_ptr, b.row_ptr[: n + 1])
+    assert b.row_ptr[-1] == b.row_ptr[n]
+    np.testing.assert_array_equal(a.col, b.col)
+    np.testing.assert_array_equal(a.val, b.val)
+    assert len(a.col) > 0
