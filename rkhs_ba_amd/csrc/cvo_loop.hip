@@ -41,6 +41,7 @@
 
 #include "cvo_assoc.h"
 #include "cvo_controller.h"
+#include "cvo_exchange.h"
 #include "cvo_loop.h"
 
 namespace cvo {
@@ -99,45 +100,37 @@ __device__ __forceinline__ void put_word(uint64_t* p, uint32_t payload, uint32_t
   __hip_atomic_store(p, ((uint64_t)tag << 32) | payload, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// The wave that reads an exchange's words (read_words).
+template <int PER>
+struct ExchangeWave {
+  static constexpr int kWords = PER;
+  uint64_t v[PER];
+  template <class F>
+  __device__ __forceinline__ void each(F f) {
+    f((int)(threadIdx.x & 63), v);
+  }
+  template <class F>
+  __device__ __forceinline__ bool every(F f) {
+    return __all(f((int)(threadIdx.x & 63), v)) != 0;
+  }
+};
+
 // One wave reads the n lines of NW words at base until every tag matches and
 // returns the sum over the lines of this lane's word (lane & (NW - 1)): a
 // double's two words both return the double's sum, a count's word its sum, the
-// word max_word its maximum.  ok is cleared when the wait runs out.
+// word max_word its maximum.  ok is cleared, in all lanes, when the wait runs out.
 template <int NW, int USED, int DOUBLE_WORDS, int LINES>
 __device__ __forceinline__ double read_lines(uint64_t* base, int n_lines, uint32_t tag, uint64_t wait_ticks,
                                              int max_word, bool& ok) {
   constexpr int PER = (LINES * NW + 63) / 64;
   const int lane = threadIdx.x & 63, w = lane & (NW - 1);
-  const int n = w < USED ? n_lines * NW : 0;
-  uint64_t v[PER];
-#pragma unroll
-  for (int u = 0; u < PER; ++u) {
-    const int i = lane + u * 64;
-    v[u] = (uint64_t)tag << 32;
-    if (i < n) v[u] = __hip_atomic_load(base + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  uint64_t t0 = 0;
-  for (uint32_t tries = 0;; ++tries) {
-    bool all = true;
-#pragma unroll
-    for (int u = 0; u < PER; ++u) all = all && (uint32_t)(v[u] >> 32) == tag;
-    if (all) break;
-    // only the words still missing
-#pragma unroll
-    for (int u = 0; u < PER; ++u)
-      if ((uint32_t)(v[u] >> 32) != tag)
-        v[u] = __hip_atomic_load(base + lane + u * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // the clock's own read costs as much as a poll: every 64th (a wait of 0 ends
-    // at the first missing word)
-    if ((tries & 63) == 63 || wait_ticks == 0) {
-      const uint64_t now = wall_clock64();
-      if (t0 == 0) t0 = now;
-      if (now - t0 >= wait_ticks) {
-        ok = false;
-        break;
-      }
-    }
-  }
+  ExchangeWave<PER> wave;
+  ok = read_words<NW, USED>(
+           wave, n_lines, tag, wait_ticks,
+           [&](int i) { return __hip_atomic_load(base + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); },
+           []() { return (uint64_t)wall_clock64(); }) &&
+       ok;
+  const uint64_t(&v)[PER] = wave.v;
   double x = 0.0;
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
@@ -173,7 +166,8 @@ __device__ __forceinline__ double exchange(uint64_t* words, uint32_t mine, int n
     const uint64_t bits = (uint64_t)__double_as_longlong(x);
     const uint32_t word = lane < DOUBLE_WORDS ? (uint32_t)((lane & 1) ? bits >> 32 : bits) : (uint32_t)x;
     // a wait that ran out publishes nothing: the other blocks run out too
-    if (lane < USED && ok) put_word(sums + grp * NW + lane, word, tag);
+    if (!ok) return 0.0;
+    if (lane < USED) put_word(sums + grp * NW + lane, word, tag);
   }
   return read_lines<NW, USED, DOUBLE_WORDS, 8>(sums, 8, tag, wait_ticks, max_word, ok);
 }
