@@ -530,6 +530,21 @@ cvo_status cvo_set_profiling(cvo_ctx* ctx, int32_t on);
 cvo_status cvo_get_kernel_stats(cvo_ctx* ctx, cvo_kernel_stats* out);
 cvo_status cvo_reset_kernel_stats(cvo_ctx* ctx);
 
+/* How a context's registrations (align, adaptive lengthscale) ran since it was
+ * created.  A registration runs as one resident launch where its rows fit the
+ * compute units' LDS and no other resident launch of the process holds the
+ * units; otherwise, and from where a resident launch was abandoned, it runs
+ * pass by pass.  An abandoned launch is one whose blocks waited longer than
+ * CVO_LOOP_WAIT_MS (environment; milliseconds) for one another, as when another
+ * process holds some of the compute units; its result is that of the passes. */
+enum {
+  CVO_LOOP_COMPLETED = 0,  /* registrations that ran resident to their end    */
+  CVO_LOOP_ABANDONED = 1,  /* resident launches given up for the passes       */
+  CVO_LOOP_DECLINED = 2,   /* registrations that did not try                  */
+  CVO_LOOP_COUNT = 3
+};
+cvo_status cvo_get_loop_counts(const cvo_ctx* ctx, int64_t counts[CVO_LOOP_COUNT]);
+
 /* Library version string. */
 const char* cvo_version(void);
 

@@ -519,14 +519,20 @@ static cvo_status run_resident(cvo_ctx* ctx, const Problems& pr, const KConsts& 
   for (int q = 0; q < np; ++q) rows[q] = pr.host[q].n_src;
   LoopShape shape;
   LoopUnits held;
+  int64_t* counts = ctx->loop_counts;
+  counts[CVO_LOOP_DECLINED]++;  // until it is known to run
   if (!loop_shape(kc, rows, np, units, &shape) || !held.claim(ctx->device, shape.blocks, units)) return CVO_OK;
   hipStream_t st = ctx->stream;
   const size_t words = loop_words_bytes(), backup = sizeof(ProblemState) * np;
-  // a workspace limit that holds the rest of the call must not fail for this
+  // memory or a workspace limit that holds the rest of the call must not fail for this
   const size_t args_at = align_up(words + 256 + backup, 256), need = args_at + sizeof(LoopArgs);
   const bool limited = ctx->ws_limit > 0 && ctx->b_loop.cap < need;
   if (limited && ctx->ws_bytes + need + need / 4 > ctx->ws_limit) return CVO_OK;
-  CVO_TRY(ensure(ctx, ctx->b_loop, need));
+  if (ensure(ctx, ctx->b_loop, need) != CVO_OK) {
+    (void)hipGetLastError();
+    return CVO_OK;
+  }
+  counts[CVO_LOOP_DECLINED]--;
   char* base = as<char>(ctx->b_loop);
   launch_zero(base, words + 256, st);
   LoopArgs a{};
@@ -557,11 +563,15 @@ static cvo_status run_resident(cvo_ctx* ctx, const Problems& pr, const KConsts& 
     if (e == hipSuccess && flags[1]) {
       e = hipMemcpyAsync(pr.states, saved, backup, hipMemcpyDeviceToDevice, st);
       if (e == hipSuccess) e = hipStreamSynchronize(st);
-      if (e == hipSuccess) break;
+      if (e == hipSuccess) {
+        counts[CVO_LOOP_ABANDONED]++;
+        break;
+      }
     }
     if (e != hipSuccess) status = hip_check(ctx, e, "resident loop");
     else if (flags[0] || it + kLoopChunk >= max_iter) {
       *ran = true;
+      counts[CVO_LOOP_COMPLETED]++;
       break;
     }
   }
@@ -1008,6 +1018,12 @@ extern "C" cvo_status cvo_set_profiling(cvo_ctx* ctx, int32_t on) {
 extern "C" cvo_status cvo_get_kernel_stats(cvo_ctx* ctx, cvo_kernel_stats* out) {
   if (!ctx || !out) return CVO_ERR_INVALID_ARG;
   *out = ctx->stats;
+  return CVO_OK;
+}
+
+extern "C" cvo_status cvo_get_loop_counts(const cvo_ctx* ctx, int64_t counts[CVO_LOOP_COUNT]) {
+  if (!ctx || !counts) return CVO_ERR_INVALID_ARG;
+  for (int i = 0; i < CVO_LOOP_COUNT; ++i) counts[i] = ctx->loop_counts[i];
   return CVO_OK;
 }
 

@@ -227,6 +227,7 @@ struct cvo_ctx {
   DevBuf b_tmp0, b_tmp1, b_tmp2, b_tmp3, b_cub;
   DevBuf b_export;
   DevBuf b_loop;  // resident loop: exchange words, wait flag, saved states
+  int64_t loop_counts[CVO_LOOP_COUNT] = {0, 0, 0};
   void* pinned = nullptr;  // small pinned host buffer for flags
   size_t pinned_cap = 0;
   hipEvent_t ev_a = nullptr, ev_b = nullptr;

@@ -76,6 +76,7 @@ def lib() -> C.CDLL:
         L.cvo_workspace_bytes.argtypes = [P, P]
         L.cvo_set_workspace_limit.argtypes = [P, C.c_uint64]
         L.cvo_release_workspace.argtypes = [P]
+        L.cvo_get_loop_counts.argtypes = [P, P]
         L.cvo_get_tuning.argtypes = [P, P]
         L.cvo_set_tuning.argtypes = [P, P]
         L.cvo_autotune.argtypes = [P, P, P, P, C.c_char_p, P]
@@ -683,6 +684,14 @@ class CvoGPU:
 
     def reset_kernel_stats(self) -> None:
         _check(lib().cvo_reset_kernel_stats(self._ctx), self._ctx)
+
+    def loop_counts(self) -> dict:
+        """Registrations of this context that ran as one resident launch to
+        their end, resident launches abandoned for the pass-by-pass loop, and
+        registrations that did not try (cvo_get_loop_counts)."""
+        n = (C.c_int64 * 3)()
+        _check(lib().cvo_get_loop_counts(self._ctx, n), self._ctx)
+        return dict(zip(("completed", "abandoned", "declined"), n))
 
 
 def version() -> str:
