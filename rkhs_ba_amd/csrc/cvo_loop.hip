@@ -51,6 +51,10 @@ constexpr int kLoopWaves = kLoopThreads / 64;
 constexpr int kLoopMaxBlocks = 256;
 constexpr int kGroupBlocks = kLoopMaxBlocks / 8;  // blocks of an exchange's first level
 constexpr uint32_t kCapped = 0x80000000u;  // a row over its cap, to be redone
+// Lanes a row of the K-nearest association, whatever the tuning: at 8 the
+// histograms of the rows in flight (a kilobyte each) would take the 128 KB that
+// the rows need too.
+constexpr int kKnnLanes = 16;
 
 // Rows go to blocks in chunks of kChunk consecutive (Morton-sorted) rows dealt
 // round robin: a block's rows come from all over its XCD's range, so dense and
@@ -719,8 +723,7 @@ __global__ __launch_bounds__(kLoopThreads) void loop_kernel(const LoopArgs* args
   loop_rows<FC, KC, KNN, G>(P, kc, GL, mp, mode, ell0, K, seg[q], seg[q + 1], R, &S.any_capped, acc, nz[q], mxq)
       // as many lanes a row as one round of the block's threads holds
       if constexpr (KNN) {
-        if (uni(state_group(&st)) == 8) CVO_LOOP_ROWS(8);
-        else CVO_LOOP_ROWS(16);
+        CVO_LOOP_ROWS(kKnnLanes);
       } else {
         if (n * 64 <= kLoopThreads) CVO_LOOP_ROWS(64);
         else if (n * 32 <= kLoopThreads) CVO_LOOP_ROWS(32);
@@ -946,7 +949,7 @@ bool loop_shape(const KConsts& kc, const int* rows, int n_probs, int units, Loop
   if (kc.use_col) row += sizeof(float) * kc.F;
   if (kc.use_sem) row += sizeof(float) * kc.Ks;
   // 256-bin histograms: one per row in flight (K nearest), else one per wave
-  const int hists = kc.knn > 0 ? kLoopThreads / std::min(kc.pol.group_big, kc.pol.group_small) : kLoopWaves;
+  const int hists = kc.knn > 0 ? kLoopThreads / kKnnLanes : kLoopWaves;
   s.lds = row * s.rows + sizeof(uint32_t) * 256 * (size_t)hists;
   *out = s;
   return s.lds <= kLoopMaxLds;

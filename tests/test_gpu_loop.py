@@ -99,8 +99,8 @@ def test_sizes(n, m):
     (dict(is_using_semantics=1, s_ell=0.5, s_sigma=1.0, nearest_neighbors_max=9), dict(classes=7, feats=3), {}),
     (dict(is_using_intensity=0, is_using_geometric_type=1), dict(geo=True), {}),
     (dict(is_using_kdtree=2), {}, {}),
-    # its histograms leave no LDS for the rows
-    (dict(is_using_kdtree=1), {}, dict(tuning=dict(lanes_per_row=8), ran="declined")),
+    (dict(is_using_kdtree=1), {}, dict(tuning=dict(lanes_per_row=8))),
+    (dict(is_using_kdtree=1), dict(classes=19), dict(tuning=dict(lanes_per_row=16, lanes_small_ell=4, split_ell=0.3))),
     ({}, {}, dict(pose="reference")),
     ({}, {}, dict(tuning=dict(lanes_per_row=4, cell_scale=0.5, xcd_remap=0))),
     ({}, dict(feats=8), dict(adaptive=True)),
