@@ -535,8 +535,10 @@ cvo_status cvo_reset_kernel_stats(cvo_ctx* ctx);
  * compute units' LDS and no other resident launch of the process holds the
  * units; otherwise, and from where a resident launch was abandoned, it runs
  * pass by pass.  An abandoned launch is one whose blocks waited longer than
- * CVO_LOOP_WAIT_MS (environment; milliseconds) for one another, as when another
- * process holds some of the compute units; its result is that of the passes. */
+ * CVO_LOOP_WAIT_MS (environment; milliseconds, 100 by default) for one another,
+ * as when another process holds some of the compute units; its result is that of
+ * the passes, and the context's next 32 registrations do not try (twice as many
+ * after each further one, at most 1024, until one completes). */
 enum {
   CVO_LOOP_COMPLETED = 0,  /* registrations that ran resident to their end    */
   CVO_LOOP_ABANDONED = 1,  /* resident launches given up for the passes       */

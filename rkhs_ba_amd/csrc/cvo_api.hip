@@ -503,6 +503,16 @@ static constexpr int kChunk = 24;
 
 // Iterations of one resident launch.
 static constexpr int kLoopChunk = 1024;
+// Longest wait of one of its exchanges (CVO_LOOP_WAIT_MS overrides it).  Blocks of
+// one launch start within a millisecond of one another unless something else
+// holds compute units: another process, whose resident blocks may be waiting for
+// ours to leave, or long kernels of other streams.
+static constexpr double kLoopWaitMs = 100.0;
+// Registrations of a context that leave the loop alone after an abandoned launch;
+// twice as many after each that follows.  Where two processes keep colliding an
+// attempt costs each up to two waits, so the pause bounds the loss to a few
+// milliseconds a registration.
+static constexpr int kLoopPause = 32, kLoopPauseMax = 1024;
 
 // The iteration loop as resident launches (cvo_loop.hip), where its rows fit
 // the blocks' LDS and the device's compute units are not held by other such
@@ -521,6 +531,10 @@ static cvo_status run_resident(cvo_ctx* ctx, const Problems& pr, const KConsts& 
   LoopUnits held;
   int64_t* counts = ctx->loop_counts;
   counts[CVO_LOOP_DECLINED]++;  // until it is known to run
+  if (ctx->loop_rest > 0) {
+    ctx->loop_rest--;
+    return CVO_OK;
+  }
   if (!loop_shape(kc, rows, np, units, &shape) || !held.claim(ctx->device, shape.blocks, units)) return CVO_OK;
   hipStream_t st = ctx->stream;
   const size_t words = loop_words_bytes(), backup = sizeof(ProblemState) * np;
@@ -545,9 +559,8 @@ static cvo_status run_resident(cvo_ctx* ctx, const Problems& pr, const KConsts& 
   a.xb = loop_step_words(a.xa);
   a.fail = reinterpret_cast<uint32_t*>(base + words);
   char* saved = base + words + 256;
-  // CVO_LOOP_WAIT_MS: longest wait of one exchange (2 s)
   const char* wm = std::getenv("CVO_LOOP_WAIT_MS");
-  a.wait_ticks = (uint64_t)((wm && wm[0] ? std::max(0.0, std::atof(wm)) : 2000.0) * 1e5);
+  a.wait_ticks = (uint64_t)((wm && wm[0] ? std::max(0.0, std::atof(wm)) : kLoopWaitMs) * 1e5);
   volatile int32_t* flags = reinterpret_cast<volatile int32_t*>(ctx->pinned);
   cvo_status status = CVO_OK;
   for (int it = 0; it < max_iter && status == CVO_OK; it += kLoopChunk) {
@@ -565,6 +578,8 @@ static cvo_status run_resident(cvo_ctx* ctx, const Problems& pr, const KConsts& 
       if (e == hipSuccess) e = hipStreamSynchronize(st);
       if (e == hipSuccess) {
         counts[CVO_LOOP_ABANDONED]++;
+        ctx->loop_pause = std::min(kLoopPauseMax, std::max(kLoopPause, 2 * ctx->loop_pause));
+        ctx->loop_rest = ctx->loop_pause;
         break;
       }
     }
@@ -572,6 +587,7 @@ static cvo_status run_resident(cvo_ctx* ctx, const Problems& pr, const KConsts& 
     else if (flags[0] || it + kLoopChunk >= max_iter) {
       *ran = true;
       counts[CVO_LOOP_COMPLETED]++;
+      ctx->loop_pause = 0;
       break;
     }
   }

@@ -118,6 +118,37 @@ def test_a_wait_that_runs_out_falls_back():
     both(params(), src, tgt, env={"CVO_LOOP_WAIT_MS": "0"}, ran="abandoned")
 
 
+def test_a_context_pauses_after_an_abandoned_launch():
+    # the launch itself ends at once (no wait); each later one that is abandoned
+    # doubles the pause, one that completes ends it
+    src, tgt = pair(513, 300)
+    cvo = CvoGPU(params=params())
+    try:
+        def align(times, wait=None):
+            before = cvo.loop_counts()
+            if wait is not None:
+                os.environ["CVO_LOOP_WAIT_MS"] = wait
+            try:
+                Ts = [cvo.align(src, tgt, np.eye(4))[1] for _ in range(times)]
+            finally:
+                os.environ.pop("CVO_LOOP_WAIT_MS", None)
+            for T in Ts:
+                np.testing.assert_allclose(T, want, rtol=0, atol=2e-6)
+            return [v - before[k] for k, v in cvo.loop_counts().items()]
+
+        want = cvo.align(src, tgt, np.eye(4))[1]
+        print("pause after an abandoned launch", flush=True)
+        assert align(1, "0") == [0, 1, 0]
+        assert align(32, "0") == [0, 0, 32]
+        assert align(1, "0") == [0, 1, 0]
+        assert align(64) == [0, 0, 64]
+        assert align(3) == [3, 0, 0]
+        assert align(1, "0") == [0, 1, 0]
+        assert align(33) == [1, 0, 32]
+    finally:
+        cvo.close()
+
+
 def test_threads_share_the_compute_units():
     # four registrations at once, each wanting every compute unit
     src, tgt = pair(4500, 4500)
