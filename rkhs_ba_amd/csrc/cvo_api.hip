@@ -353,8 +353,15 @@ cvo_status build_grid(cvo_ctx* ctx, const cvo_dcloud* t, const std::vector<float
   return build_grid_into(ctx, t, hs, gh, ctx->b_grid_store, ctx->b_gridhdr);
 }
 
+// Cell size for one lengthscale: cell_scale x the ball's radius.
+float one_level_size(const KConsts& kc, float ell, float max_norm, float tq, float cell_scale) {
+  const float r = radius_for(kc, ell, max_norm, tq);
+  return (r > 0 ? r : 1.0f) * cell_scale * 1.02f;
+}
+
 // Cell sizes for lengthscales from ell_hi down to ell_lo, ratio 0.7, the finest
-// reaching cell_scale x the radius at ell_lo.
+// reaching cell_scale x the radius at ell_lo.  One lengthscale has one level, of
+// the launch policy's scale there (cell_scale is the least of both its scales).
 std::vector<float> level_sizes(const KConsts& kc, float ell_hi, float ell_lo, float max_norm, float tq,
                                float cell_scale) {
   std::vector<float> hs;
@@ -363,8 +370,10 @@ std::vector<float> level_sizes(const KConsts& kc, float ell_hi, float ell_lo, fl
   float r_hi = radius_for(kc, ell_hi, max_norm, tq);
   float r_lo = radius_for(kc, ell_lo, max_norm, tq) * cell_scale;
   if (!(r_hi > 0)) r_hi = 1.0f;
-  // one lengthscale: the one level its passes use
-  if (ell_hi == ell_lo) return {r_hi * cell_scale * 1.02f};
+  if (ell_hi == ell_lo) {
+    const float scale = policy_big(kc.pol, ell_hi) ? kc.pol.scale_big : kc.pol.scale_small;
+    return {one_level_size(kc, ell_hi, max_norm, tq, std::max(cell_scale, scale))};
+  }
   float h = r_hi * 1.02f;
   for (int l = 0; l < kMaxLevels; ++l) {
     hs.push_back(h);

@@ -263,6 +263,7 @@ cvo_status ensure(cvo_ctx* ctx, DevBuf& b, size_t bytes);
 KConsts make_kconsts(const cvo_params& p, int F, int Ks, int mode);
 cvo_status validate_pair(cvo_ctx* ctx, const cvo_dcloud* s, const cvo_dcloud* t);
 float radius_for(const KConsts& kc, float ell, float max_norm, float tq);
+float one_level_size(const KConsts& kc, float ell, float max_norm, float tq, float cell_scale);
 std::vector<float> level_sizes(const KConsts& kc, float ell_hi, float ell_lo, float max_norm, float tq,
                                float cell_scale);
 void apply_tuning(const cvo_ctx* ctx, KConsts& kc, bool batched = false);

@@ -185,3 +185,43 @@ def test_four_lane_tuning_in_batched_launches(ctx):
         ret, T, secs, iters, _ = ctx.align(src, tgt, Ts[s])
         assert iters == out["per_start_iters"][s]
         assert rot_dist_rad(T, out["per_start_T"][s]) <= 1e-9 and trans_err(T, out["per_start_T"][s]) <= 1e-9, s
+
+
+def test_one_lengthscale_has_the_level_its_policy_takes():
+    """With ell_init == ell_min a registration has one grid level: that of the
+    policy's half which the lengthscale is in, whatever the other half's scale
+    (the arena holds what a context with that scale alone holds); the autotuner
+    times its three scales on a level each."""
+    p = params_from_yaml("planes_spheres_5k.yaml")
+    p.ell_init = p.ell_min = 0.3
+    p.MAX_ITER = 2
+    n = 9000
+    src, tgt, _ = synth.planes_spheres_pair(3, n, n)
+
+    def arena(call):
+        c = CvoGPU(params=p)
+        try:
+            call(c, c.upload(src), c.upload(tgt))
+            return c.workspace_bytes()
+        finally:
+            c.close()
+
+    def aligned(**tuning):
+        def call(c, ds, dt):
+            c.set_tuning(16, 1, **tuning)
+            c.align(ds, dt, np.eye(4))
+        say(f"one lengthscale {tuning}")
+        return arena(call)
+
+    coarse, fine = aligned(cell_scale=1.0), aligned(cell_scale=0.4)
+    assert coarse < fine
+    assert aligned(cell_scale=1.0, split_ell=0.1, cell_scale_small_ell=0.4) == coarse
+    assert aligned(cell_scale=1.0, split_ell=0.5, cell_scale_small_ell=0.4) == fine
+    assert aligned(cell_scale=0.4, split_ell=0.1, cell_scale_small_ell=1.0) == fine
+    say("autotune at one lengthscale")
+    tuned = arena(lambda c, ds, dt: c.autotune(ds, dt, np.eye(4), cache=None))
+    # two levels more than the registration at the finest scale: a point's
+    # position, id and five features each, with the arena's headroom; the
+    # registration holds the resident loop's words besides
+    level = 1.25 * n * (16 + 4 + 4 * 5)
+    assert tuned >= aligned(cell_scale=0.5) + 2 * level - 200_000, tuned
