@@ -28,10 +28,15 @@
 // iteration, into sums over them of {1, d0, d0 d0^T}, a {1, d0, d0 d0^T, |d0|^2 d0}
 // and a^2 {1, d0, d0 d0^T, |d0|^2 d0, |d0|^4} times the monomials of p1 up to the
 // degree that each meets, and every candidate of the solve evaluates the
-// polynomials.  d0 is small (the association's radius) and p1 is taken about its
-// cloud's centre, so that the expansion loses no digits: the poses of a 12-frame
-// window after 12 outer iterations equal those of sums over the pairs at every
-// candidate to 2e-16 (relative).
+// polynomials.  p1 is taken about the mean of the edge's paired points, where the
+// parts of e cancel least (about the middle of a cloud's bounding box one stray
+// return at 30 km moved the poses of two outer iterations by 5e-9, one at 1000
+// km, as a sensor's mark for no return, by 8e-3).  What the expansion loses is the
+// cancellation of d0 against e: relative to FP64's 2e-16 a factor of
+// (max(|d0|, |e|) / |d|) to the power 2 in S, 3 in h and 4 in c, none where a
+// candidate moves the points by less than their offsets.  Observed: a 12-frame
+// window's pose entries after 12 outer iterations against those of sums over the
+// pairs at every candidate, 2e-16 of the largest.
 //
 // The Ceres solve is replaced by this Levenberg-Marquardt schedule:
 //   D = clamp(diag(H), 1e-6, 1e32); solve (H + D/mu) d = -g;
@@ -77,7 +82,7 @@ struct BaEdge {
   int32_t f1, f2;
   int32_t K, last_max, iters_per_ell, on;
   int32_t n_rows, n_blocks;
-  int32_t pad0, pad1;
+  double centre[3];  // mean of the paired source points, in their frame
 };
 
 struct BaDev {
@@ -93,7 +98,6 @@ struct BaDev {
   int32_t free_idx[kBaMaxFrames];
   int32_t frame_of_free[kBaMaxFree];
   float frame_norm[kBaMaxFrames];
-  double centre[kBaMaxFrames * 3];  // of each cloud, in its frame
   double X[kBaMaxFrames * 12];     // current poses, row-major 3x4 (world <- sensor)
   double Xe[kBaMaxFrames * 12];    // poses of the pending pair pass
   double Xold[kBaMaxFrames * 12];  // poses at the start of the outer iteration
@@ -289,6 +293,43 @@ __device__ __forceinline__ void relative_map(const double* T1, const double* T2,
   }
 }
 
+// The mean of each edge's paired source points (a point counts once a pair), the
+// origin of its moments.  One block an edge, sums in fixed order; bound by the
+// latency of its rows' reads.
+__global__ __launch_bounds__(1024) void ba_centre_kernel(const BaDev* __restrict__ ba, BaEdge* __restrict__ edges,
+                                                         const AssocProblem* __restrict__ probs) {
+  if (ba->done || !ba->eval_pending) return;
+  BaEdge& ed = edges[blockIdx.x];
+  if (!ed.on) return;
+  const AssocProblem& P = probs[blockIdx.x];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  double v[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+  for (int r = tid; r < P.n_src; r += 1024) {
+    const double n = (double)ld_global(P.counts + r);
+    const float4 p = ld_global(P.src_pos + r);
+    v[0] = fma(n, (double)p.x, v[0]);
+    v[1] = fma(n, (double)p.y, v[1]);
+    v[2] = fma(n, (double)p.z, v[2]);
+    v[3] += n;
+  }
+  __shared__ double s_v[16][4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o, 64);
+    if (lane == 0) s_v[wave][k] = v[k];
+  }
+  __syncthreads();
+  if (tid < 3) {
+    double x = 0.0, n = 0.0;
+    for (int w = 0; w < 16; ++w) {
+      x += s_v[w][tid];
+      n += s_v[w][3];
+    }
+    ed.centre[tid] = x / n;  // an edge that is on has pairs
+  }
+}
+
 // The pairs' moments, once an outer iteration (at the association's poses, X).
 // A lane owns a source row and reads its pairs in order, four loads in flight;
 // FP64 sums of 37 moments in registers.  Then the wave's 64 rows times their
@@ -318,7 +359,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   const size_t row_stride = (size_t)P.st->K;
   double A[12];
   relative_map(ba->X + 12 * ed.f1, ba->X + 12 * ed.f2, A);
-  const double c0 = ba->centre[3 * ed.f1], c1 = ba->centre[3 * ed.f1 + 1], c2 = ba->centre[3 * ed.f1 + 2];
+  const double c0 = ed.centre[0], c1 = ed.centre[1], c2 = ed.centre[2];
   double4_t acc[kMomTiles];
 #pragma unroll
   for (int t = 0; t < kMomTiles; ++t) acc[t] = (double4_t){0.0, 0.0, 0.0, 0.0};
@@ -516,7 +557,7 @@ __global__ __launch_bounds__(384) void ba_eval_kernel(const BaDev* __restrict__ 
     double A[12], A0[12];
     relative_map(ba->Xe + 12 * ed.f1, T2, A);
     relative_map(ba->Xold + 12 * ed.f1, ba->Xold + 12 * ed.f2, A0);
-    const double* c = ba->centre + 3 * ed.f1;
+    const double* c = ed.centre;
     const int r = tid;
     double Ar[4], A0r[4];
 #pragma unroll
@@ -1247,6 +1288,7 @@ static void ba_assoc_phase(const BaLaunch& L, hipStream_t s) {
 // e0 / e1 (optional): events at the moment kernel's own start and end.
 static void ba_moments_phase(const BaLaunch& L, hipStream_t s, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
   const dim3 g(L.max_mom_blocks, L.n_edges), b(256);
+  hipLaunchKernelGGL(ba_centre_kernel, dim3(L.n_edges), dim3(1024), 0, s, L.ba, L.edges, L.probs);
   if (e0) hipExtLaunchKernelGGL(ba_moments_kernel, g, b, 0, s, e0, e1, 0, L.ba, L.edges, L.probs, L.part, L.max_mom_blocks);
   else hipLaunchKernelGGL(ba_moments_kernel, g, b, 0, s, L.ba, L.edges, L.probs, L.part, L.max_mom_blocks);
   hipLaunchKernelGGL(ba_moments_sum_kernel, dim3(L.n_edges, kMomTiles), dim3(256), 0, s, L.ba, L.edges, L.part,
@@ -1419,7 +1461,6 @@ extern "C" cvo_status cvo_align_multiframe(cvo_ctx* ctx, int32_t n_frames, const
     hb->free_idx[f] = (!hold_const || !hold_const[f]) ? o++ : -1;
     if (hb->free_idx[f] >= 0) hb->frame_of_free[hb->free_idx[f]] = f;
     hb->frame_norm[f] = frames[f]->max_norm;
-    for (int d = 0; d < 3; ++d) hb->centre[3 * f + d] = 0.5 * ((double)frames[f]->bmin[d] + (double)frames[f]->bmax[d]);
     for (int i = 0; i < 12; ++i) hb->X[12 * f + i] = poses[12 * f + i];
   }
   hb->done = p.multiframe_max_iters <= 0 ? 1 : 0;

@@ -180,6 +180,24 @@ def test_moments_match_oracle(ba_gpu, oracle, sizes, shift):
     np.testing.assert_allclose(g["poses"][:, :3, :4], P[:, :3, :4], rtol=0, atol=1e-8 if shift else 1e-9)
 
 
+@pytest.mark.parametrize("far", [200.0, 4000.0, 3e4, 1e5, 1e6])
+def test_moments_of_clouds_with_a_stray_return_match_oracle(ba_gpu, oracle, far):
+    """One point of each cloud far from the rest moves the middle of its bounding
+    box by half as much, and no pair: the moments are taken about the paired
+    points.  1e-9 as above."""
+    p = params_from_yaml("ba_window.yaml")
+    p.multiframe_max_iters = 2
+    p.multiframe_min_nonzeros = 1
+    clouds, gts, inits = window(seed=11, n_frames=3)
+    away = [(far, 0.3 * far, 0.0), (-0.6 * far, far, 1.0), (0.2 * far, -far, -2.0)]
+    clouds = [synth.Cloud(np.concatenate([c.xyz, np.float32([a])]), *(None if x is None else np.concatenate([x, x[:1]])
+                          for x in (c.feat, c.sem))) for c, a in zip(clouds, away)]
+    g, P, it = run_both(ba_gpu, oracle, p, clouds, inits, [1, 0, 0], [(0, 1), (1, 2), (2, 0)])
+    assert g["iters"] == it
+    say(f"stray at {far}: {np.abs(g['poses'][:, :3, :4] - P[:, :3, :4]).max():.3e}")
+    np.testing.assert_allclose(g["poses"][:, :3, :4], P[:, :3, :4], rtol=0, atol=1e-9)
+
+
 @pytest.mark.parametrize("free", [1, 2, 10, 11, 20])
 def test_solve_sizes_match_oracle(ba_gpu, oracle, free):
     """The normal equations of 6 dof (less than a factorisation block) to 120
