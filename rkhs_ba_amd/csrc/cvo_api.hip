@@ -98,7 +98,7 @@ cvo_status ensure(cvo_ctx* ctx, DevBuf& b, size_t bytes) {
   return CVO_OK;
 }
 
-static void free_buf(cvo_ctx* ctx, DevBuf& b) {
+void free_buf(cvo_ctx* ctx, DevBuf& b) {
   if (b.p) (void)hipFree(b.p);
   ctx->ws_bytes -= b.cap;
   b.p = nullptr;

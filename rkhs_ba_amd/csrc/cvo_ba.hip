@@ -68,9 +68,10 @@ constexpr int kBaMaxFree = 20;                 // free frames: 120 dof, Cholesky
 constexpr int kBaMaxDof = 6 * kBaMaxFree;
 constexpr int kBaMaxEdges = 4096;
 constexpr int kBaContrib = 121;                // B11, B12, B22 (36 each), g1, g2 (6 each), c
-constexpr int kMomRows = 512;                  // source rows of a moment block
+constexpr int kMomRows = 512;                  // source rows of a moment block (more where memory is short)
 constexpr int kMomTiles = 5;                   // 16 x 16 tiles of the moment matrix that are used
 constexpr int kMomPart = kMomTiles * 256;
+constexpr int kMomUsed = 670;                  // their entries that are (mom_index)
 constexpr int kSolveThreads = 256;             // four waves: the Cholesky's trailing update spread over rows
 static_assert(kSolveThreads == 256 && 6 * kBaMaxFree <= kSolveThreads, "the solve's reductions assume four waves");
 constexpr int kChol = 8;                       // Cholesky block: columns a panel (even, as the dof are)
@@ -82,6 +83,7 @@ struct BaEdge {
   int32_t f1, f2;
   int32_t K, last_max, iters_per_ell, on;
   int32_t n_rows, n_blocks;
+  int32_t part0, pad;  // the first of its blocks' partials
   double centre[3];  // mean of the paired source points, in their frame
 };
 
@@ -276,6 +278,19 @@ __constant__ MonoTables kMonoTab;
 constexpr int kM_n = 0, kM_a0 = 1, kM_b0 = 2, kM_D1 = 3, kM_a1 = 6, kM_b1 = 9;
 constexpr int kM_D2 = 16, kM_a2 = 22, kM_b2 = 28, kM_a3 = 34, kM_b3 = 37, kM_b4 = 40, kMomRowsUsed = 41;
 
+// Where an entry of the tiles lies in a stored set of moments, -1 if nothing
+// uses it.  Tiles 0 to 2 have 12 rows, the last of them 3 columns; tiles 3 and 4
+// have 10 columns, the last of them 9 rows.
+__device__ __forceinline__ int mom_index(int i) {
+  const int t = i >> 8, r = (i >> 4) & 15, c = i & 15;
+  if (t < 3) return r < 12 && (t < 2 || c < kMono - 32) ? (t < 2 ? t * 192 + r * 16 + c : 384 + r * 3 + c) : -1;
+  return c < kQuad && (t < 4 || r < kMomRowsUsed - 32) ? 420 + (t - 3) * 160 + r * kQuad + c : -1;
+}
+static_assert(kMomUsed == 2 * 12 * 16 + 12 * (kMono - 32) + 16 * kQuad + (kMomRowsUsed - 32) * kQuad, "the stored entries");
+// An edge's moments lie in its slot of the association's capped-row partials,
+// which the association is done with by then.
+static_assert(kMomUsed <= 10 * kOvfBlocks, "the moments fit the slots");
+
 // Sum of moment m times monomial q in the summed tiles.
 __device__ __forceinline__ double mom(const double* s_m, int m, int q) {
   const int tile = m < 16 ? q >> 4 : 2 + (m >> 4);
@@ -342,7 +357,7 @@ __global__ __launch_bounds__(1024) void ba_centre_kernel(const BaDev* __restrict
 // iterations).
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void ba_moments_kernel(const BaDev* __restrict__ ba, const BaEdge* __restrict__ edges,
                                                          const AssocProblem* __restrict__ probs,
-                                                         double* __restrict__ part, int max_blocks) {
+                                                         double* __restrict__ part, int rows) {
   if (ba->done || !ba->eval_pending) return;
   const int e = blockIdx.y;
   const BaEdge& ed = edges[e];
@@ -363,7 +378,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   double4_t acc[kMomTiles];
 #pragma unroll
   for (int t = 0; t < kMomTiles; ++t) acc[t] = (double4_t){0.0, 0.0, 0.0, 0.0};
-  for (int base = blockIdx.x * kMomRows; base < (int)(blockIdx.x + 1) * kMomRows && base < P.n_src; base += 256) {
+  for (int base = blockIdx.x * rows; base < (int)(blockIdx.x + 1) * rows && base < P.n_src; base += 256) {
     const int r = base + wave * 64 + lane;
     uint32_t cnt = 0;
     double y0 = 0.0, y1 = 0.0, y2 = 0.0, x = 0.0, y = 0.0, z = 0.0;
@@ -494,7 +509,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     }
   }
   // the four waves' tiles in order; lane: rows (lane >> 4) + 4 v, column lane & 15
-  double* out = part + ((size_t)e * max_blocks + blockIdx.x) * kMomPart;
+  double* out = part + (size_t)(ed.part0 + blockIdx.x) * kMomUsed;
   static_assert(16 * (kSM + kSQ) >= kMomPart, "a wave's tiles fit its staging");
   __syncthreads();
 #pragma unroll
@@ -502,25 +517,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 #pragma unroll
     for (int v = 0; v < 4; ++v) s_stage[wave][t * 256 + ((lane >> 4) + 4 * v) * 16 + (lane & 15)] = acc[t][v];
   __syncthreads();
-  for (int i = tid; i < kMomPart; i += 256)
-    out[i] = ((s_stage[0][i] + s_stage[1][i]) + s_stage[2][i]) + s_stage[3][i];
+  for (int i = tid; i < kMomPart; i += 256) {
+    const int k = mom_index(i);
+    if (k >= 0) out[k] = ((s_stage[0][i] + s_stage[1][i]) + s_stage[2][i]) + s_stage[3][i];
+  }
 }
 
 // An edge's moments: the blocks' partials in order.
 __global__ __launch_bounds__(256) void ba_moments_sum_kernel(const BaDev* __restrict__ ba,
                                                              const BaEdge* __restrict__ edges,
-                                                             const double* __restrict__ part, int max_blocks,
+                                                             const double* __restrict__ part,
                                                              double* __restrict__ moments) {
   if (ba->done || !ba->eval_pending) return;
   const int e = blockIdx.x;
   const BaEdge& ed = edges[e];
   if (!ed.on) return;
   const int i = blockIdx.y * 256 + threadIdx.x;
-  const double* p = part + (size_t)e * max_blocks * kMomPart + i;
+  if (i >= kMomUsed) return;
+  const double* p = part + (size_t)ed.part0 * kMomUsed + i;
   double v = 0.0;
 #pragma unroll 8
-  for (int b = 0; b < ed.n_blocks; ++b) v += p[(size_t)b * kMomPart];
-  moments[(size_t)e * kMomPart + i] = v;
+  for (int b = 0; b < ed.n_blocks; ++b) v += p[(size_t)b * kMomUsed];
+  moments[(size_t)e * kMomUsed + i] = v;
 }
 
 // S, h and c of an edge at the poses Xe from its moments, and the edge's blocks
@@ -548,7 +566,10 @@ __global__ __launch_bounds__(384) void ba_eval_kernel(const BaDev* __restrict__ 
   __shared__ double s_V[60], s_F[12], s_c;
   __shared__ int8_t s_mul[kQuad][kQuad];
   __shared__ double s_M1[36], s_M2[36], s_N1[36], s_N2[36], s_S[36], s_h[6], s_T1[36], s_T2[36];
-  for (int i = tid; i < kMomPart; i += blockDim.x) s_m[i] = moments[(size_t)e * kMomPart + i];
+  for (int i = tid; i < kMomPart; i += blockDim.x) {
+    const int k = mom_index(i);
+    s_m[i] = k >= 0 ? moments[(size_t)e * kMomUsed + k] : 0.0;
+  }
   if (tid < kQuad * kQuad) s_mul[tid / kQuad][tid % kQuad] = kMonoTab.mul[tid / kQuad][tid % kQuad];
   const double* T2 = ba->Xe + 12 * ed.f2;
   if (tid == 128) pose_M(ba->Xe + 12 * ed.f1, s_M1);
@@ -1219,7 +1240,7 @@ static T* as(DevBuf& b) {
 
 enum {
   BA_PAIRS = 0, BA_COUNTS, BA_OVF, BA_STATE, BA_PROBS, BA_PART_A, BA_PART_OVF, BA_PART_CNT,
-  BA_DEV, BA_EDGES, BA_H, BA_HN, BA_PAIR_PART, BA_CONTRIB, BA_MOMENTS, BA_PAIR_IDS
+  BA_DEV, BA_EDGES, BA_H, BA_HN, BA_MOM_PART, BA_CONTRIB, BA_PAIR_IDS
 };
 
 // Six buffers per frame: sorted source (pos, feat, sem, geo), grid store and
@@ -1268,8 +1289,8 @@ struct BaLaunch {
   BaDev* ba;
   BaEdge* edges;
   AssocProblem* probs;
-  int n_edges, total_blocks, max_mom_blocks, lm_rounds, n_asm_blocks;
-  double* part;
+  int n_edges, total_blocks, mom_rows, max_mom_blocks, lm_rounds, n_asm_blocks;
+  double* part;     // blocks' moments; the edges' own where each edge has one block
   double* moments;
   double* contrib;
   double* H;  // two n x n halves: current linearisation and evaluation
@@ -1289,10 +1310,11 @@ static void ba_assoc_phase(const BaLaunch& L, hipStream_t s) {
 static void ba_moments_phase(const BaLaunch& L, hipStream_t s, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
   const dim3 g(L.max_mom_blocks, L.n_edges), b(256);
   hipLaunchKernelGGL(ba_centre_kernel, dim3(L.n_edges), dim3(1024), 0, s, L.ba, L.edges, L.probs);
-  if (e0) hipExtLaunchKernelGGL(ba_moments_kernel, g, b, 0, s, e0, e1, 0, L.ba, L.edges, L.probs, L.part, L.max_mom_blocks);
-  else hipLaunchKernelGGL(ba_moments_kernel, g, b, 0, s, L.ba, L.edges, L.probs, L.part, L.max_mom_blocks);
-  hipLaunchKernelGGL(ba_moments_sum_kernel, dim3(L.n_edges, kMomTiles), dim3(256), 0, s, L.ba, L.edges, L.part,
-                     L.max_mom_blocks, L.moments);
+  if (e0) hipExtLaunchKernelGGL(ba_moments_kernel, g, b, 0, s, e0, e1, 0, L.ba, L.edges, L.probs, L.part, L.mom_rows);
+  else hipLaunchKernelGGL(ba_moments_kernel, g, b, 0, s, L.ba, L.edges, L.probs, L.part, L.mom_rows);
+  if (L.part != L.moments)
+    hipLaunchKernelGGL(ba_moments_sum_kernel, dim3(L.n_edges, (kMomUsed + 255) / 256), dim3(256), 0, s, L.ba, L.edges,
+                       L.part, L.moments);
 }
 
 static void ba_lm_round(const BaLaunch& L, hipStream_t s) {
@@ -1313,6 +1335,17 @@ static void ba_iteration(const BaLaunch& L, hipStream_t s) {
 }  // namespace cvo
 
 using namespace cvo;
+
+// Under a workspace limit the moment partials are given back at the end: other
+// calls may need the room that this one used.
+struct PartHolder {
+  cvo_ctx* ctx;
+  DevBuf& b;
+  void release() {
+    if (ctx->ws_limit > 0) free_buf(ctx, b);
+  }
+  ~PartHolder() { release(); }
+};
 
 extern "C" cvo_status cvo_align_multiframe(cvo_ctx* ctx, int32_t n_frames, const cvo_dcloud* const* frames,
                                            double* poses, const uint8_t* hold_const, int32_t n_edges,
@@ -1359,13 +1392,13 @@ extern "C" cvo_status cvo_align_multiframe(cvo_ctx* ctx, int32_t n_frames, const
   // per-edge association problems
   const int cap = p.multiframe_num_neighbors;
   size_t tot_rows = 0;
-  int total_blocks = 0, max_mom_blocks = 1;
+  int total_blocks = 0, max_rows = 1;
   std::vector<size_t> row_off(n_edges + 1, 0);
   for (int e = 0; e < n_edges; ++e) {
     const int n = frames[edges[2 * e]]->n;
     row_off[e + 1] = row_off[e] + (size_t)n;
     total_blocks += (n + rb - 1) / rb;
-    max_mom_blocks = std::max(max_mom_blocks, (n + kMomRows - 1) / kMomRows);
+    max_rows = std::max(max_rows, n);
   }
   tot_rows = row_off[n_edges];
   const size_t E1 = (size_t)std::max(n_edges, 1);
@@ -1381,17 +1414,33 @@ extern "C" cvo_status cvo_align_multiframe(cvo_ctx* ctx, int32_t n_frames, const
   CVO_TRY(ensure(ctx, B[BA_DEV], sizeof(BaDev)));
   CVO_TRY(ensure(ctx, B[BA_EDGES], sizeof(BaEdge) * E1));
   CVO_TRY(ensure(ctx, B[BA_H], sizeof(double) * 2 * kBaMaxDof * kBaMaxDof));
-  CVO_TRY(ensure(ctx, B[BA_PAIR_PART], sizeof(double) * kMomPart * (size_t)max_mom_blocks * E1));
   CVO_TRY(ensure(ctx, B[BA_CONTRIB], sizeof(double) * kBaContrib * E1));
-  CVO_TRY(ensure(ctx, B[BA_MOMENTS], sizeof(double) * kMomPart * E1));
   // the export needs each stored pair's target (its sorted position)
   if (per_edge) CVO_TRY(ensure(ctx, B[BA_PAIR_IDS], sizeof(uint32_t) * std::max<size_t>(tot_rows, 1) * cap));
+  // Moment blocks of kMomRows rows; of twice as many, and so on, where a workspace
+  // limit would not hold their partials.  One block an edge needs none: it writes
+  // the edge's moments, in memory that the association has anyway.
+  int mom_rows = kMomRows;
+  auto mom_blocks = [&](int n) { return (n + mom_rows - 1) / mom_rows; };
+  auto part_bytes = [&]() {
+    size_t blocks = 0;
+    if (max_rows > mom_rows)
+      for (int e = 0; e < n_edges; ++e) blocks += (size_t)mom_blocks(frames[edges[2 * e]]->n);
+    return sizeof(double) * kMomUsed * blocks;
+  };
+  if (ctx->ws_limit > 0) {
+    const size_t held = ctx->ws_bytes - B[BA_MOM_PART].cap;
+    const size_t room = ctx->ws_limit > held ? (ctx->ws_limit - held) / 5 * 4 : 0;  // the arena's headroom
+    while (part_bytes() > room) mom_rows *= 2;
+  }
+  PartHolder part_holder{ctx, B[BA_MOM_PART]};
+  if (part_bytes() > 0) CVO_TRY(ensure(ctx, B[BA_MOM_PART], part_bytes()));
   CVO_HIP(ctx, hipMemsetAsync(B[BA_OVF].p, 0, sizeof(uint32_t) * std::max<size_t>(tot_rows, 1), st));
   CVO_HIP(ctx, hipMemsetAsync(B[BA_STATE].p, 0, sizeof(ProblemState) * E1, st));
 
   std::vector<AssocProblem> hp(E1);
   std::vector<BaEdge> he(E1);
-  int blk = 0;
+  int blk = 0, mom_blk = 0;
   for (int e = 0; e < n_edges; ++e) {
     const int f1 = edges[2 * e], f2 = edges[2 * e + 1];
     const cvo_dcloud* s = frames[f1];
@@ -1433,7 +1482,9 @@ extern "C" cvo_status cvo_align_multiframe(cvo_ctx* ctx, int32_t n_frames, const
     ed.f2 = f2;
     ed.K = cap;
     ed.n_rows = n;
-    ed.n_blocks = (n + kMomRows - 1) / kMomRows;
+    ed.n_blocks = mom_blocks(n);
+    ed.part0 = mom_blk;
+    mom_blk += ed.n_blocks;
   }
   if (n_edges > 0) {
     CVO_HIP(ctx, hipMemcpyAsync(B[BA_PROBS].p, hp.data(), sizeof(AssocProblem) * n_edges, hipMemcpyHostToDevice, st));
@@ -1476,11 +1527,12 @@ extern "C" cvo_status cvo_align_multiframe(cvo_ctx* ctx, int32_t n_frames, const
   L.probs = as<AssocProblem>(B[BA_PROBS]);
   L.n_edges = n_edges;
   L.total_blocks = total_blocks;
-  L.max_mom_blocks = max_mom_blocks;
+  L.mom_rows = mom_rows;
+  L.max_mom_blocks = mom_blocks(max_rows);
   L.lm_rounds = std::max(0, p.multiframe_iterations_per_solve) + 1;
   L.n_asm_blocks = std::max(1, nfree * nfree + nfree);
-  L.part = as<double>(B[BA_PAIR_PART]);
-  L.moments = as<double>(B[BA_MOMENTS]);
+  L.moments = as<double>(B[BA_PART_OVF]);
+  L.part = part_bytes() > 0 ? as<double>(B[BA_MOM_PART]) : L.moments;
   L.contrib = as<double>(B[BA_CONTRIB]);
   L.H = as<double>(B[BA_H]);
   L.kc = kc;
@@ -1620,6 +1672,7 @@ extern "C" cvo_status cvo_align_multiframe(cvo_ctx* ctx, int32_t n_frames, const
   ctx->ba_last_accepted = out->accepted_total;
   ctx->ba_last_evals = out->evals_total;
   delete out;
+  part_holder.release();  // the exports need the room
   // with multiframe_max_iters > 0 the first outer iteration associates
   const bool any_pass = p.multiframe_max_iters > 0;
   // each edge's pairs of the last association pass (BinaryStateGPU::

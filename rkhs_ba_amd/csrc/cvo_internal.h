@@ -260,6 +260,7 @@ struct GridHost {
 cvo_status set_err(cvo_ctx* ctx, cvo_status s, const std::string& msg);
 cvo_status hip_check(cvo_ctx* ctx, hipError_t e, const char* what);
 cvo_status ensure(cvo_ctx* ctx, DevBuf& b, size_t bytes);
+void free_buf(cvo_ctx* ctx, DevBuf& b);  // waits for the device
 KConsts make_kconsts(const cvo_params& p, int F, int Ks, int mode);
 cvo_status validate_pair(cvo_ctx* ctx, const cvo_dcloud* s, const cvo_dcloud* t);
 float radius_for(const KConsts& kc, float ell, float max_norm, float tq);

@@ -198,6 +198,40 @@ def test_moments_of_clouds_with_a_stray_return_match_oracle(ba_gpu, oracle, far)
     np.testing.assert_allclose(g["poses"][:, :3, :4], P[:, :3, :4], rtol=0, atol=1e-9)
 
 
+def test_ragged_window_within_a_workspace_limit():
+    """One long frame among short ones: the moments' partials are those of each
+    edge's own blocks, and under a limit that does not hold them the blocks walk
+    more rows, down to one an edge.  Same pairs, FP64 sums in another order: 1e-9."""
+    p = params_from_yaml("ba_window.yaml")
+    p.multiframe_max_iters = 2
+    p.multiframe_min_nonzeros = 1
+    p.multiframe_num_neighbors = 64
+    sizes = [20000] + [400] * 7
+    clouds, gts, inits = window(seed=11, n_frames=8, n_min=20000, n_max=20000)
+    clouds = [c.subset(np.arange(n)) for c, n in zip(clouds, sizes)]
+    edges, hold = all_edges(8), [1] + [0] * 7
+
+    def run(limit):
+        c = CvoGPU(params=p)
+        try:
+            c.set_workspace_limit(limit)
+            say(f"ragged window, limit {limit}")
+            r = c.align_multiframe(clouds, inits, hold, edges)
+            return r["poses"], c.workspace_bytes()
+        finally:
+            c.close()
+
+    want, used = run(0)
+    # 7 edges of 20000 rows and 21 of 400: 301 blocks of 512 rows, 670 doubles each
+    partials = 5 * 8 * 670 * 301 // 4
+    for short in (0, partials // 3, partials // 4 * 3, partials):
+        got, held = run(used - short)
+        assert held <= used - partials + 4096  # given back
+        np.testing.assert_allclose(got[:, :3, :4], want[:, :3, :4], rtol=0, atol=1e-9)
+    with pytest.raises(CvoError):
+        run(used // 2)
+
+
 @pytest.mark.parametrize("free", [1, 2, 10, 11, 20])
 def test_solve_sizes_match_oracle(ba_gpu, oracle, free):
     """The normal equations of 6 dof (less than a factorisation block) to 120
