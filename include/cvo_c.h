@@ -519,7 +519,9 @@ cvo_status cvo_tuning_cache_store(const char* path, const char* key, const cvo_t
 /* Device bytes the context's arena holds now. */
 cvo_status cvo_workspace_bytes(const cvo_ctx* ctx, uint64_t* out);
 /* Caps the arena (0: no cap).  A call that would grow it beyond the cap fails
- * with CVO_ERR_LIMIT before allocating, and the context stays usable. */
+ * with CVO_ERR_LIMIT before allocating, and the context stays usable.  A limit
+ * set where there was none frees the arena, and the untuned launch shape takes
+ * the coarsest grid cells under one (results as with another tuning). */
 cvo_status cvo_set_workspace_limit(cvo_ctx* ctx, uint64_t bytes);
 /* Frees the arena (the next call grows it again). */
 cvo_status cvo_release_workspace(cvo_ctx* ctx);

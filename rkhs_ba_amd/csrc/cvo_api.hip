@@ -411,12 +411,16 @@ void apply_tuning(const cvo_tuning& t, KConsts& kc, bool batched) {
 // (one-variant build) 625 / 517 / 489; the 12-frame window 42.3 / 39.2 / 38.7 and
 // 41.2 / 39.8 / 38.0.  A single registration takes cell scale 0.7: 60k street
 // 86.4 / 82.3 / 82.6 ms, K nearest at 20k 24.0 / 22.7 / 23.6, no difference below
-// 5k points; a single pass keeps 1 (its one grid is built for it alone).
+// 5k points; a single pass keeps 1 (its one grid is built for it alone).  The finer
+// cells and the levels that reach them take arena: 21 -> 110 MB for an adaptive
+// registration of 300 points, 69 -> 106 for a registration of 9000.  So a context
+// with a workspace limit keeps cells of the radius.
 void apply_tuning(const cvo_ctx* ctx, KConsts& kc, bool batched) {
   cvo_tuning t = ctx->tuning;
   if (t.source == CVO_TUNE_DEFAULT) {
     if (batched) t.lanes_per_row = t.lanes_small_ell = 8;
-    t.cell_scale = t.cell_scale_small_ell = batched ? 0.5f : (kc.mode == MODE_ALIGN ? 0.7f : 1.0f);
+    const float scale = batched ? 0.5f : (kc.mode == MODE_ALIGN ? 0.7f : 1.0f);
+    t.cell_scale = t.cell_scale_small_ell = ctx->ws_limit > 0 ? 1.0f : scale;
   }
   apply_tuning(t, kc, batched);
 }
@@ -1882,6 +1886,11 @@ extern "C" cvo_status cvo_workspace_bytes(const cvo_ctx* ctx, uint64_t* out) {
 
 extern "C" cvo_status cvo_set_workspace_limit(cvo_ctx* ctx, uint64_t bytes) {
   if (!ctx) return CVO_ERR_INVALID_ARG;
+  if (ctx->ws_limit == 0 && bytes > 0) {
+    // calls without a limit took more than they need under one
+    CVO_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    for_each_buf(ctx, free_buf);
+  }
   ctx->ws_limit = (size_t)bytes;
   return CVO_OK;
 }

@@ -95,3 +95,43 @@ def test_value_ordered_association_rows():
         else:
             assert (np.diff(cb) > 0).all()
     assert n_sorted > 100
+
+
+@pytest.mark.parametrize("n", [300, 1100, 9000])
+def test_a_limit_holds_the_coarsest_launch_shape(n):
+    """An untuned context's finer grid cells take more arena than cells of the
+    ball's radius; under a limit that holds only these a call still runs, from a
+    fresh context and from one that ran without a limit.  Same pairs, FP64 sums in
+    another order: poses to 2e-6 (float output) over 12 iterations, 1e-9 over two
+    outer iterations of a window."""
+    src, tgt, _ = synth.planes_spheres_pair(1, n, n)
+    p = params_from_yaml("planes_spheres_5k.yaml")
+    p.MAX_ITER = 12
+    pb = params_from_yaml("ba_window.yaml")
+    pb.multiframe_max_iters = 2
+    pb.multiframe_num_neighbors = 32
+    pb.multiframe_min_nonzeros = 1
+    clouds, _, inits = synth.window_frames(1, n_frames=3, n_min=n, n_max=n + 50)
+    starts = np.stack([np.eye(4, dtype=np.float32)] * 4)
+    calls = {
+        "align": (p, 16, lambda c: c.align(src, tgt, np.eye(4))[1], 2e-6),
+        "adaptive": (p, 8, lambda c: c.align_adaptive(src, tgt, np.eye(4))[1], 2e-6),
+        "starts": (p, 8, lambda c: c.align_multistart(c.upload(src), c.upload(tgt), starts, 0.3)["per_start_T"], 2e-6),
+        "window": (pb, 8, lambda c: c.align_multiframe(clouds, inits, [1, 0, 0], [(0, 1), (1, 2), (0, 2)])["poses"], 1e-9),
+    }
+    for name, (params, lanes, call, tol) in calls.items():
+        say(f"limit of the coarsest shape: {name} n={n}")
+        coarse, fine, limited = (CvoGPU(params=params) for _ in range(3))
+        try:
+            coarse.set_tuning(lanes, 1, 1.0)
+            want = call(coarse)
+            limit = coarse.workspace_bytes()
+            np.testing.assert_allclose(call(fine), want, rtol=0, atol=tol)
+            assert fine.workspace_bytes() > limit
+            for c in (limited, fine):
+                c.set_workspace_limit(limit)
+                np.testing.assert_allclose(call(c), want, rtol=0, atol=tol)
+                assert c.workspace_bytes() <= limit
+        finally:
+            for c in (coarse, fine, limited):
+                c.close()
