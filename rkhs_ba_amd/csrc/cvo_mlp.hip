@@ -934,8 +934,8 @@ struct cvo_model {
 namespace {
 
 enum {
-  WS_PTS = 0, WS_X, WS_CEN, WS_H1, WS_H2, WS_POOL, WS_Z, WS_GVAL, WS_GARG, WS_Z1, WS_O, WS_TGT, WS_DO, WS_DOB,
-  WS_DZ1, WS_DZ, WS_ROWV, WS_XG, WS_H1G, WS_DH2, WS_DH1, WS_LOSS, WS_QT, WS_CONF, WS_STAGE, WS_PART, WS_COUNT
+  WS_PTS = 0, WS_X, WS_CEN, WS_H1, WS_H2, WS_Z, WS_GVAL, WS_GARG, WS_Z1, WS_O, WS_TGT, WS_DO, WS_DOB,
+  WS_DZ1, WS_DZ, WS_ROWV, WS_XG, WS_H1G, WS_DH2, WS_DH1, WS_LOSS, WS_QT, WS_CONF, WS_STAGE, WS_COUNT
 };
 static_assert(WS_COUNT <= 32, "the model's workspace array holds 32 buffers");
 
@@ -965,7 +965,11 @@ cvo_status forward(cvo_model* m, int n_pairs, int npts, bool train) {
     CVO_TRY(ensure(ctx, m->ws[WS_H2], sizeof(uint16_t) * P * kH2));
   }
   const int splits = encoder_splits(clouds, npts);
-  CVO_TRY(ensure(ctx, m->ws[WS_POOL], sizeof(unsigned long long) * clouds * splits * kH3));
+  // the blocks' pooled keys (2 KB for every 128 points of a cloud, and 2 KB at
+  // least) go where the points were (32 bytes each, 64 points at least), which
+  // the preparation is done with by then
+  static_assert(kH3 * sizeof(unsigned long long) * 2 <= sizeof(float) * kMlpIn * kFT, "the keys fit the points");
+  unsigned long long* pool = wsp<unsigned long long>(m, WS_PTS);
   CVO_TRY(ensure(ctx, m->ws[WS_Z], sizeof(uint16_t) * n_pairs * kZ));
   CVO_TRY(ensure(ctx, m->ws[WS_GVAL], sizeof(float) * clouds * kH3));
   CVO_TRY(ensure(ctx, m->ws[WS_GARG], sizeof(int32_t) * clouds * kH3));
@@ -977,12 +981,10 @@ cvo_status forward(cvo_model* m, int n_pairs, int npts, bool train) {
   const int64_t npool = (int64_t)clouds * kH3;
   GemmArgs g;
   hipLaunchKernelGGL(train ? encoder_fused_kernel<true> : encoder_fused_kernel<false>, dim3(clouds * splits), dim3(256),
-                     0, s, wsp<uint16_t>(m, WS_X), npts, m->W1b, m->W2b, m->W3b, w,
-                     wsp<unsigned long long>(m, WS_POOL), splits, train ? wsp<uint16_t>(m, WS_H1) : nullptr,
-                     train ? wsp<uint16_t>(m, WS_H2) : nullptr);
+                     0, s, wsp<uint16_t>(m, WS_X), npts, m->W1b, m->W2b, m->W3b, w, pool, splits,
+                     train ? wsp<uint16_t>(m, WS_H1) : nullptr, train ? wsp<uint16_t>(m, WS_H2) : nullptr);
   hipLaunchKernelGGL(mlp_unpack_pool_kernel, dim3((unsigned)((npool + 255) / 256)), dim3(256), 0, s,
-                     wsp<unsigned long long>(m, WS_POOL), splits, n_pairs, wsp<uint16_t>(m, WS_Z), wsp<float>(m, WS_GVAL),
-                     wsp<int32_t>(m, WS_GARG));
+                     pool, splits, n_pairs, wsp<uint16_t>(m, WS_Z), wsp<float>(m, WS_GVAL), wsp<int32_t>(m, WS_GARG));
   // head
   g = gemm_args(wsp<uint16_t>(m, WS_Z), kZ, 1, m->W4b, kZ1, 1, n_pairs, kZ1, kZ);
   g.bias = w + oB4;
@@ -1145,9 +1147,13 @@ extern "C" cvo_status cvo_model_gradient(cvo_ctx* ctx, cvo_model* m, int32_t n_p
   CVO_TRY(ensure(ctx, m->ws[WS_DH2], sizeof(uint16_t) * (size_t)R * kH2));
   CVO_TRY(ensure(ctx, m->ws[WS_DH1], sizeof(uint16_t) * (size_t)R * kH1));
   CVO_TRY(ensure(ctx, m->ws[WS_LOSS], sizeof(float) * n_pairs));
-  // at most 128 partials, of at least two tiles (R = 512 rows a pair)
-  const int rows_per = std::max(2, (R / kRgTile + 127) / 128) * kRgTile, parts = (R + rows_per - 1) / rows_per;
-  CVO_TRY(ensure(ctx, m->ws[WS_PART], sizeof(float) * (size_t)parts * kRgPart));
+  // at most 128 partials, of at least two tiles (R = 512 rows a pair), and what
+  // fits where the second layer's activations were, which nothing reads by then
+  // (one does with 64 points a cloud, all do from 300)
+  const int most = (int)std::min<size_t>(128, m->ws[WS_H2].cap / (sizeof(float) * kRgPart));
+  if (most < 1) return set_err(ctx, CVO_ERR_LIMIT, "the gradient's partials exceed their buffer");
+  const int rows_per = std::max(2, (R / kRgTile + most - 1) / most) * kRgTile, parts = (R + rows_per - 1) / rows_per;
+  float* part = wsp<float>(m, WS_H2);
   CVO_HIP(ctx, hipMemcpyAsync(m->ws[WS_TGT].p, targets, sizeof(float) * 7 * n_pairs, hipMemcpyHostToDevice, s));
   hipLaunchKernelGGL(mlp_loss_kernel, dim3((n_pairs + 63) / 64), dim3(64), 0, s, wsp<float>(m, WS_O),
                      wsp<float>(m, WS_TGT), wsp<float>(m, WS_CEN), n_pairs, wsp<float>(m, WS_DO),
@@ -1194,9 +1200,8 @@ extern "C" cvo_status cvo_model_gradient(cvo_ctx* ctx, cvo_model* m, int32_t n_p
   gemm(g, s);
   hipLaunchKernelGGL(mlp_rowgrad_kernel, dim3(parts), dim3(256), 0, s, wsp<uint16_t>(m, WS_H1G),
                      wsp<uint16_t>(m, WS_DH2), wsp<uint16_t>(m, WS_XG), wsp<uint16_t>(m, WS_DH1), R, rows_per,
-                     wsp<float>(m, WS_PART));
-  hipLaunchKernelGGL(mlp_rowgrad_sum_kernel, dim3((kRgPart + 255) / 256), dim3(256), 0, s, wsp<float>(m, WS_PART), parts,
-                     gr);
+                     part);
+  hipLaunchKernelGGL(mlp_rowgrad_sum_kernel, dim3((kRgPart + 255) / 256), dim3(256), 0, s, part, parts, gr);
   CVO_HIP(ctx, hipGetLastError());
   if (grad_out) {
     CVO_HIP(ctx, hipMemcpyAsync(grad_out, gr, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost, s));

@@ -139,3 +139,27 @@ def test_split_clouds_match_oracle(prop, n, npts):
     Lo, go = M.gradient(w, a.astype(np.float64), b.astype(np.float64), t.astype(np.float64), quantize=True)
     assert abs(loss - Lo) <= 1e-2 * abs(Lo)
     assert rel(g, go) < 1e-2
+
+
+@pytest.mark.parametrize("n,npts", [(1, 64), (1, 2048), (40, 128), (128, 512)])
+def test_gradient_fits_its_activations(cvo_gpu, n, npts):
+    """The pooled keys of a cloud's blocks and the weight gradients' partials take
+    no arena of their own: a gradient runs within a workspace limit of its points,
+    activations, gathered rows and head (each with the arena's headroom)."""
+    from rkhs_ba_amd import CvoGPU
+    from rkhs_ba_amd.proposer import PoseProposer
+    a, b, t = batch(7, 1, npts)
+    a, b, t = (np.tile(x, (n,) + (1,) * (x.ndim - 1)) for x in (a, b, t))
+    points = 2 * n * npts * (2 * 32 + 32 + 128 + 256)
+    rows = 512 * n * (32 + 128 + 256 + 128 + 4)
+    head = n * (96 + 1024 + 2048 + 2048 + 512 + 256 + 28 + 256 + 128 + 512 + 2048 + 4)
+    c = CvoGPU(params=cvo_gpu.get_params())
+    p = PoseProposer(c, seed=3)
+    try:
+        c.set_workspace_limit(c.workspace_bytes() + 5 * (points + rows + head) // 4 + 256)
+        say(f"gradient within a limit: {n} pairs x {npts}")
+        loss, g = p.gradient(a, b, t)
+    finally:
+        p.close()
+        c.close()
+    assert np.isfinite(loss) and np.isfinite(g).all()
