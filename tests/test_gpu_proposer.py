@@ -120,7 +120,8 @@ def test_training_reduces_loss(cvo_gpu):
 def test_split_clouds_match_oracle(prop, n, npts):
     """Forward and gradient where a cloud's points are one wave's rows, part of a
     tile, several tiles over several blocks, and one block a cloud (260 clouds);
-    rows of the weight gradients in two tiles a block and more."""
+    rows of the weight gradients in two tiles a block and, at 130 pairs, in nine
+    with a short last range."""
     a, b, t = batch(5, min(n, 3), npts)
     reps = -(-n // a.shape[0])
     a, b, t = (np.tile(x, (reps,) + (1,) * (x.ndim - 1))[:n] for x in (a, b, t))
@@ -134,11 +135,16 @@ def test_split_clouds_match_oracle(prop, n, npts):
     _, _, alone = prop.propose(a[:1], b[:1])
     assert np.array_equal(alone[0], raw[0])
     loss, g = prop.gradient(a, b, t)
-    if n > 3:
-        return
     Lo, go = M.gradient(w, a.astype(np.float64), b.astype(np.float64), t.astype(np.float64), quantize=True)
     assert abs(loss - Lo) <= 1e-2 * abs(Lo)
     assert rel(g, go) < 1e-2
+    # every layer's weights and biases by themselves
+    at = 0
+    for rows, cols in ((8, 64), (64, 128), (128, 256), (512, 256), (256, 64)):
+        for size in (rows * cols, cols):
+            assert rel(g[at:at + size], go[at:at + size]) < 1e-2, (at, size)
+            at += size
+    assert at == g.size
 
 
 @pytest.mark.parametrize("n,npts", [(1, 64), (1, 2048), (40, 128), (128, 512)])
