@@ -721,13 +721,16 @@ __global__ __launch_bounds__(kLoopThreads) void loop_kernel(const LoopArgs* args
       const int n = seg[q + 1] - seg[q];
 #define CVO_LOOP_ROWS(G)                                                                                         \
   loop_rows<FC, KC, KNN, G>(P, kc, GL, mp, mode, ell0, K, seg[q], seg[q + 1], R, &S.any_capped, acc, nz[q], mxq)
-      // as many lanes a row as one round of the block's threads holds
+      // As many lanes a row as one round of the block's threads holds, else 16, or 4
+      // where the tuning says 4.  8 lanes are 16 here: at 60000 rows (street pair,
+      // 300 iterations, cell scale 1 / 0.5) 16 took 39.7 / 31.9 ms, 4 took 59.0 /
+      // 49.7, and the launch-per-pass loop at its 8 51.8 / 44.6.
       if constexpr (KNN) {
         CVO_LOOP_ROWS(kKnnLanes);
       } else {
         if (n * 64 <= kLoopThreads) CVO_LOOP_ROWS(64);
         else if (n * 32 <= kLoopThreads) CVO_LOOP_ROWS(32);
-        else if (n * 16 <= kLoopThreads || uni(state_group(&st)) == 16) CVO_LOOP_ROWS(16);
+        else if (n * 16 <= kLoopThreads || uni(state_group(&st)) > 4) CVO_LOOP_ROWS(16);
         else CVO_LOOP_ROWS(4);
       }
 #undef CVO_LOOP_ROWS

@@ -93,6 +93,12 @@ def test_sizes(n, m):
     both(params(), src, tgt)
 
 
+@pytest.mark.parametrize("lanes", [4, 8])
+def test_lanes_of_more_rows_than_a_round(lanes):
+    src, tgt = pair(20011, 20011)
+    both(params(), src, tgt, tuning=dict(lanes_per_row=lanes, cell_scale=0.7))
+
+
 @pytest.mark.parametrize("kw,cloud,opts", [
     (dict(nearest_neighbors_max=6), {}, {}),                                   # rows over the cap
     (dict(is_using_semantics=1, s_ell=0.5, s_sigma=1.0), dict(classes=19), {}),
