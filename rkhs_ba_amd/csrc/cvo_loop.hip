@@ -935,8 +935,20 @@ bool loop_shape(const KConsts& kc, const int* rows, int n_probs, int units, Loop
   // without the distance gate every row scans all targets: that work is not
   // spread by rows
   if (!kc.use_geo || kc.uncapped || kc.mode != MODE_ALIGN) return false;
+  // The loop saves launches, states read back and counters, about 15 us an
+  // iteration; the passes have more waves in flight a row.  Registrations of 1000
+  // iterations, passes / loop: planes at 60k rows 129 / 117 ms, at 80k 186 / 178,
+  // street at 100k 136 / 110, at 150k 226 / 204; their first 200 iterations, which
+  // have the most pairs, street at 80k 46.0 / 43.9, 120k 81.9 / 81.1, 200k 184 / 209.
+  // K nearest, 600 iterations: planes at 20k 45.5 / 42.7, 30k 68.4 / 69.0, 60k 181 /
+  // 196 (street at 60k 69.6 / 64.4).  Adaptive lengthscale: 15k 12.8 / 11.5, 20k 16.2 /
+  // 18.7, 40k 34.0 / 41.2, from where a problem's rows take the blocks a second round.
+  const int most = kc.adaptive ? 16384 : (kc.knn > 0 ? 32768 : 131072);
   int64_t total = 0;
-  for (int q = 0; q < n_probs; ++q) total += rows[q];
+  for (int q = 0; q < n_probs; ++q) {
+    if (rows[q] > most) return false;
+    total += rows[q];
+  }
   if (total <= 0) return false;
   // 16 rows a block (a wave each) as far as the units go; whole XCD rounds
   int blocks = (int)std::min<int64_t>(std::min(units, kLoopMaxBlocks), (total + 15) / 16);

@@ -93,6 +93,17 @@ def test_sizes(n, m):
     both(params(), src, tgt)
 
 
+@pytest.mark.parametrize("n,kw,adaptive", [(131072, {}, False), (32768, dict(is_using_kdtree=1), False),
+                                           (16384, {}, True)])
+def test_most_rows(n, kw, adaptive):
+    src, tgt = pair(n + 1, 700)
+    both(params(MAX_ITER=2, **kw), src.subset(np.arange(n)), tgt, adaptive)
+    both(params(MAX_ITER=2, **kw), src, tgt, adaptive, ran="declined")
+    if adaptive:  # the self problem of the target has rows too
+        both(params(MAX_ITER=2), tgt, src.subset(np.arange(n)), adaptive)
+        both(params(MAX_ITER=2), tgt, src, adaptive, ran="declined")
+
+
 @pytest.mark.parametrize("lanes", [4, 8])
 def test_lanes_of_more_rows_than_a_round(lanes):
     src, tgt = pair(20011, 20011)
