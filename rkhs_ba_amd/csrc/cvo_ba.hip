@@ -28,7 +28,7 @@
 // iteration, into sums over them of {1, d0, d0 d0^T}, a {1, d0, d0 d0^T, |d0|^2 d0}
 // and a^2 {1, d0, d0 d0^T, |d0|^2 d0, |d0|^4} times the monomials of p1 up to the
 // degree that each meets, and every candidate of the solve evaluates the
-// polynomials.  p1 is taken about the mean of the edge's paired points, where the
+// polynomials.  p1 is taken about a mean of the edge's paired points, where the
 // parts of e cancel least (about the middle of a cloud's bounding box one stray
 // return at 30 km moved the poses of two outer iterations by 5e-9, one at 1000
 // km, as a sensor's mark for no return, by 8e-3).  What the expansion loses is the
@@ -84,7 +84,7 @@ struct BaEdge {
   int32_t K, last_max, iters_per_ell, on;
   int32_t n_rows, n_blocks;
   int32_t part0, pad;  // the first of its blocks' partials
-  double centre[3];  // mean of the paired source points, in their frame
+  double centre[3];  // origin of the moments, in the source's frame (moment_origin)
 };
 
 struct BaDev {
@@ -308,41 +308,36 @@ __device__ __forceinline__ void relative_map(const double* T1, const double* T2,
   }
 }
 
-// The mean of each edge's paired source points (a point counts once a pair), the
-// origin of its moments.  One block an edge, sums in fixed order; bound by the
-// latency of its rows' reads.
-__global__ __launch_bounds__(1024) void ba_centre_kernel(const BaDev* __restrict__ ba, BaEdge* __restrict__ edges,
-                                                         const AssocProblem* __restrict__ probs) {
-  if (ba->done || !ba->eval_pending) return;
-  BaEdge& ed = edges[blockIdx.x];
-  if (!ed.on) return;
-  const AssocProblem& P = probs[blockIdx.x];
+// The origin of an edge's moments: the mean of the paired rows among 256 spread
+// over the edge's rows, of the next such set where none of these has a pair.  Each
+// block of the edge forms it, with the same operations; a launch of its own for the
+// mean of all would add 10 us to an outer iteration.  s: 16 words of LDS.
+__device__ __forceinline__ void moment_origin(const AssocProblem& P, double* s, double c[3]) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int stride = (P.n_src + 255) / 256;
   double v[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll 4
-  for (int r = tid; r < P.n_src; r += 1024) {
-    const double n = (double)ld_global(P.counts + r);
-    const float4 p = ld_global(P.src_pos + r);
-    v[0] = fma(n, (double)p.x, v[0]);
-    v[1] = fma(n, (double)p.y, v[1]);
-    v[2] = fma(n, (double)p.z, v[2]);
-    v[3] += n;
+  for (int k = 0; k < stride; ++k) {
+    const int r = tid * stride + k;
+    if (r < P.n_src && ld_global(P.counts + r) != 0u) {
+      const float4 p = ld_global(P.src_pos + r);
+      v[0] = (double)p.x;
+      v[1] = (double)p.y;
+      v[2] = (double)p.z;
+      v[3] = 1.0;
+    }
+    if (__syncthreads_or(v[3] != 0.0)) break;  // an edge that is on has pairs
   }
-  __shared__ double s_v[16][4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o, 64);
-    if (lane == 0) s_v[wave][k] = v[k];
+    if (lane == 0) s[wave * 4 + k] = v[k];
   }
   __syncthreads();
-  if (tid < 3) {
-    double x = 0.0, n = 0.0;
-    for (int w = 0; w < 16; ++w) {
-      x += s_v[w][tid];
-      n += s_v[w][3];
-    }
-    ed.centre[tid] = x / n;  // an edge that is on has pairs
-  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) v[k] = ((s[k] + s[4 + k]) + s[8 + k]) + s[12 + k];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) c[k] = uni(v[k] / v[3]);
+  __syncthreads();  // s is used again
 }
 
 // The pairs' moments, once an outer iteration (at the association's poses, X).
@@ -355,7 +350,7 @@ __global__ __launch_bounds__(1024) void ba_centre_kernel(const BaDev* __restrict
 // times an outer iteration (window of 12 frames of 5k to 40k points), this 298 us
 // once and 8 us for each candidate's polynomials (window: 61.7 -> 45.3 ms for 12 outer
 // iterations).
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void ba_moments_kernel(const BaDev* __restrict__ ba, const BaEdge* __restrict__ edges,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void ba_moments_kernel(const BaDev* __restrict__ ba, BaEdge* __restrict__ edges,
                                                          const AssocProblem* __restrict__ probs,
                                                          double* __restrict__ part, int rows) {
   if (ba->done || !ba->eval_pending) return;
@@ -374,7 +369,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   const size_t row_stride = (size_t)P.st->K;
   double A[12];
   relative_map(ba->X + 12 * ed.f1, ba->X + 12 * ed.f2, A);
-  const double c0 = ed.centre[0], c1 = ed.centre[1], c2 = ed.centre[2];
+  double c[3];
+  moment_origin(P, s_stage[0], c);
+  const double c0 = c[0], c1 = c[1], c2 = c[2];
+  if (blockIdx.x == 0 && tid < 3) edges[e].centre[tid] = tid == 0 ? c0 : (tid == 1 ? c1 : c2);
   double4_t acc[kMomTiles];
 #pragma unroll
   for (int t = 0; t < kMomTiles; ++t) acc[t] = (double4_t){0.0, 0.0, 0.0, 0.0};
@@ -1309,7 +1307,6 @@ static void ba_assoc_phase(const BaLaunch& L, hipStream_t s) {
 // e0 / e1 (optional): events at the moment kernel's own start and end.
 static void ba_moments_phase(const BaLaunch& L, hipStream_t s, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
   const dim3 g(L.max_mom_blocks, L.n_edges), b(256);
-  hipLaunchKernelGGL(ba_centre_kernel, dim3(L.n_edges), dim3(1024), 0, s, L.ba, L.edges, L.probs);
   if (e0) hipExtLaunchKernelGGL(ba_moments_kernel, g, b, 0, s, e0, e1, 0, L.ba, L.edges, L.probs, L.part, L.mom_rows);
   else hipLaunchKernelGGL(ba_moments_kernel, g, b, 0, s, L.ba, L.edges, L.probs, L.part, L.mom_rows);
   if (L.part != L.moments)
