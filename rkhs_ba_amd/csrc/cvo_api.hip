@@ -403,22 +403,27 @@ void apply_tuning(const cvo_tuning& t, KConsts& kc, bool batched) {
   kc.xcd_remap = t.xcd_remap;
 }
 
-// Until a context is tuned, batched launches take 8 lanes a row and cells of half
-// the ball's radius: they fill the device whatever the lanes, so what counts is
-// the work, and clipped to the ball smaller cells and smaller groups enumerate
-// and mask less of it.  96 starts over 20k points, 300 iterations: 16 lanes
-// 729 / 601 / 590 ms at cell scale 1 / 0.7 / 0.5, 8 lanes 583 / 504 / 480, 4 lanes
-// (one-variant build) 625 / 517 / 489; the 12-frame window 42.3 / 39.2 / 38.7 and
-// 41.2 / 39.8 / 38.0.  A single registration takes cell scale 0.7: 60k street
+// Until a context is tuned, batched launches take cells of half the ball's radius,
+// and 8 lanes a row from 49152 rows: with that many they fill the device whatever
+// the lanes, so what counts is the work, and clipped to the ball smaller cells and
+// smaller groups enumerate and mask less of it.  96 starts over 20k points, 300
+// iterations: 16 lanes 729 / 601 / 590 ms at cell scale 1 / 0.7 / 0.5, 8 lanes 583 /
+// 504 / 480, 4 lanes (one-variant build) 625 / 517 / 489; the 12-frame window 42.3 /
+// 39.2 / 38.7 and 41.2 / 39.8 / 38.0.  Fewer rows leave compute units idle at 8:
+// 60 iterations of 2 starts over 8000 points 4.04 ms at 16 lanes, 5.34 at 8, of 6
+// over 4000 5.05 and 5.56, 6 over 8000 5.31 and 5.75, 48 over 1100 6.07 and 5.65, 48
+// over 4000 10.5 and 9.8.  The adaptive lengthscale keeps 16 (40k points 33.9 and
+// 37.9).  A single registration takes cell scale 0.7: 60k street
 // 86.4 / 82.3 / 82.6 ms, K nearest at 20k 24.0 / 22.7 / 23.6, no difference below
 // 5k points; a single pass keeps 1 (its one grid is built for it alone).  The finer
 // cells and the levels that reach them take arena: 21 -> 110 MB for an adaptive
 // registration of 300 points, 69 -> 106 for a registration of 9000.  So a context
 // with a workspace limit keeps cells of the radius.
-void apply_tuning(const cvo_ctx* ctx, KConsts& kc, bool batched) {
+void apply_tuning(const cvo_ctx* ctx, KConsts& kc, int64_t batched_rows) {
   cvo_tuning t = ctx->tuning;
+  const bool batched = batched_rows > 0;
   if (t.source == CVO_TUNE_DEFAULT) {
-    if (batched) t.lanes_per_row = t.lanes_small_ell = 8;
+    if (batched_rows >= 49152 && !kc.adaptive) t.lanes_per_row = t.lanes_small_ell = 8;
     const float scale = batched ? 0.5f : (kc.mode == MODE_ALIGN ? 0.7f : 1.0f);
     t.cell_scale = t.cell_scale_small_ell = ctx->ws_limit > 0 ? 1.0f : scale;
   }
@@ -1206,7 +1211,7 @@ static cvo_status score_poses(cvo_ctx* ctx, const cvo_dcloud* src, const cvo_dcl
   const cvo_params& p = ctx->params;
   KConsts kc = make_kconsts(p, src->F, src->K, MODE_IP);
   kc.knn = 0;
-  apply_tuning(ctx, kc, n > 1);
+  apply_tuning(ctx, kc, n > 1 ? (int64_t)n * src->n : 0);
   kc.n_src_f = (float)src->n;
   kc.n_tgt_f = (float)tgt->n;
   kc.max_src_norm = src->max_norm;
@@ -1572,7 +1577,7 @@ extern "C" cvo_status cvo_align_multistart(cvo_ctx* ctx, const cvo_dcloud* src, 
   hipEvent_t e0 = ctx->ev_pool[4], e1 = ctx->ev_pool[5];
   CVO_HIP(ctx, hipEventRecord(e0, ctx->stream));
   KConsts kc = make_kconsts(p, src->F, src->K, MODE_ALIGN);
-  apply_tuning(ctx, kc, true);  // batched launches
+  apply_tuning(ctx, kc, (int64_t)n_starts * src->n);  // batched launches
   kc.mirror_pose = ctx->pose_arith == CVO_POSE_REFERENCE ? 1 : 0;
   kc.n_src_f = (float)src->n;
   kc.n_tgt_f = (float)tgt->n;
@@ -1705,7 +1710,7 @@ extern "C" cvo_status cvo_align_adaptive_d(cvo_ctx* ctx, const cvo_dcloud* src, 
   KConsts kc = adaptive_kconsts(p, src->F, p.is_using_semantics ? src->K : 0);
   if (!p.is_using_semantics) kc.use_sem = 0;
   kc.amp = kc.sigma2 * kc.c_sigma2 * (kc.use_sem ? kc.s_sigma2 : 1.0f);
-  apply_tuning(ctx, kc, true);  // batched launches
+  apply_tuning(ctx, kc, 2 * (int64_t)src->n + tgt->n);  // batched launches
   kc.mirror_pose = ctx->pose_arith == CVO_POSE_REFERENCE ? 1 : 0;
   kc.n_src_f = (float)src->n;
   kc.n_tgt_f = (float)tgt->n;

@@ -267,7 +267,8 @@ float radius_for(const KConsts& kc, float ell, float max_norm, float tq);
 float one_level_size(const KConsts& kc, float ell, float max_norm, float tq, float cell_scale);
 std::vector<float> level_sizes(const KConsts& kc, float ell_hi, float ell_lo, float max_norm, float tq,
                                float cell_scale);
-void apply_tuning(const cvo_ctx* ctx, KConsts& kc, bool batched = false);
+// batched_rows: the source rows of all problems of a batched launch, 0 for one problem
+void apply_tuning(const cvo_ctx* ctx, KConsts& kc, int64_t batched_rows = 0);
 void apply_tuning(const cvo_tuning& t, KConsts& kc, bool batched = false);
 cvo_status ensure_events(cvo_ctx* ctx, size_t n);
 cvo_status pinned(cvo_ctx* ctx, size_t bytes);

@@ -225,3 +225,30 @@ def test_one_lengthscale_has_the_level_its_policy_takes():
     # registration holds the resident loop's words besides
     level = 1.25 * n * (16 + 4 + 4 * 5)
     assert tuned >= aligned(cell_scale=0.5) + 2 * level - 200_000, tuned
+
+
+@pytest.mark.parametrize("starts,n,lanes", [(2, 4000, 16), (49, 1003, 16), (48, 1024, 8), (64, 1000, 8)])
+def test_untuned_lanes_follow_the_rows(starts, n, lanes):
+    """Untuned batched launches take 16 lanes a row below 49152 rows and 8 from
+    there: their arena (partials a block of rows) is that of the tuned shape, and
+    their poses its poses bit for bit."""
+    p = params_from_yaml("planes_spheres_5k.yaml")
+    p.MAX_ITER = 3
+    p.nearest_neighbors_max = 64
+    src, tgt, _ = synth.planes_spheres_pair(3, n, n)
+    Ts = np.stack([np.eye(4, dtype=np.float32)] * starts)
+
+    def run(**tuning):
+        c = CvoGPU(params=p)
+        try:
+            if tuning:
+                c.set_tuning(**tuning)
+            say(f"{starts} starts over {n} points {tuning}")
+            r = c.align_multistart(c.upload(src), c.upload(tgt), Ts, 0.3)
+            return c.workspace_bytes(), r["per_start_T"]
+        finally:
+            c.close()
+
+    got, want, other = run(), run(lanes_per_row=lanes, cell_scale=0.5), run(lanes_per_row=24 - lanes, cell_scale=0.5)
+    assert got[0] == want[0] != other[0]
+    np.testing.assert_array_equal(got[1], want[1])

@@ -115,9 +115,9 @@ def test_a_limit_holds_the_coarsest_launch_shape(n):
     starts = np.stack([np.eye(4, dtype=np.float32)] * 4)
     calls = {
         "align": (p, 16, lambda c: c.align(src, tgt, np.eye(4))[1], 2e-6),
-        "adaptive": (p, 8, lambda c: c.align_adaptive(src, tgt, np.eye(4))[1], 2e-6),
-        "starts": (p, 8, lambda c: c.align_multistart(c.upload(src), c.upload(tgt), starts, 0.3)["per_start_T"], 2e-6),
-        "window": (pb, 8, lambda c: c.align_multiframe(clouds, inits, [1, 0, 0], [(0, 1), (1, 2), (0, 2)])["poses"], 1e-9),
+        "adaptive": (p, 16, lambda c: c.align_adaptive(src, tgt, np.eye(4))[1], 2e-6),
+        "starts": (p, 16, lambda c: c.align_multistart(c.upload(src), c.upload(tgt), starts, 0.3)["per_start_T"], 2e-6),
+        "window": (pb, 16, lambda c: c.align_multiframe(clouds, inits, [1, 0, 0], [(0, 1), (1, 2), (0, 2)])["poses"], 1e-9),
     }
     for name, (params, lanes, call, tol) in calls.items():
         say(f"limit of the coarsest shape: {name} n={n}")
