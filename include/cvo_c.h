@@ -533,10 +533,10 @@ cvo_status cvo_get_kernel_stats(cvo_ctx* ctx, cvo_kernel_stats* out);
 cvo_status cvo_reset_kernel_stats(cvo_ctx* ctx);
 
 /* How a context's registrations (align, adaptive lengthscale) ran since it was
- * created.  A registration runs as one resident launch where its rows fit the
- * compute units' LDS and no other resident launch of the process holds the
- * units; otherwise, and from where a resident launch was abandoned, it runs
- * pass by pass.  An abandoned launch is one whose blocks waited longer than
+ * created.  A registration runs as resident launches of a few milliseconds where
+ * its rows fit the compute units' LDS, beside other calls of the process on its
+ * share of the units; otherwise, and from where a launch was abandoned or found
+ * no units, it runs pass by pass.  An abandoned launch is one whose blocks waited longer than
  * CVO_LOOP_WAIT_MS (environment; milliseconds, 100 by default) for one another,
  * as when another process holds some of the compute units; its result is that of
  * the passes, and the context's next 32 registrations do not try (twice as many
@@ -544,7 +544,7 @@ cvo_status cvo_reset_kernel_stats(cvo_ctx* ctx);
 enum {
   CVO_LOOP_COMPLETED = 0,  /* registrations that ran resident to their end    */
   CVO_LOOP_ABANDONED = 1,  /* resident launches given up for the passes       */
-  CVO_LOOP_DECLINED = 2,   /* registrations that did not try                  */
+  CVO_LOOP_DECLINED = 2,   /* registrations that did not try, or lost their units */
   CVO_LOOP_COUNT = 3
 };
 cvo_status cvo_get_loop_counts(const cvo_ctx* ctx, int64_t counts[CVO_LOOP_COUNT]);

@@ -32,6 +32,7 @@
 #include <vector>
 
 #include "cvo_internal.h"
+#include "cvo_loop.h"
 #include "cvo_device.h"
 #include "cvo_ball.h"
 
@@ -392,6 +393,7 @@ extern "C" cvo_status cvo_compute_association_nonisotropic(cvo_ctx* ctx, const c
                                                            const cvo_cloud_view* tgt, const float T[16],
                                                            const float kernel[9], cvo_assoc* out) {
   if (!ctx || !src || !tgt || !T || !kernel || !out) return CVO_ERR_INVALID_ARG;
+  ActiveCall busy(ctx);
   std::memset(out, 0, sizeof(*out));
   if (src->n == 0 || tgt->n == 0) return CVO_OK;  // the reference returns without output
   AnisoArgs g{};

@@ -519,8 +519,17 @@ cvo_status ensure_events(cvo_ctx* ctx, size_t n) {
 // done.  Profiling mode launches kernel by kernel with events around each.
 static constexpr int kChunk = 24;
 
-// Iterations of one resident launch.
-static constexpr int kLoopChunk = 1024;
+// Iterations of one resident launch: 4 to 10 milliseconds' worth, the longest that
+// other streams wait for the compute units it holds, and other registrations for
+// their share.  A launch costs 50 us at 5000 rows, 130 at 60000, 0.5 to 1 % of a
+// registration.
+static int loop_chunk(int rows) { return rows > 65536 ? 64 : 256; }
+// Rows a block, at most, of a launch on a share of the units: with 156 two
+// registrations of 20000 points made 156 a second of 100 iterations (passes 147),
+// eight of 5000 488 of 200 (passes 405); with 312 four of 20000 made 176 (passes 195).
+static constexpr int kSharedRows = 160;
+// Longest wait for compute units that other registrations hold.
+static constexpr int kUnitWaitMs = 50;
 // Longest wait of one of its exchanges (CVO_LOOP_WAIT_MS overrides it).  Blocks of
 // one launch start within a millisecond of one another unless something else
 // holds compute units: another process, whose resident blocks may be waiting for
@@ -533,27 +542,33 @@ static constexpr double kLoopWaitMs = 100.0;
 static constexpr int kLoopPause = 32, kLoopPauseMax = 1024;
 
 // The iteration loop as resident launches (cvo_loop.hip), where its rows fit
-// the blocks' LDS and the device's compute units are not held by other such
-// launches.  *ran false: nothing changed, or a wait ran out and the state is
-// that of a whole number of iterations; the caller's launch-per-pass loop goes
-// on from there.
+// the blocks' LDS.  Beside other calls of the process a launch has its share of
+// the compute units: registrations side by side are bound by their own chains, and
+// one that held all units would keep the others waiting.  Four threads with 5000
+// points each, registrations of 200 iterations a second: passes 396, one launch
+// with all units and the rest by passes 218, shares 598.  *ran false: nothing
+// changed, or the state is that of a whole number of iterations (a wait ran out,
+// or the units were not to be had); the caller's launch-per-pass loop goes on from
+// there.
 static cvo_status run_resident(cvo_ctx* ctx, const Problems& pr, const KConsts& kc, int max_iter, bool* ran) {
   *ran = false;
   const int np = pr.n_probs;
   if (np != (kc.adaptive ? 3 : 1)) return CVO_OK;
   int units = 0;
   if (hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess) return CVO_OK;
-  int rows[3] = {0, 0, 0};
-  for (int q = 0; q < np; ++q) rows[q] = pr.host[q].n_src;
-  LoopShape shape;
-  LoopUnits held;
+  int rows[3] = {0, 0, 0}, all_rows = 0;
+  for (int q = 0; q < np; ++q) {
+    rows[q] = pr.host[q].n_src;
+    all_rows += rows[q];
+  }
   int64_t* counts = ctx->loop_counts;
-  counts[CVO_LOOP_DECLINED]++;  // until it is known to run
+  counts[CVO_LOOP_DECLINED]++;  // until it is known to end otherwise
   if (ctx->loop_rest > 0) {
     ctx->loop_rest--;
     return CVO_OK;
   }
-  if (!loop_shape(kc, rows, np, units, &shape) || !held.claim(ctx->device, shape.blocks, units)) return CVO_OK;
+  LoopShape shape;
+  if (!loop_shape(kc, rows, np, units, &shape)) return CVO_OK;
   hipStream_t st = ctx->stream;
   const size_t words = loop_words_bytes(), backup = sizeof(ProblemState) * np;
   // memory or a workspace limit that holds the rest of the call must not fail for this
@@ -564,7 +579,6 @@ static cvo_status run_resident(cvo_ctx* ctx, const Problems& pr, const KConsts& 
     (void)hipGetLastError();
     return CVO_OK;
   }
-  counts[CVO_LOOP_DECLINED]--;
   char* base = as<char>(ctx->b_loop);
   launch_zero(base, words + 256, st);
   LoopArgs a{};
@@ -572,29 +586,38 @@ static cvo_status run_resident(cvo_ctx* ctx, const Problems& pr, const KConsts& 
   for (int q = 0; q < np; ++q) a.prob[q] = pr.host[q];
   // the self problems only sum
   for (int q = 1; q < np; ++q) a.prob[q].pairs = nullptr;
-  a.rows = shape.rows;
   a.xa = reinterpret_cast<uint64_t*>(base);
   a.xb = loop_step_words(a.xa);
-  a.fail = reinterpret_cast<uint32_t*>(base + words);
+  a.flags = reinterpret_cast<uint32_t*>(base + words);
   char* saved = base + words + 256;
   const char* wm = std::getenv("CVO_LOOP_WAIT_MS");
   a.wait_ticks = (uint64_t)((wm && wm[0] ? std::max(0.0, std::atof(wm)) : kLoopWaitMs) * 1e5);
-  volatile int32_t* flags = reinterpret_cast<volatile int32_t*>(ctx->pinned);
+  volatile uint32_t* flags = reinterpret_cast<volatile uint32_t*>(ctx->pinned);
+  const LoopArgs* args = reinterpret_cast<const LoopArgs*>(base + args_at);
+  const int chunk = loop_chunk(all_rows);
+  a.max_iters = chunk;  // the controller ends the registration at its own limit
+  int blocks = 0;  // of the arguments in memory
   cvo_status status = CVO_OK;
-  for (int it = 0; it < max_iter && status == CVO_OK; it += kLoopChunk) {
-    a.max_iters = std::min(kLoopChunk, max_iter - it);
-    a.tag0 = (uint32_t)it + 1u;
+  for (int it = 0; it < max_iter && status == CVO_OK; it += chunk) {
+    LoopUnits held;
+    const int share = loop_share(ctx->device, units);
+    if (!loop_shape(kc, rows, np, share, &shape) || (share < units && shape.rows > kSharedRows) ||
+        !held.claim(ctx->device, shape.blocks, units, kUnitWaitMs))
+      break;
     hipError_t e = hipMemcpyAsync(saved, pr.states, backup, hipMemcpyDeviceToDevice, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(base + args_at, &a, sizeof(a), hipMemcpyHostToDevice, st);
-    if (e == hipSuccess) e = launch_loop(reinterpret_cast<const LoopArgs*>(base + args_at), kc, shape, st);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync((void*)flags, &pr.states[0].done, sizeof(int32_t), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipMemcpyAsync((void*)(flags + 1), a.fail, sizeof(int32_t), hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess && shape.blocks != blocks) {
+      a.rows = shape.rows;
+      e = hipMemcpyAsync(base + args_at, &a, sizeof(a), hipMemcpyHostToDevice, st);
+      blocks = shape.blocks;
+    }
+    if (e == hipSuccess) e = launch_loop(args, kc, shape, st);
+    if (e == hipSuccess) e = hipMemcpyAsync((void*)flags, a.flags, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e == hipSuccess && flags[1]) {
+    if (e == hipSuccess && flags[0]) {
       e = hipMemcpyAsync(pr.states, saved, backup, hipMemcpyDeviceToDevice, st);
       if (e == hipSuccess) e = hipStreamSynchronize(st);
       if (e == hipSuccess) {
+        counts[CVO_LOOP_DECLINED]--;
         counts[CVO_LOOP_ABANDONED]++;
         ctx->loop_pause = std::min(kLoopPauseMax, std::max(kLoopPause, 2 * ctx->loop_pause));
         ctx->loop_rest = ctx->loop_pause;
@@ -602,8 +625,9 @@ static cvo_status run_resident(cvo_ctx* ctx, const Problems& pr, const KConsts& 
       }
     }
     if (e != hipSuccess) status = hip_check(ctx, e, "resident loop");
-    else if (flags[0] || it + kLoopChunk >= max_iter) {
+    else if (flags[1] || it + chunk >= max_iter) {
       *ran = true;
+      counts[CVO_LOOP_DECLINED]--;
       counts[CVO_LOOP_COMPLETED]++;
       ctx->loop_pause = 0;
       break;
@@ -1100,6 +1124,7 @@ static cvo_status align_impl_d(cvo_ctx* ctx, const cvo_dcloud* src, const cvo_dc
                                float T_out[16], cvo_assoc* assoc_out, double* seconds, int32_t* iters,
                                int32_t* ret_code) {
   if (!ctx || !T_init || !T_out) return CVO_ERR_INVALID_ARG;
+  ActiveCall busy(ctx);
   if (ret_code) *ret_code = 0;
   if (iters) *iters = 0;
   if (seconds) *seconds = 0.0;
@@ -1207,6 +1232,7 @@ static void inverse4(const float m[16], float out[16]) {
 // function_angle scores of get_nearest_init_pose (CvoGPU.cpp:381-389).
 static cvo_status score_poses(cvo_ctx* ctx, const cvo_dcloud* src, const cvo_dcloud* tgt, int n, const float* T16,
                               float ell, std::vector<double>& ip) {
+  ActiveCall busy(ctx);
   CVO_TRY(validate_pair(ctx, src, tgt));
   const cvo_params& p = ctx->params;
   KConsts kc = make_kconsts(p, src->F, src->K, MODE_IP);
@@ -1380,6 +1406,7 @@ static KConsts adaptive_kconsts(const cvo_params& p, int F, int Ks);
 static cvo_status single_pass(cvo_ctx* ctx, const cvo_dcloud* src, const cvo_dcloud* tgt, const float T[16], float ell,
                               Problems& pr, KConsts& kc, double* ip, int knn_K = 0, const KConsts* kc_in = nullptr,
                               bool keep_pairs = true) {
+  ActiveCall busy(ctx);
   CVO_TRY(validate_pair(ctx, src, tgt));
   const cvo_params& p = ctx->params;
   kc = kc_in ? *kc_in : make_kconsts(p, src->F, src->K, MODE_IP);
@@ -1569,6 +1596,7 @@ extern "C" cvo_status cvo_align_multistart(cvo_ctx* ctx, const cvo_dcloud* src, 
                                            int32_t* best_index, float* per_start_T, double* per_start_cos,
                                            int32_t* per_start_iters, double* seconds) {
   if (!ctx || !T_starts || !T_best || n_starts <= 0 || !(score_ell > 0)) return CVO_ERR_INVALID_ARG;
+  ActiveCall busy(ctx);
   if (n_starts > 4096) return set_err(ctx, CVO_ERR_LIMIT, "at most 4096 starts per call");
   if (!src || !tgt || src->n == 0 || tgt->n == 0) return set_err(ctx, CVO_ERR_EMPTY, "empty point cloud");
   CVO_TRY(validate_pair(ctx, src, tgt));
@@ -1694,6 +1722,7 @@ extern "C" cvo_status cvo_align_adaptive_d(cvo_ctx* ctx, const cvo_dcloud* src, 
                                            const float T_init[16], float T_out[16], double* seconds, int32_t* iters,
                                            int32_t* ret_code) {
   if (!ctx || !T_init || !T_out) return CVO_ERR_INVALID_ARG;
+  ActiveCall busy(ctx);
   if (ret_code) *ret_code = 0;
   if (iters) *iters = 0;
   if (seconds) *seconds = 0.0;

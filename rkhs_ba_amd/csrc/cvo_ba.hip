@@ -60,6 +60,7 @@
 
 #include "cvo_device.h"
 #include "cvo_internal.h"
+#include "cvo_loop.h"
 
 namespace cvo {
 
@@ -1349,6 +1350,7 @@ extern "C" cvo_status cvo_align_multiframe(cvo_ctx* ctx, int32_t n_frames, const
                                            const int32_t* edges, cvo_assoc* per_edge, double* seconds,
                                            int32_t* iters, double* per_iter_seconds, int32_t max_iter_records) {
   if (!ctx) return CVO_ERR_INVALID_ARG;
+  ActiveCall busy(ctx);
   if (per_edge)
     for (int e = 0; e < n_edges; ++e) std::memset(&per_edge[e], 0, sizeof(cvo_assoc));
   if (seconds) *seconds = 0.0;

@@ -228,6 +228,7 @@ struct cvo_ctx {
   DevBuf b_export;
   DevBuf b_loop;  // resident loop: exchange words, wait flag, saved states
   int64_t loop_counts[CVO_LOOP_COUNT] = {0, 0, 0};
+  int32_t call_depth = 0;  // calls in progress, one inside the other
   int32_t loop_rest = 0, loop_pause = 0;  // registrations left, and in all, that do not try after an abandoned launch
   void* pinned = nullptr;  // small pinned host buffer for flags
   size_t pinned_cap = 0;

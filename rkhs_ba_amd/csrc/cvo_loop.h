@@ -12,14 +12,13 @@ namespace cvo {
 constexpr int kMaxLoopDevices = 64;
 constexpr size_t kLoopMaxLds = 128 * 1024;  // dynamic LDS of a block, beside up to 8 KB of static LDS
 
-// Arguments of a launch, in device memory.
+// Arguments of the launches of one shape, in device memory.
 struct LoopArgs {
   KConsts kc;
   AssocProblem prob[3];  // the registration; adaptive lengthscale: and its two self problems
   int32_t rows;          // LDS rows of a block
-  int32_t max_iters;     // iterations of this launch
-  uint32_t tag0;         // tag of its first iteration (never 0, never used before on these words)
-  uint32_t* fail;        // set when a wait ran out
+  int32_t max_iters;     // iterations of a launch
+  uint32_t* flags;       // [0] set when a wait ran out, [1] the registration is done
   uint64_t* xa;          // words of the two exchanges
   uint64_t* xb;
   uint64_t wait_ticks;   // longest wait of an exchange, in ticks of the 100 MHz clock
@@ -30,11 +29,29 @@ struct LoopShape {
   size_t lds = 0;
 };
 
+// A call that uses the device, counted while the object lives (once a context).
+class ActiveCall {
+ public:
+  explicit ActiveCall(cvo_ctx* ctx);
+  ~ActiveCall();
+
+ private:
+  cvo_ctx* ctx_;
+};
+
+// Blocks that a resident launch may have of a device's units: all of them for the
+// process's only call, an equal part beside others; 0 where that is too small.
+int loop_share(int dev, int units);
+
 // The compute units a resident launch holds until the object goes.
-struct LoopUnits {
-  int device = 0, n = 0;
+class LoopUnits {
+ public:
   ~LoopUnits();
-  bool claim(int dev, int blocks, int units);
+  // Waits up to wait_ms for other launches to give units back.
+  bool claim(int dev, int blocks, int units, int wait_ms);
+
+ private:
+  int device_ = 0, n_ = 0;
 };
 
 size_t loop_words_bytes();

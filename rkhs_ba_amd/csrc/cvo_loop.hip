@@ -28,7 +28,8 @@
 //
 // All blocks must be resident at once: one block fits a compute unit, the host
 // keeps the blocks of all such launches of the process within the device's
-// compute units, and every wait is bounded by a clock: a launch whose wait runs
+// compute units (a launch beside other calls has its share of them, and gives them
+// back every few milliseconds), and every wait is bounded by a clock: a launch whose wait runs
 // out leaves the state as it was, and the caller goes on with the
 // launch-per-pass loop.
 
@@ -38,6 +39,9 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
+#include <condition_variable>
+#include <mutex>
 
 #include "cvo_assoc.h"
 #include "cvo_controller.h"
@@ -680,10 +684,9 @@ __global__ __launch_bounds__(kLoopThreads) void loop_kernel(const LoopArgs* args
   }
   __syncthreads();
   const int max_iters = fresh(ap).max_iters;
-  const uint32_t tag0 = fresh(ap).tag0;
   for (int it = 0; it < max_iters; ++it) {
     if (S.st[0].done) break;  // uniform: every block holds the same state
-    const uint32_t tag = tag0 + (uint32_t)it;
+    const uint32_t tag = (uint32_t)uni(S.st[0].iter) + 1u;  // never 0, and each iteration its own
     const float ell0 = uni(S.st[0].ell);
     if (ell0 != S.rows_ell) {  // uniform
       // one lengthscale for all problems; rows with their own lengthscale are
@@ -889,9 +892,10 @@ __global__ __launch_bounds__(kLoopThreads) void loop_kernel(const LoopArgs* args
   const LoopArgs& Ae = fresh(ap);
   if (S.bad) {
     // the state in memory stays as this launch found it
-    if (tid == 0) __hip_atomic_store(Ae.fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) __hip_atomic_store(Ae.flags, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return;
   }
+  if (blockIdx.x == 0 && tid == 0) st_global(Ae.flags + 1, (uint32_t)S.st[0].done);
 #pragma unroll
   for (int q = 0; q < NP; ++q) {
     const AssocProblem& P = Ae.prob[q];
@@ -909,20 +913,52 @@ __global__ __launch_bounds__(kLoopThreads) void loop_kernel(const LoopArgs* args
 // Host
 // ---------------------------------------------------------------------------
 
-// Compute units claimed by resident launches, per device (one block a unit).
-static std::atomic<int> g_units[kMaxLoopDevices];
+// Per device, the calls of the process that use it and the compute units that its
+// resident launches hold (one block a unit, whole XCD rounds: each XCD has an
+// eighth of the units, and a block can only go where one is free).
+struct LoopDevice {
+  std::mutex mutex;
+  std::condition_variable freed;
+  int held = 0;
+  std::atomic<int> calls{0};
+};
+static LoopDevice g_devices[kMaxLoopDevices];
+
+static LoopDevice* loop_device(int dev) { return dev >= 0 && dev < kMaxLoopDevices ? &g_devices[dev] : nullptr; }
+
+ActiveCall::ActiveCall(cvo_ctx* ctx) : ctx_(ctx) {
+  LoopDevice* d = loop_device(ctx->device);
+  if (ctx->call_depth++ == 0 && d) d->calls.fetch_add(1);
+}
+ActiveCall::~ActiveCall() {
+  LoopDevice* d = loop_device(ctx_->device);
+  if (--ctx_->call_depth == 0 && d) d->calls.fetch_sub(1);
+}
+
+int loop_share(int dev, int units) {
+  const LoopDevice* d = loop_device(dev);
+  const int calls = d ? d->calls.load() : 1;
+  return calls <= 1 ? units : (units / calls) & ~7;
+}
 
 LoopUnits::~LoopUnits() {
-  if (n > 0) g_units[device].fetch_sub(n);
-}
-bool LoopUnits::claim(int dev, int blocks, int units) {
-  if (dev < 0 || dev >= kMaxLoopDevices || blocks <= 0) return false;
-  if (g_units[dev].fetch_add(blocks) + blocks > units) {
-    g_units[dev].fetch_sub(blocks);
-    return false;
+  if (n_ == 0) return;
+  LoopDevice* d = loop_device(device_);
+  {
+    std::lock_guard<std::mutex> lock(d->mutex);
+    d->held -= n_;
   }
-  device = dev;
-  n = blocks;
+  d->freed.notify_all();
+}
+bool LoopUnits::claim(int dev, int blocks, int units, int wait_ms) {
+  LoopDevice* d = loop_device(dev);
+  if (!d || blocks <= 0) return false;
+  const int n = std::min((blocks + 7) & ~7, units);
+  std::unique_lock<std::mutex> lock(d->mutex);
+  if (!d->freed.wait_for(lock, std::chrono::milliseconds(wait_ms), [&] { return d->held + n <= units; })) return false;
+  d->held += n;
+  device_ = dev;
+  n_ = n;
   return true;
 }
 
@@ -934,7 +970,7 @@ uint64_t* loop_step_words(uint64_t* words) { return words + kXaWords; }
 bool loop_shape(const KConsts& kc, const int* rows, int n_probs, int units, LoopShape* out) {
   // without the distance gate every row scans all targets: that work is not
   // spread by rows
-  if (!kc.use_geo || kc.uncapped || kc.mode != MODE_ALIGN) return false;
+  if (!kc.use_geo || kc.uncapped || kc.mode != MODE_ALIGN || units <= 0) return false;
   // The loop saves launches, states read back and counters, about 15 us an
   // iteration; the passes have more waves in flight a row.  Registrations of 1000
   // iterations, passes / loop: planes at 60k rows 129 / 117 ms, at 80k 186 / 178,
@@ -971,7 +1007,7 @@ bool loop_shape(const KConsts& kc, const int* rows, int n_probs, int units, Loop
 }
 
 template <int FC, int KC, bool KNN, int NP>
-static hipError_t launch_loop_t(const LoopArgs* a, const KConsts& kc, const LoopShape& s, hipStream_t st) {
+static hipError_t launch_loop_t(const LoopArgs* a, const LoopShape& s, hipStream_t st) {
   const void* fn = reinterpret_cast<const void*>(&loop_kernel<FC, KC, KNN, NP>);
   if (s.lds > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLoopMaxLds);
@@ -984,10 +1020,10 @@ static hipError_t launch_loop_t(const LoopArgs* a, const KConsts& kc, const Loop
 template <int FC, int KC>
 static hipError_t launch_loop_fk(const LoopArgs* a, const KConsts& kc, const LoopShape& s, hipStream_t st) {
   if (kc.adaptive) {
-    if constexpr (FC != 0) return launch_loop_t<FC, KC, false, 3>(a, kc, s, st);
+    if constexpr (FC != 0) return launch_loop_t<FC, KC, false, 3>(a, s, st);
     else return hipErrorInvalidValue;  // the adaptive association always compares features
   }
-  return kc.knn > 0 ? launch_loop_t<FC, KC, true, 1>(a, kc, s, st) : launch_loop_t<FC, KC, false, 1>(a, kc, s, st);
+  return kc.knn > 0 ? launch_loop_t<FC, KC, true, 1>(a, s, st) : launch_loop_t<FC, KC, false, 1>(a, s, st);
 }
 
 hipError_t launch_loop(const LoopArgs* a, const KConsts& kc, const LoopShape& s, hipStream_t st) {

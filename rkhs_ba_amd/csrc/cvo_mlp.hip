@@ -36,6 +36,7 @@
 #include <vector>
 
 #include "cvo_internal.h"
+#include "cvo_loop.h"
 
 namespace cvo {
 
@@ -1130,6 +1131,7 @@ extern "C" cvo_status cvo_model_set_weights(cvo_model* m, const float* w, int64_
 extern "C" cvo_status cvo_model_gradient(cvo_ctx* ctx, cvo_model* m, int32_t n_pairs, int32_t npts, const float* a,
                                          const float* b, const float* targets, float* grad_out, float* loss_out) {
   if (!ctx || !m || !a || !b || !targets) return CVO_ERR_INVALID_ARG;
+  ActiveCall busy(ctx);
   CVO_TRY(check_batch(ctx, n_pairs, npts));
   hipStream_t s = ctx->stream;
   CVO_TRY(upload_points(m, n_pairs, npts, a, b, false));
@@ -1236,6 +1238,7 @@ extern "C" cvo_status cvo_model_train_step(cvo_ctx* ctx, cvo_model* m, int32_t n
 static cvo_status propose_impl(cvo_ctx* ctx, const cvo_model* mc, int32_t n_pairs, int32_t npts, const float* a,
                                const float* b, bool on_device, float* quat_t, float* conf, float* raw_out) {
   if (!ctx || !mc || !a || !b || !quat_t || !conf) return CVO_ERR_INVALID_ARG;
+  ActiveCall busy(ctx);
   CVO_TRY(check_batch(ctx, n_pairs, npts));
   cvo_model* m = const_cast<cvo_model*>(mc);
   hipStream_t s = ctx->stream;

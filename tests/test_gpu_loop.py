@@ -104,6 +104,29 @@ def test_most_rows(n, kw, adaptive):
         both(params(MAX_ITER=2), tgt, src, adaptive, ran="declined")
 
 
+def test_launches_follow_one_another():
+    # 600 iterations in three launches: the state goes through memory, the words
+    # of the exchanges stay
+    src, tgt = pair(1501, 1303)
+    p = params(MAX_ITER=600)
+    cvo = CvoGPU(params=p)
+    try:
+        cvo.set_trace(600)
+        print("launches one after another", flush=True)
+        a = cvo.align(src, tgt, np.eye(4)), [(r.nnz, r.max_row, r.num_neighbors, r.ell) for r in cvo.get_trace()]
+        b = cvo.align(src, tgt, np.eye(4)), [(r.nnz, r.max_row, r.num_neighbors, r.ell) for r in cvo.get_trace()]
+        assert cvo.loop_counts() == dict(completed=2, abandoned=0, declined=0)
+        assert a[0][3] > 256
+        # fewer iterations than a launch: the same first ones
+        p.MAX_ITER = 250
+        cvo.write_params(p)
+        c = cvo.align(src, tgt, np.eye(4)), [(r.nnz, r.max_row, r.num_neighbors, r.ell) for r in cvo.get_trace()]
+    finally:
+        cvo.close()
+    np.testing.assert_array_equal(a[0][1], b[0][1])
+    assert a[1] == b[1] and a[1][:249] == c[1][:249]
+
+
 @pytest.mark.parametrize("lanes", [4, 8])
 def test_lanes_of_more_rows_than_a_round(lanes):
     src, tgt = pair(20011, 20011)
@@ -185,7 +208,9 @@ def test_threads_share_the_compute_units():
         t.start()
     for t in ts:
         t.join()
-    assert all(sum(c.values()) == 3 for c in counts) and sum(c["completed"] for c in counts) > 0, counts
+    assert all(sum(c.values()) == 3 for c in counts), counts
+    # each has its share of the units, so nearly all run resident
+    assert sum(c["completed"] for c in counts) >= 9, counts
     for g in got:
         for T in g:
             np.testing.assert_allclose(T, want[1], rtol=0, atol=2e-6)
