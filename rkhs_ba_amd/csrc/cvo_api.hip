@@ -497,6 +497,14 @@ cvo_status setup_problems(cvo_ctx* ctx, const cvo_dcloud* s, const cvo_dcloud* t
   return CVO_OK;
 }
 
+// On the context's own stream: a copy on the null stream fails while another
+// thread's stream captures.
+cvo_status read_back(cvo_ctx* ctx, void* dst, const void* src, size_t bytes) {
+  CVO_HIP(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
+  CVO_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  return CVO_OK;
+}
+
 cvo_status pinned(cvo_ctx* ctx, size_t bytes) {
   if (ctx->pinned_cap >= bytes) return CVO_OK;
   if (ctx->pinned) CVO_HIP(ctx, hipHostFree(ctx->pinned));
@@ -1176,8 +1184,7 @@ static cvo_status align_impl_d(cvo_ctx* ctx, const cvo_dcloud* src, const cvo_dc
   if (want_trace) {
     int n_rec = std::min(trace_cap, n_it + 1);
     ctx->trace.resize(n_rec);
-    if (n_rec > 0)
-      CVO_HIP(ctx, hipMemcpy(ctx->trace.data(), pr.trace, sizeof(cvo_iter_record) * n_rec, hipMemcpyDeviceToHost));
+    if (n_rec > 0) CVO_TRY(read_back(ctx, ctx->trace.data(), pr.trace, sizeof(cvo_iter_record) * n_rec));
     ctx->trace_n = n_rec;
     if (ctx->profiling) account_bytes(ctx, src, tgt, kc, ctx->trace, n_rec, true);
   }
@@ -1846,8 +1853,7 @@ extern "C" cvo_status cvo_align_adaptive_d(cvo_ctx* ctx, const cvo_dcloud* src, 
   if (want_trace) {
     const int n_rec = std::min(trace_cap, n_it + 1);
     ctx->trace.resize(n_rec);
-    if (n_rec > 0)
-      CVO_HIP(ctx, hipMemcpy(ctx->trace.data(), pr.trace, sizeof(cvo_iter_record) * n_rec, hipMemcpyDeviceToHost));
+    if (n_rec > 0) CVO_TRY(read_back(ctx, ctx->trace.data(), pr.trace, sizeof(cvo_iter_record) * n_rec));
     ctx->trace_n = n_rec;
     if (ctx->profiling) account_bytes_adaptive(ctx, src, tgt, kc, ctx->trace, n_rec);
   }

@@ -1662,10 +1662,10 @@ extern "C" cvo_status cvo_align_multiframe(cvo_ctx* ctx, int32_t n_frames, const
   }
   if (status != CVO_OK) return status;
   BaDev* out = new BaDev;
-  hipError_t re = hipMemcpy(out, L.ba, sizeof(BaDev), hipMemcpyDeviceToHost);
-  if (re != hipSuccess) {
+  const cvo_status re = read_back(ctx, out, L.ba, sizeof(BaDev));
+  if (re != CVO_OK) {
     delete out;
-    return hip_check(ctx, re, "BA state readback");
+    return re;
   }
   for (int f = 0; f < n_frames; ++f)
     for (int i = 0; i < 12; ++i) poses[12 * f + i] = out->X[12 * f + i];

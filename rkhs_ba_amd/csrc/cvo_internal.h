@@ -273,6 +273,7 @@ void apply_tuning(const cvo_ctx* ctx, KConsts& kc, int64_t batched_rows = 0);
 void apply_tuning(const cvo_tuning& t, KConsts& kc, bool batched = false);
 cvo_status ensure_events(cvo_ctx* ctx, size_t n);
 cvo_status pinned(cvo_ctx* ctx, size_t bytes);
+cvo_status read_back(cvo_ctx* ctx, void* dst, const void* src, size_t bytes);
 cvo_status prepare_source_into(cvo_ctx* ctx, const cvo_dcloud* s, DevBuf& b_pos, DevBuf& b_feat, DevBuf& b_sem,
                                DevBuf& b_geo);
 cvo_status build_grid_into(cvo_ctx* ctx, const cvo_dcloud* t, const std::vector<float>& hs, GridHost& gh,

@@ -214,3 +214,47 @@ def test_threads_share_the_compute_units():
     for g in got:
         for T in g:
             np.testing.assert_allclose(T, want[1], rtol=0, atol=2e-6)
+
+
+def test_calls_beside_a_window_that_captures():
+    # every window captures its outer iteration; a registration by passes captures
+    # too, and both read back at their end
+    src, tgt = pair(2000, 2000)
+    clouds, _, inits = synth.window_frames(1, n_frames=3, n_min=800, n_max=900)
+    pb = params_from_yaml("ba_window.yaml")
+    pb.multiframe_max_iters = 1
+    pb.multiframe_min_nonzeros = 1
+    errors = []
+
+    def guarded(work):
+        def run():
+            try:
+                work()
+            except Exception as e:  # noqa: BLE001
+                errors.append(e)
+        return threading.Thread(target=run)
+
+    def windows():
+        cvo = CvoGPU(params=pb)
+        try:
+            for _ in range(60):
+                cvo.align_multiframe(clouds, inits, [1, 0, 0], [(0, 1), (1, 2)])
+        finally:
+            cvo.close()
+
+    def registrations():
+        cvo = CvoGPU(params=params())
+        try:
+            cvo.set_trace(ITERS)
+            for _ in range(60):
+                cvo.align(src, tgt, np.eye(4))
+        finally:
+            cvo.close()
+
+    print("windows beside registrations", flush=True)
+    ts = [guarded(windows), guarded(registrations), guarded(windows), guarded(registrations)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not errors, errors
