@@ -527,11 +527,11 @@ cvo_status ensure_events(cvo_ctx* ctx, size_t n) {
 // done.  Profiling mode launches kernel by kernel with events around each.
 static constexpr int kChunk = 24;
 
-// Iterations of one resident launch: 4 to 10 milliseconds' worth, the longest that
-// other streams wait for the compute units it holds, and other registrations for
-// their share.  A launch costs 50 us at 5000 rows, 130 at 60000, 0.5 to 1 % of a
-// registration.
-static int loop_chunk(int rows) { return rows > 65536 ? 64 : 256; }
+// Iterations of one resident launch: about 5 ms' worth, 15 where the first
+// iterations are long (60000 rows), the longest that other streams wait for the
+// compute units it holds, and other registrations for their share.  A launch costs
+// about 50 us, up to 1 % of a registration.
+static int loop_chunk(int rows) { return rows > 65536 ? 64 : (rows > 16384 ? 128 : 256); }
 // Rows a block, at most, of a launch on a share of the units: with 156 two
 // registrations of 20000 points made 156 a second of 100 iterations (passes 147),
 // eight of 5000 488 of 200 (passes 405); with 312 four of 20000 made 176 (passes 195).
