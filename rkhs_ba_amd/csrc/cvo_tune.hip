@@ -281,11 +281,12 @@ extern "C" cvo_status cvo_autotune_d(cvo_ctx* ctx, const cvo_dcloud* src, const 
   const float set_scale[kNS] = {1.0f, 1.0f, 1.0f, 0.7f, 0.7f, 0.7f, 0.5f, 0.5f, 0.5f};
   constexpr int kReps = 5, kRounds = 3;
   // one grid serves every scale: its levels reach the finest scale's radius; at
-  // one lengthscale it has the level that each scale would build alone
+  // one lengthscale it has the levels that the scales would build alone (0.5 takes
+  // 0.7's)
   std::vector<float> hs = level_sizes(kc, e_hi, e_lo, src->max_norm, tq, 0.5f);
   if (kc.use_geo && e_hi == e_lo) {
     hs.clear();
-    for (float scale : {1.0f, 0.7f, 0.5f}) hs.push_back(one_level_size(kc, e_hi, src->max_norm, tq, scale));
+    for (float scale : {1.0f, 0.7f}) hs.push_back(one_level_size(kc, e_hi, src->max_norm, tq, scale));
   }
   GridHost gh;
   CVO_TRY(build_grid(ctx, tgt, hs, gh));
