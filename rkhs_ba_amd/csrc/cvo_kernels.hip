@@ -441,13 +441,15 @@ __device__ __forceinline__ void assoc_pass(const AssocProblem& P, const KConsts&
 
 // ONE: a single problem, its descriptor by value in the kernel arguments (read
 // with scalar loads, no dependent load before the first state read).
-// Occupancy: five waves per SIMD (96 VGPRs; six spill 96 bytes: the 60k street
-// registration 125 against 157 ms).  Batched launches need the maps and the grid
-// level in scalar registers for it (with them in vector registers five waves
-// spill 64 bytes and are slower than four): 96 starts over 20k points, 300
-// iterations, 8 lanes a row, 644 -> 583 ms.
+// Occupancy: five waves per SIMD for one problem (96 VGPRs; six spill 96 bytes: the
+// 60k street registration 125 against 157 ms).  Batched launches hold the maps and
+// the grid level in scalar registers and run at four (106 VGPRs, none spilled):
+// 96 starts over 20k points, 1000 iterations, 16 lanes above ell 0.158 and 8 below
+// 1.58 s, untuned 1.54; at five waves 31 registers spill, 1.71 and 1.74 (40
+// iterations at ell 0.5 8 % faster, at 0.08 14 % slower); with the maps in vector
+// registers at four 1.61.
 template <int FC, int KC, bool ONE>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void assoc_kernel(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(ONE ? 5 : 4))) void assoc_kernel(
     const AssocProblem* __restrict__ probs, int n_probs, KConsts kc, AssocProblem one) {
   if constexpr (ONE) {
     assoc_pass<FC, KC, false, true>(one, kc);
