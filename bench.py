@@ -44,10 +44,12 @@ HBM_PEAK_GBS = 8000.0
 # FETCH_SIZE / WRITE_SIZE passes scaled by a 256 MiB copy probe
 # (profiles/assoc_street60k_pmc_traffic.md)
 ASSOC_TRAFFIC_BYTES = 25.78e6
-# HBM bytes a pass over the stored pairs of the 12-frame window moves, the same
-# way (profiles/ba_window12_pmc_traffic.md: counted on an earlier kernel that read
-# the same rows)
-BA_PAIR_TRAFFIC_BYTES = 912.5e6
+# the same of all launches of the resident loop in one registration of 2000
+# iterations (profiles/workloads_kernel_trace.md)
+LOOP_TRAFFIC_BYTES = 9.96e9
+# the same of a moment pass over the stored pairs of the 12-frame window
+# (profiles/ba_window12_pmc_traffic.md)
+BA_PAIR_TRAFFIC_BYTES = 815.6e6
 # per-launch work of the association kernel on the 60k street registration
 # with its autotuned launch shape, from rocprofv3 counters (SQ_INSTS_VALU_TRANS_F32
 # x 64 lanes; SQ_INSTS_VALU_FLOPS_FP32 x 64): the transcendental and FP32
@@ -209,7 +211,21 @@ def leg_twoview(args):
     achieved = assoc_bytes / (assoc_ms * 1e-3) / 1e9
     exp_rate = ASSOC_EXP_PER_LAUNCH / (assoc_ms * 1e-3)
     flop_rate = ASSOC_FP32_FLOP_PER_LAUNCH / (assoc_ms * 1e-3) / 1e12
-    out["roofline"] = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+    # what the timed registrations run: the resident loop's launches, over the
+    # bytes of their association and step passes
+    loop_bytes = st["bytes"]["assoc"] + st["bytes"]["step"]
+    loop_gbs = loop_bytes / (out["device_loop_ms"] * 1e-3) / 1e9
+    full = args.points == 60000 and out["iterations"] == 2000
+    out["roofline"] = {"bound": "hbm", "achieved": loop_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                       "frac": loop_gbs / HBM_PEAK_GBS, "kernel": "loop_kernel",
+                       "traffic": LOOP_TRAFFIC_BYTES if full else None,
+                       "device_loop_ms": out["device_loop_ms"], "algorithmic_bytes_per_registration": loop_bytes,
+                       "timing": "HIP events around the loop's launches of a timed registration",
+                       "note": "latency-bound: two exchanges between the blocks, the FP64 controller and dependent "
+                               "gathers an iteration; rows stay in LDS and targets in L2"}
+    # the same association as a pass of its own (the launch-per-pass loop, which
+    # profiling runs)
+    out["assoc_pass"] = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                        "frac": achieved / HBM_PEAK_GBS, "traffic": args.traffic,
                        "kernel": "assoc_kernel", "avg_launch_ms": assoc_ms,
                        "algorithmic_bytes_per_launch": assoc_bytes, "launches": n_assoc,
@@ -676,9 +692,10 @@ def leg_adaptive(args):
     n = max(1, st["launches"]["assoc"])
     ms, by = st["ms"]["assoc"] / n, st["bytes"]["assoc"] / n
     out["roofline"] = {"bound": "hbm", "achieved": by / (ms * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                       "frac": by / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, "kernel": "assoc_kernel (three problems)",
+                       "frac": by / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, "kernel": "assoc_kernel (three problems; as a pass of its own)",
                        "avg_launch_ms": ms, "algorithmic_bytes_per_launch": by, "launches": n, "traffic": None,
-                       "note": "bytes count every point three times and the registration problem's pairs only"}
+                       "note": "bytes count every point three times and the registration problem's pairs only; "
+                               "registrations up to 16384 points run the same rows in loop_kernel"}
     out["kernels_ms_per_launch"] = {k: st["ms"][k] / max(1, st["launches"][k]) for k in ("assoc", "overflow", "step")}
     if not args.no_cpu:
         from oracle import pyoracle
@@ -856,6 +873,7 @@ def main():
         "device_loop_ms": tv["device_loop_ms"],
         "pose_error": tv["pose_error"],
         "roofline": tv.get("roofline"),
+        "assoc_pass": tv.get("assoc_pass"),
         "tuning": tv.get("tuning"),
         "kernels_ms_per_launch": tv.get("kernels_ms_per_launch"),
         "host_to_host": tv.get("host_to_host"),

@@ -455,11 +455,14 @@ cvo_status cvo_set_pose_arithmetic(cvo_ctx* ctx, int32_t mode);
  *                    lengthscales >= split_ell (every lengthscale when
  *                    split_ell <= 0); launches over several problems
  *                    (multi-start, adaptive, BA) and the K-nearest pass use
- *                    at least 8;
+ *                    at least 8; resident registrations (cvo_get_loop_counts)
+ *                    take 16 for 8, 16 for K nearest, and 32 or 64 where they
+ *                    have few rows a compute unit;
  *   cell_scale       grid cells are chosen with edge >= cell_scale x the
  *                    ell-ball radius, in [0.4, 1] (smaller: more cells per
  *                    query box, fewer candidates outside the ball), at
- *                    lengthscales >= split_ell;
+ *                    lengthscales >= split_ell; 0.7 at least where a grid has
+ *                    one lengthscale;
  *   lanes_small_ell, cell_scale_small_ell
  *                    the same below split_ell (the device controller applies
  *                    them per iteration, so they follow the annealing inside
@@ -468,7 +471,10 @@ cvo_status cvo_set_pose_arithmetic(cvo_ctx* ctx, int32_t mode);
  *                    the spatially sorted row blocks (its own L2 serves the
  *                    overlapping target neighbourhoods), 0: dispatch order.
  * The tuning of a context applies to every later align / multi-start / BA /
- * inner-product call on it. */
+ * inner-product call on it.  An untuned context (source CVO_TUNE_DEFAULT) reports
+ * the shape of its inner products, 16 lanes and cell scale 1; its registrations
+ * take cell scale 0.7, its launches over several problems 0.5 and, from 49152
+ * source rows in all, 8 lanes; under a workspace limit all take cell scale 1. */
 typedef struct {
   int32_t lanes_per_row;
   int32_t lanes_small_ell;
@@ -483,13 +489,14 @@ typedef struct {
 enum { CVO_TUNE_DEFAULT = 0, CVO_TUNE_SET = 1, CVO_TUNE_MEASURED = 2, CVO_TUNE_CACHED = 3 };
 
 cvo_status cvo_get_tuning(const cvo_ctx* ctx, cvo_tuning* out);
-/* CVO_ERR_INVALID_ARG for lane counts not in {8, 16}, a negative or
+/* CVO_ERR_INVALID_ARG for lane counts not in {4, 8, 16}, a negative or
  * non-finite split_ell, xcd_remap not in {0, 1} or a cell scale outside
  * [0.4, 1]. */
 cvo_status cvo_set_tuning(cvo_ctx* ctx, const cvo_tuning* t);
-/* Times the association pass of this source / target pair at T_init for
- * every lane count (8, 16), block order (2) and cell scale (1, 0.7, 0.5) at
- * four lengthscales log-spaced from ell_init to ell_min, then keeps the
+/* Times the association pass of this source / target pair (one problem, a launch
+ * of its own) at T_init for every lane count (4, 8, 16), block order (2) and cell
+ * scale (1, 0.7, 0.5) at four lengthscales log-spaced from ell_init to ell_min
+ * (one where they are equal), then keeps the
  * block order and the two-segment (lanes, cell scale) policy with the least
  * modelled time per registration: the three annealing samples share the
  * iterations of the decay schedule (decays x 2 x indicator window), ell_min

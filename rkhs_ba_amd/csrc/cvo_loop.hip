@@ -7,11 +7,12 @@
 // controller itself, so all blocks hold the same state and no block waits for
 // a broadcast.  What bounds the launch-per-pass loop at small and middle sizes
 // is not work but the chain of kernel starts, state reads and completion
-// counters; here an iteration has two exchanges of 1.2 to 1.8 us.  Measured per
-// registration, launch-per-pass loop to this one: 1.1k points without colour, 500
-// iterations 16.3 -> 9.3 ms; 5k with colour, 2000 iterations 60.0 -> 35.1; 60k
-// with colour and 19 classes, 2000 iterations 111.6 -> 82.3; K nearest at 20k,
-// 600 iterations 29.9 -> 24.5; adaptive lengthscale at 5k 7.9 -> 6.9.
+// counters; here an iteration has two exchanges (2.5 us each at 256 blocks, skew of
+// the blocks included).  Measured per registration, launch-per-pass loop to this
+// one: 1.1k points without colour, 500 iterations 16.3 -> 9.3 ms; 5k with colour,
+// 2000 iterations 60.0 -> 35.1; 60k with colour and 19 classes, 2000 iterations
+// 111.6 -> 82.3; K nearest at 20k, 600 iterations 29.9 -> 24.5; adaptive
+// lengthscale at 5k 7.9 -> 6.9.
 //
 // Exchange: a block stores its partials as 8-byte words {payload, tag} with
 // device-scope stores (tag: the iteration), and its readers read all words with
@@ -21,7 +22,8 @@
 // publishes the group's words, and every block reads the eight groups.  One
 // wave per block takes part: at 256 blocks an exchange among all (32 KB read by
 // every block) measured 2.1 to 2.4 us in isolation and 4.0 in the loop, where
-// sixteen waves a block poll and add; two levels measured 1.8.
+// sixteen waves a block poll and add; two levels 1.8 in isolation and 2.5 in the
+// loop; 32 blocks in one level 1.2 in isolation.
 // A block can only publish iteration i + 1 of one exchange after it has read
 // iteration i of the other, which every block published after reading iteration
 // i of the first: one buffer per exchange and level is enough.
@@ -29,8 +31,8 @@
 // All blocks must be resident at once: one block fits a compute unit, the host
 // keeps the blocks of all such launches of the process within the device's
 // compute units (a launch beside other calls has its share of them, and gives them
-// back every few milliseconds), and every wait is bounded by a clock: a launch whose wait runs
-// out leaves the state as it was, and the caller goes on with the
+// back every few milliseconds), and every wait is bounded by a clock: a launch
+// whose wait runs out leaves the state as it was, and the caller goes on with the
 // launch-per-pass loop.
 
 #include <hip/hip_runtime.h>

@@ -650,7 +650,8 @@ class CvoGPU:
         _check(lib().cvo_set_tuning(self._ctx, C.byref(t)), self._ctx)
 
     def apply_tuning(self, t: dict) -> None:
-        """Sets a tuning dict as returned by autotune / get_tuning."""
+        """Sets a tuning dict as returned by autotune / get_tuning (an untuned
+        context's is the shape of its inner products, see cvo_tuning)."""
         self.set_tuning(t["lanes_per_row"], t["xcd_remap"], t["cell_scale"], lanes_small_ell=t["lanes_small_ell"],
                         split_ell=t["split_ell"], cell_scale_small_ell=t["cell_scale_small_ell"])
 
