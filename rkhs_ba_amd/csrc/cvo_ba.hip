@@ -346,14 +346,14 @@ __device__ __forceinline__ void moment_origin(const AssocProblem& P, double* s, 
 // FP64 sums of 37 moments in registers.  Then the wave's 64 rows times their
 // monomials: sums over rows of products, so FP64 matrix instructions
 // (v_mfma_f64_16x16x4, 16 rows of the cloud staged in LDS at a time).  Block
-// partials of the five tiles.  Bound by FP64 issue and the rows' uneven lengths;
+// partials of the five tiles' 670 used entries.  Bound by FP64 issue and the rows' uneven lengths;
 // a pass over the pairs of each candidate took 187 us and 11 for its sums, nine
-// times an outer iteration (window of 12 frames of 5k to 40k points), this 298 us
-// once and 8 us for each candidate's polynomials (window: 61.7 -> 45.3 ms for 12 outer
-// iterations).
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void ba_moments_kernel(const BaDev* __restrict__ ba, BaEdge* __restrict__ edges,
-                                                         const AssocProblem* __restrict__ probs,
-                                                         double* __restrict__ part, int rows) {
+// times an outer iteration (window of 12 frames of 5k to 40k points), this 306 us
+// once and 8.6 us for each candidate's polynomials (window: 61.7 -> 45.3 ms for 12
+// outer iterations; over 60, whose rows get longer, 420 us a pass).
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void ba_moments_kernel(
+    const BaDev* __restrict__ ba, BaEdge* __restrict__ edges, const AssocProblem* __restrict__ probs,
+    double* __restrict__ part, int rows) {
   if (ba->done || !ba->eval_pending) return;
   const int e = blockIdx.y;
   const BaEdge& ed = edges[e];
